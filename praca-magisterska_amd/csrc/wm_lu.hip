@@ -9,11 +9,11 @@
 // Blocked right-looking algorithm with panel width NB = 64, in outer blocks
 // of kSub panels.  Per panel k:
 //   1. k_panel      : GEPP of the n-k x NB panel.  A cluster of P workgroups
-//                     per matrix holds the panel in registers (one row per
-//                     thread, or two threads per row for complex128); per
-//                     column the workgroups exchange their pivot candidates
-//                     through tagged packets, all reduce them to the same
-//                     pivot, swap and apply the rank-1 update locally.  It
+//                     per matrix holds the panel in registers (a row split
+//                     over four threads, two for complex64); per column the
+//                     workgroups exchange their pivot candidates through
+//                     tagged packets, all reduce them to the same pivot,
+//                     relabel and apply the rank-1 update locally.  It
 //                     also emits the composite row permutation of the panel.
 //   2. k_swap_trsm  : applies that permutation to the columns outside the
 //                     panel and computes U12 = L11^{-1} A12 for the outer
@@ -46,8 +46,12 @@ constexpr int NB = 64;
 // more narrow updates inside the block; measured on MI355X at N = 8192, 8
 // panels beat 4 by 1.4-6.5 % for every factor precision.
 constexpr int kSubDefault = 4, kSubLarge = 8, kSubLargeN = 8192;
-constexpr int kTprF32 = 1;      // parts per panel row (waves sharing a row) for complex64 factors: one
-                                // part keeps the cluster small enough for 16 matrices per launch at N = 8192
+// Parts per panel row (waves sharing a row).  Narrow parts shorten what each
+// wave does per column (16 or 32 columns of updates, the transposition of a
+// candidate row); complex128 panels measured 208 us with two parts (3 -> 2
+// workgroups per CU) and 165 us with four, complex64 ones 280 us with one and
+// 196 us with two (64 columns, N = 512 .. 4096).
+constexpr int kTprF64 = 4, kTprF32 = 2;
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -64,33 +68,42 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // every workgroup published after its reads of column j.
 //
 // Per launch member and parity:
-//   slot [pmax][4] : |candidate| as two 32-bit halves of a double, its position, unused
-//   cand [pmax][NW]: each workgroup's candidate row (NW 32-bit words)
+//   slot [slots][SLS]: |candidate| as two 32-bit halves of a double, its position, unused
+//   cand [slots][NWS]: each candidate's row (NW 32-bit words, per chunk the low
+//                     or real halves of its 32 values, then the high or
+//                     imaginary ones) and the reciprocal of its pivot (4 words)
 // followed by the panel permutation: cnt, rows[2NB], src[2NB].
 template <typename V>
 struct XLayout {
     static constexpr int NW = NB * (int)sizeof(V) / 4;  // 32-bit words per panel row
+    static constexpr int NWS = NW + 16;  // stride of the candidate rows (whole 128-byte lines)
+    static constexpr int SLS = 4;        // stride of the slots: dense, a poll reads few lines
     size_t par_bytes, perm_off, mat_bytes;
-    int pmax;
-    __host__ __device__ XLayout(int pmax_) : pmax(pmax_)
+    int slots;  // candidates per column: one per wave of 64 rows
+    __host__ __device__ XLayout(int slots_) : slots(slots_)
     {
-        par_bytes = ((size_t)pmax * 4 + (size_t)pmax * NW) * sizeof(uint64_t);
+        par_bytes = (size_t)slots * (SLS + NWS) * sizeof(uint64_t);
         par_bytes = (par_bytes + 255) & ~(size_t)255;
         perm_off = 2 * par_bytes;
         mat_bytes = perm_off + (1 + 4 * NB) * sizeof(int);
         mat_bytes = (mat_bytes + 255) & ~(size_t)255;
     }
     __device__ uint64_t *slot(char *m, int par) const { return (uint64_t *)(m + par * par_bytes); }
-    __device__ uint64_t *cand(char *m, int par) const { return slot(m, par) + (size_t)pmax * 4; }
+    __device__ uint64_t *cand(char *m, int par) const { return slot(m, par) + (size_t)slots * SLS; }
     __device__ int *perm(char *m) const { return (int *)(m + perm_off); }
 };
+
+// Columns of the panel updated together, and workgroups per CU that the
+// register allocation allows for (4 per CU, 128 registers, spill: 205 against
+// 159 us per complex128 panel).
+constexpr int kPanelGroup = 4, kPanelOcc = 3;
 
 template <typename T>
 struct PanelArgs {
     typename CT<T>::V *A;
     int lda;
     int64_t strideA;
-    int n, k, P, pmax;
+    int n, k, P, slots;
     int *ipiv;
     int64_t strideP;
     int *info;
@@ -108,14 +121,6 @@ __device__ inline bool better(double v2, int r2, double v1, int r1) { return v2 
 // Cross-lane moves within rows of 16 lanes (DPP: quad permutations and row
 // rotations, every source lane valid).
 template <int CTRL>
-__device__ inline double dpp_f64(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-template <int CTRL>
 __device__ inline int dpp_i32(int v)
 {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
@@ -126,16 +131,8 @@ __device__ inline double readlane_f64(double v, int l)
     const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-// Maximum over the wave (quad_perm [1,0,3,2], [2,3,0,1], row_ror 4, row_ror 8,
-// then the four row maxima); every lane gets the result.
-__device__ inline double wave_max_f64(double v)
-{
-    v = fmax(v, dpp_f64<0xB1>(v));
-    v = fmax(v, dpp_f64<0x4E>(v));
-    v = fmax(v, dpp_f64<0x124>(v));
-    v = fmax(v, dpp_f64<0x128>(v));
-    return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)), fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
-}
+// Reductions over the wave (quad_perm [1,0,3,2], [2,3,0,1], row_ror 4, row_ror 8,
+// then the four rows' results); every lane gets the result.
 __device__ inline int wave_min_i32(int v)
 {
     v = min(v, dpp_i32<0xB1>(v));
@@ -146,14 +143,79 @@ __device__ inline int wave_min_i32(int v)
                min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
+__device__ inline int wave_max_i32(int v)
+{
+    v = max(v, dpp_i32<0xB1>(v));
+    v = max(v, dpp_i32<0x4E>(v));
+    v = max(v, dpp_i32<0x124>(v));
+    v = max(v, dpp_i32<0x128>(v));
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+constexpr int kNoRow = 0x7fffffff;
+
+// Lane with the largest v >= 0 among those with cand (the lowest position on
+// ties; v of a candidate is not NaN), or -1.  The high words of non-negative
+// doubles order as integers, so one 32-bit reduction decides unless two
+// candidates agree in them (or there is none).
+__device__ inline int wave_best(double v, int pos, bool cand)
+{
+    const long long bits = __double_as_longlong(v);
+    const int hi = cand ? (int)(bits >> 32) : -1;
+    const int m = wave_max_i32(hi);
+    unsigned long long t = __ballot(hi == m);
+    if (t & (t - 1)) {
+        // the low words as signed integers in the order of unsigned ones; every
+        // lane takes part in the reductions
+        bool in = cand && hi == m;
+        const int lo = in ? (int)((unsigned)bits ^ 0x80000000u) : (int)0x80000000;
+        const int lm = wave_max_i32(lo);
+        in = in && lo == lm;
+        const int first = wave_min_i32(in ? pos : kNoRow);
+        in = in && pos == first;
+        t = __ballot(in);
+    }
+    return t ? (int)__builtin_ctzll(t) : -1;
+}
+
+__device__ inline double readlane_t(double v, int l) { return readlane_f64(v, l); }
+__device__ inline float readlane_t(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ inline double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// (re, im) - (lr, li) * (ur, ui): the complex product is rounded before it is
+// subtracted.  Fused into the subtraction it would save a third of the
+// operations, but wire matrices eliminate by exact cancellations (their
+// charge terms): with l = x / p, a rounded l * p gives x back where the fused
+// form keeps l's rounding error, and Zin of a 1024-unknown grid at 1 MHz came
+// out 100 times less accurate (1.9e-10 instead of 2e-12).
+template <typename T>
+__device__ inline T sub_mul_re(T re, T lr, T li, T ur, T ui)
+{
+#pragma clang fp contract(off)
+    const T p = li * ui;
+    return re - fma_t(lr, ur, -p);
+}
+template <typename T>
+__device__ inline T sub_mul_im(T im, T lr, T li, T ur, T ui)
+{
+#pragma clang fp contract(off)
+    const T p = li * ur;
+    return im - fma_t(lr, ui, p);
+}
+
 // GEPP of the (n-k) x NB panel at column k for one matrix per blockIdx.y.
 // Workgroup w holds rows k + w*RW .. k + (w+1)*RW - 1 in registers.  A row is
 // split into TPR parts of W = NB/TPR columns held by different waves ("chunk"
-// c = wave / NWC), so that within a wave the column index is uniform:
-// finished columns are skipped by uniform branches, only the waves owning
-// column j take part in its argmax (a DPP reduction), and each thread carries
-// its row's value in the next pivot column (nxr, nxi), taken from the rank-1
-// update that produces it, so registers are only indexed statically.
+// c = wave / NWC), so that within a wave the column index is uniform: only
+// the waves owning column j take part in its argmax (a DPP reduction), and
+// each thread carries its row's value in the next pivot column (nxr, nxi),
+// taken from the update that produces it, so registers are only indexed
+// statically.
 //
 // Interchanges move labels, not data: each thread keeps its row and carries
 // the row's current position lr (initially the row itself).  Exchanging rows
@@ -162,16 +224,41 @@ __device__ inline int wave_min_i32(int v)
 // The arithmetic and the pivots are those of the interchanging algorithm
 // (ties go to the lowest position, as izamax), and each row is stored at its
 // final position at the end.
+//
+// A column costs a chain of latencies, not work (the panel's flops would take
+// a few microseconds on the CUs it occupies), so the chain is kept short:
+//  * each wave publishes its own candidate's slot as soon as its argmax is
+//    known, and its row right after: the candidate row is transposed through
+//    LDS, so that one lane per value brings it up to date (by the last column)
+//    and publishes it, before the wave updates all its rows;
+//  * that update (of the columns right of j by column j-1) and the reciprocal
+//    of the candidate's pivot run while the slots travel.  The update walks
+//    groups of G columns without branches, so a group's pivot-row reads from
+//    LDS are in flight together (a branch per column made each read's latency
+//    serial: half the time of a column);
+//  * after the pivot is known only its column's multipliers and the next
+//    column's values are computed before the next argmax;
+//  * the row of slot 0 is polled along with the slots, so a pivot near the
+//    diagonal (995 of 1000 columns of the wire matrices) costs one round trip;
+//  * a cluster of one workgroup exchanges nothing.
+// Measured per 64-column complex128 panel, pivots near the diagonal: 341 -> 144
+// us (one matrix of N = 512), 348 -> 158 us (two, N = 8192), 418 -> 204 us (16,
+// N = 8192, three workgroups per CU); random pivots 352 -> 165, 356 -> 180, 430
+// -> 225 us; complex64 panels (12 of N = 8192) 433 -> 207 us.  What is left of
+// a column's 2.3 us: the argmax and the candidate row (0.8 us), the packets'
+// way to memory and back (0.9 us; the same inside one XCD), the pivot row to
+// all waves and the next column (0.3 us).
 template <typename T, int TPR>
-__global__ __launch_bounds__(256, 3) void k_panel(PanelArgs<T> a)
+__global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
 {
     using V = typename CT<T>::V;
     constexpr int W = NB / TPR;     // columns per thread
-    constexpr int NWC = 4 / TPR;    // waves per chunk
+    constexpr int NWC = 4 / TPR;    // waves per chunk: candidates per workgroup
     constexpr int RW = 64 * NWC;    // rows per workgroup
-    constexpr int NW = XLayout<V>::NW;
-    constexpr int kNone = 0x7fffffff;
-    static_assert(NW <= 256 && NW % 64 == 0 && RW >= NB, "panel layout");
+    constexpr int NW = XLayout<V>::NW, NWS = XLayout<V>::NWS, SLS = XLayout<V>::SLS;
+    constexpr int G = kPanelGroup;  // columns updated together
+    constexpr int NE = NW / TPR / 2;  // values of a chunk's part of a row: one lane each (complex128: re and im apart)
+    static_assert(NE == 32 && RW >= NB && W % 8 == 0 && W % G == 0, "panel layout");
     const int bl = blockIdx.y, w = blockIdx.x;          // bl: member of this launch
     const int b = a.bidx ? a.bidx[bl] : bl;              // b: matrix index
     const int tid = threadIdx.x, lane = tid & 63;
@@ -181,7 +268,7 @@ __global__ __launch_bounds__(256, 3) void k_panel(PanelArgs<T> a)
     const int row = base + rb * 64 + lane;
     const bool valid = row < a.n;
     V *Ab = a.A + (size_t)b * a.strideA;
-    const XLayout<V> X(a.pmax);
+    const XLayout<V> X(a.slots);
     char *xm = a.xbuf + (size_t)bl * X.mat_bytes;
     if (a.nmem && k >= a.nmem[b]) {
         // the member's own matrix ends above this panel: an identity panel, no
@@ -200,170 +287,320 @@ __global__ __launch_bounds__(256, 3) void k_panel(PanelArgs<T> a)
         im[i] = x.y;
     }
 
+    // s_u, s_nx and the pivot's data alternate with the column parity: a wave
+    // may still use column j-1's pivot row while wave 0 writes column j's
     __shared__ double s_wv[NWC];
-    __shared__ int s_wr[NWC];
-    __shared__ V s_cand[NB];  // this workgroup's best row
-    __shared__ V s_u[NB];     // pivot row
-    __shared__ V s_l[TPR > 1 ? RW : 1];  // multipliers for the other chunks
-    __shared__ double s_gv;
-    __shared__ int s_gr;
-    __shared__ double2 s_rinv;  // reciprocal of the pivot
-    __shared__ int s_piv[NB];  // pivot row of each column (workgroup 0)
+    __shared__ int s_wr[NWC], s_wl[NWC];    // each row block's candidate: value, position, lane (-1: none)
+    __shared__ T s_cand[NWC][2][NB];        // its row, real and imaginary parts
+    __shared__ V s_u[2][NB];                // pivot row
+    __shared__ V s_nx[TPR > 1 ? 2 : 1][TPR > 1 ? RW : 1];  // values in the pivot column, for the other chunks
+    __shared__ double s_gv[2];
+    __shared__ int s_gr[2];
+    __shared__ double2 s_rinv[2];           // reciprocal of the pivot
+    __shared__ int s_piv[NB];               // pivot row of each column (workgroup 0)
 
     const uint32_t tag0 = *a.tagp + a.toff;
+    const bool solo = a.P == 1;
+    const int nslots = a.P * NWC;
     int lr = row;  // current position of this thread's row
     // this row's value in the column of the next step (column 0 is in chunk 0)
     T nxr = re[0], nxi = im[0];
+    T lre = 0, lim = 0;  // this row's multiplier of the last column
+    bool act = false;    // this row takes the last column's update
+    int zero = -1;       // first column with a zero pivot
     for (int j = 0; j < NB; ++j) {
         const int par = j & 1;
         const int pr = k + j;
         const int cj = j / W;
         const uint32_t tag = tag0 + (uint32_t)j + 1u;
+        uint64_t *slot = X.slot(xm, par);
+        uint64_t *cand = X.cand(xm, par);
 
         // 1. best row of each wave of the chunk holding column j: largest
         //    |re|+|im| among positions >= k+j, the lowest position on ties
+        //    (NaN is never a candidate); its slot is published at once
         if (c == cj) {
-            const double v = (valid && lr >= pr) ? fabs((double)nxr) + fabs((double)nxi) : -1.0;
-            const double m = wave_max_f64(v);
-            const int r = wave_min_i32(v == m && v >= 0.0 ? lr : kNone);
+            const double v = fabs((double)nxr) + fabs((double)nxi);
+            const int l = wave_best(v, lr, valid && lr >= pr && v == v);
+            const int ll = max(l, 0);
+            const double wv = l < 0 ? -1.0 : readlane_f64(v, ll);
+            const int wr = l < 0 ? kNoRow : __builtin_amdgcn_readlane(lr, ll);
+            if (!solo && lane < 3) {  // one store of three packets
+                const uint64_t bits = (uint64_t)__double_as_longlong(wv);
+                const uint32_t word = lane == 0 ? (uint32_t)bits : lane == 1 ? (uint32_t)(bits >> 32) : (uint32_t)wr;
+                put_pkt(slot + (w * NWC + rb) * SLS + lane, tag, word);
+            }
             if (lane == 0) {
-                s_wv[rb] = m;
-                s_wr[rb] = r;
+                s_wl[rb] = l;
+                if (solo) {
+                    s_wv[rb] = wv;
+                    s_wr[rb] = wr;
+                }
+            }
+            if (TPR > 1) s_nx[par][rb * 64 + lane] = V{nxr, nxi};
+        }
+        __syncthreads();
+        const int wl = __builtin_amdgcn_readfirstlane(s_wl[rb]);
+
+        // 2. the candidate's row from column j on, brought up to date, and the
+        //    reciprocal of its pivot; in a cluster of one workgroup the best
+        //    row block's is the pivot row
+        bool owner = true;
+        if (solo) {
+            double bv = s_wv[0];
+            int br = s_wr[0], bq = 0;
+#pragma unroll
+            for (int q = 1; q < NWC; ++q)
+                if (better(s_wv[q], s_wr[q], bv, br)) { bv = s_wv[q]; br = s_wr[q]; bq = q; }
+            owner = rb == __builtin_amdgcn_readfirstlane(bq);
+            if (tid == 0) {
+                const bool ok = br >= pr && br < a.n;  // else: a zero pivot in place
+                s_gv[par] = ok ? bv : 0.0;
+                s_gr[par] = ok ? br : pr;
             }
         }
-        __syncthreads();
-
-        // 2. this workgroup's candidate: its slot is published at once, so the
-        //    other workgroups' reductions start while the row is staged in LDS
-        double wv = s_wv[0];
-        int wr = s_wr[0];
-#pragma unroll
-        for (int q = 1; q < NWC; ++q)
-            if (better(s_wv[q], s_wr[q], wv, wr)) { wv = s_wv[q]; wr = s_wr[q]; }
-        uint64_t *slot = X.slot(xm, par);
-        uint64_t *cand = X.cand(xm, par);
-        if (tid < 3) {
-            const uint64_t bits = (uint64_t)__double_as_longlong(wv);
-            const uint32_t word = tid == 0 ? (uint32_t)bits : tid == 1 ? (uint32_t)(bits >> 32) : (uint32_t)wr;
-            put_pkt(slot + (size_t)w * 4 + tid, tag, word);
+        // the pivot's reciprocal: by a wave whose columns are finished, where
+        // there is one
+        if (wl >= 0 && owner && c == (cj > 0 ? cj - 1 : 0) && lane == 0) {
+            const V p = TPR > 1 ? s_nx[par][rb * 64 + wl] : V{readlane_t(nxr, wl), readlane_t(nxi, wl)};
+            const double2 rp = p.x != 0 || p.y != 0 ? crecip((double)p.x, (double)p.y) : make_double2(0.0, 0.0);
+            if (solo) {
+                s_rinv[par] = rp;
+            } else {
+                uint64_t *pq = cand + (w * NWC + rb) * NWS + NW;
+                const uint64_t xb = (uint64_t)__double_as_longlong(rp.x), yb = (uint64_t)__double_as_longlong(rp.y);
+                put_pkt(pq, tag, (uint32_t)xb);
+                put_pkt(pq + 1, tag, (uint32_t)(xb >> 32));
+                put_pkt(pq + 2, tag, (uint32_t)yb);
+                put_pkt(pq + 3, tag, (uint32_t)(yb >> 32));
+            }
         }
-        if (wr != kNone && lr == wr) {
+        if (wl >= 0 && owner && c >= cj) {
+            T *dre = s_cand[rb][0] + c * W, *dim = s_cand[rb][1] + c * W;
+            const bool upd = j > 0 && (sizeof(T) == 4 || __builtin_amdgcn_readlane((int)act, wl));
+            const T wlr = readlane_t(lre, wl), wli = readlane_t(lim, wl);
+            if (lane == wl) {
 #pragma unroll
-            for (int i = 0; i < W; ++i) s_cand[c * W + i] = V{re[i], im[i]};
+                for (int g = 0; g < W; g += 8)
+                    if (c * W + g + 7 >= j) {
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) {
+                            dre[g + q] = re[g + q];
+                            dim[g + q] = im[g + q];
+                        }
+                    }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            uint64_t *pc = cand + (w * NWC + rb) * NWS + 2 * c * NE + lane;
+            if constexpr (sizeof(T) == 8) {  // two lanes per column: real and imaginary part
+                const bool imag = lane & 1;
+                const int i = (lane % NE) / 2, col = c * W + i;
+                double x = imag ? dim[i] : dre[i];
+                const V u = s_u[par ^ 1][col];
+                if (upd) {
+                    // sub_mul_re or sub_mul_im
+                    x = sub_mul_im(x, wlr, imag ? wli : -wli, imag ? u.x : u.y, imag ? u.y : u.x);
+                }
+                if (lane < NE && col >= j) {
+                    if (solo) {
+                        ((double *)s_u[par])[2 * col + imag] = x;
+                    } else {
+                        const uint64_t xb = (uint64_t)__double_as_longlong(x);
+                        put_pkt(pc, tag, (uint32_t)xb);
+                        put_pkt(pc + NE, tag, (uint32_t)(xb >> 32));
+                    }
+                }
+            } else {  // one lane per column
+                const int i = lane % NE, col = c * W + i;
+                V x = V{dre[i], dim[i]};
+                const V u = s_u[par ^ 1][col];
+                if (upd) {
+                    x = V{sub_mul_re(x.x, wlr, wli, u.x, u.y), sub_mul_im(x.y, wlr, wli, u.x, u.y)};
+                }
+                if (lane < NE && col >= j) {
+                    if (solo) {
+                        s_u[par][col] = x;
+                    } else {
+                        put_pkt(pc, tag, (uint32_t)__float_as_int(x.x));
+                        put_pkt(pc + NE, tag, (uint32_t)__float_as_int(x.y));
+                    }
+                }
+            }
         }
-        __syncthreads();
 
-        // 3. publish the candidate row
-        if (tid < NW) put_pkt(cand + (size_t)w * NW + tid, tag, ((const uint32_t *)s_cand)[tid]);
+        // 3. column j-1's multipliers and its update of the columns from j on.
+        //    complex64 factors: rows that take no update have a zero
+        //    multiplier, so the update needs no per-row branch (a non-finite
+        //    pivot row then spreads to finished rows, and the refinement of
+        //    such factors fails over to FP64 factors); complex128 factors keep
+        //    LAPACK's untouched finished rows
+        if (j > 0 && (sizeof(T) == 4 || act)) {
+            const V *su = s_u[par ^ 1] + c * W;
+            const int jc = j - 1 - c * W;
+            auto upd = [&](int i, const V &u) {
+                re[i] = sub_mul_re(re[i], lre, lim, u.x, u.y);
+                im[i] = sub_mul_im(im[i], lre, lim, u.x, u.y);
+            };
+#pragma unroll
+            for (int g = 0; g < W; g += G) {
+                if (g > jc) {
+                    V u[G];
+#pragma unroll
+                    for (int q = 0; q < G; ++q) u[q] = su[g + q];
+#pragma unroll
+                    for (int q = 0; q < G; ++q) upd(g + q, u[q]);
+                } else if (g + G > jc) {
+#pragma unroll
+                    for (int q = 0; q < G; ++q) {
+                        if (g + q > jc) upd(g + q, su[g + q]);
+                        if (g + q == jc && act) {
+                            re[g + q] = lre;
+                            im[g + q] = lim;
+                        }
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the next column's values before column j's update
+        T xr = 0, xi = 0;
+        {
+            const int jn = j + 1 - c * W;
+#pragma unroll
+            for (int g = 0; g < W; g += 8)
+                if (jn >= g && jn < g + 8) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        if (g + q == jn) {
+                            xr = re[g + q];
+                            xi = im[g + q];
+                        }
+                }
+        }
 
         // 4. wave 0 reduces all candidates to the same pivot (first max), then
-        //    fetches the pivot row from the workgroup holding it and takes the
-        //    pivot's reciprocal, so one barrier hands everything to the others
-        if (wave == 0) {
+        //    fetches the pivot row and reciprocal of the winner; one barrier
+        //    hands everything to the others
+        if (!solo && wave == 0) {
+            // The row of slot 0 (the panel's top 64 rows) is polled along with the
+            // slots: it is the pivot row in 995 of 1000 columns of the wire
+            // matrices, whose pivots stay near the diagonal.
+            constexpr int PL = NW / 64;  // pivot-row words per lane, loaded together
+            uint64_t wu[PL], wi;
+            auto val = [&](int e) { return e * NE + lane % NE; };  // value whose word this lane takes
+            auto load_row = [&](int sl) {
+                const uint64_t *pu = cand + sl * NWS;
+#pragma unroll
+                for (int e = 0; e < PL; ++e) wu[e] = ld_pkt(pu + lane + 64 * e);
+                wi = ld_pkt(pu + NW + (lane & 3));
+            };
+            auto row_ready = [&]() {
+                bool got = (uint32_t)(wi >> 32) == tag;
+#pragma unroll
+                for (int e = 0; e < PL; ++e)  // columns left of j are not published
+                    got = got && ((uint32_t)(wu[e] >> 32) == tag || (sizeof(T) == 8 ? val(e) / 2 : val(e)) < j);
+                return __all(got) != 0;
+            };
             double gv = -1.0;
-            int gr = kNone, gs = 0;
-            for (int s = lane; s < a.P; s += 64) {
-                const uint64_t *ps = slot + (size_t)s * 4;
-                uint64_t w0, w1, w2;
+            int gr = kNoRow, gs = 0;
+            for (int s0 = 0; s0 < nslots; s0 += 128) {  // two slots per lane at a time
+                uint64_t w0[2], w1[2], w2[2];
                 long it = 0;
                 for (;;) {
-                    w0 = ld_pkt(ps);
-                    w1 = ld_pkt(ps + 1);
-                    w2 = ld_pkt(ps + 2);
-                    if ((uint32_t)(w0 >> 32) == tag && (uint32_t)(w1 >> 32) == tag && (uint32_t)(w2 >> 32) == tag)
-                        break;
+                    bool got = true;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int s = s0 + 64 * h + lane;
+                        if (s < nslots) {
+                            const uint64_t *ps = slot + s * SLS;
+                            w0[h] = ld_pkt(ps);
+                            w1[h] = ld_pkt(ps + 1);
+                            w2[h] = ld_pkt(ps + 2);
+                        }
+                    }
+                    load_row(0);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        if (s0 + 64 * h + lane < nslots)
+                            got = got && (uint32_t)(w0[h] >> 32) == tag && (uint32_t)(w1[h] >> 32) == tag &&
+                                  (uint32_t)(w2[h] >> 32) == tag;
+                    if (__all(got)) break;
                     if (spin_give_up(it, a.err)) break;
                 }
-                const double v2 = __longlong_as_double((long long)(((w1 & 0xffffffffull) << 32) | (w0 & 0xffffffffull)));
-                const int r2 = (int)(uint32_t)w2;
-                if (better(v2, r2, gv, gr)) { gv = v2; gr = r2; gs = s; }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int s = s0 + 64 * h + lane;
+                    if (s < nslots) {
+                        const double v2 = __longlong_as_double(
+                            (long long)(((w1[h] & 0xffffffffull) << 32) | (w0[h] & 0xffffffffull)));
+                        const int r2 = (int)(uint32_t)w2[h];
+                        if (better(v2, r2, gv, gr)) { gv = v2; gr = r2; gs = s; }
+                    }
+                }
             }
-            const double m = wave_max_f64(gv);
-            const int r = wave_min_i32(gv == m ? gr : kNone);
-            const unsigned long long win = __ballot(gv == m && gr == r);
-            const int ws = __builtin_amdgcn_readlane(gs, win ? (int)__builtin_ctzll(win) : 0);
+            const int l = wave_best(gv, gr, gr != kNoRow);
+            const int r = l >= 0 ? __builtin_amdgcn_readlane(gr, l) : kNoRow;
             // no usable candidate (non-finite column): a zero pivot in place
             const bool ok = r >= pr && r < a.n;
-            constexpr int PL = NW / 64;  // pivot-row words per lane, loaded together
-            const uint64_t *pu = cand + (size_t)(ok ? ws : 0) * NW + lane;
-            uint64_t wu[PL];
-            long it = 0;
-            for (;;) {
-                bool got = true;
-#pragma unroll
-                for (int e = 0; e < PL; ++e) {
-                    wu[e] = ld_pkt(pu + 64 * e);
-                    got = got && (uint32_t)(wu[e] >> 32) == tag;
+            double2 rinv = make_double2(0.0, 0.0);
+            double m = 0.0;
+            if (ok) {
+                m = readlane_f64(gv, l);
+                const int ws = __builtin_amdgcn_readlane(gs, l);
+                long it = 0;
+                if (ws != 0) load_row(ws);
+                while (!row_ready()) {
+                    if (spin_give_up(it, a.err)) break;
+                    load_row(ws);
                 }
-                if (got) break;
-                if (spin_give_up(it, a.err)) break;
-            }
 #pragma unroll
-            for (int e = 0; e < PL; ++e) ((uint32_t *)s_u)[lane + 64 * e] = (uint32_t)wu[e];
+                for (int e = 0; e < PL; ++e) ((uint32_t *)s_u[par])[2 * val(e) + lane / NE] = (uint32_t)wu[e];
+                const uint32_t ri = (uint32_t)wi;
+                auto word = [&](int q) { return (unsigned long long)(unsigned)__builtin_amdgcn_readlane(ri, q); };
+                rinv.x = __longlong_as_double((long long)((word(1) << 32) | word(0)));
+                rinv.y = __longlong_as_double((long long)((word(3) << 32) | word(2)));
+            }
             if (lane == 0) {
-                s_gv = ok ? m : 0.0;
-                s_gr = ok ? r : pr;
-                const V p = s_u[j];  // written by this wave above
-                s_rinv = ok && m != 0.0 ? crecip((double)p.x, (double)p.y) : make_double2(0.0, 0.0);
+                s_gv[par] = m;
+                s_gr[par] = ok ? r : pr;
+                s_rinv[par] = rinv;
             }
         }
         __syncthreads();
-        const double gv = s_gv;
-        const int gr = s_gr;
-
-        // 5. interchange positions k+j and gr, scale column j, rank-1 update
-        const double2 rinv = s_rinv;
-        if (w == 0 && tid == 0) {
-            s_piv[j] = gr;
-            a.ipiv[(size_t)b * a.strideP + pr] = gr + 1;
-            if (gv == 0.0 && a.info[b] == 0) a.info[b] = pr + 1;
+        const double gv = s_gv[par];
+        const int gr = s_gr[par];
+        const double2 rinv = s_rinv[par];
+        const V un = s_u[par][j + 1 < NB ? j + 1 : j];
+        if (TPR > 1 && c != cj) {
+            const V x = s_nx[par][rb * 64 + lane];
+            nxr = x.x;
+            nxi = x.y;
         }
+
+        // 5. interchange positions k+j and gr, the multipliers of column j,
+        //    and the next column's values for the next argmax
+        if (tid == 0) s_piv[j] = gr;
+        if (gv == 0.0 && zero < 0) zero = pr;
         if (lr == gr) lr = pr;
         else if (lr == pr) lr = gr;
-        const bool act = gv != 0.0 && valid && lr > pr;
-        T lre = 0, lim = 0;
-        if (c == cj) {
-            if (act) {
-                lre = (T)((double)nxr * rinv.x - (double)nxi * rinv.y);
-                lim = (T)((double)nxr * rinv.y + (double)nxi * rinv.x);
-            }
-            if (TPR > 1) s_l[rb * 64 + lane] = V{lre, lim};
+        act = gv != 0.0 && valid && lr > pr;
+        lre = lim = 0;
+        if (act) {
+            lre = (T)((double)nxr * rinv.x - (double)nxi * rinv.y);
+            lim = (T)((double)nxr * rinv.y + (double)nxi * rinv.x);
         }
-        if (TPR > 1) {
-            __syncthreads();
-            if (c != cj) {
-                const V l = s_l[rb * 64 + lane];
-                lre = l.x;
-                lim = l.y;
-            }
+        nxr = xr;
+        nxi = xi;
+        if (sizeof(T) == 4 || act) {
+            nxr = sub_mul_re(xr, lre, lim, un.x, un.y);
+            nxi = sub_mul_im(xi, lre, lim, un.x, un.y);
         }
-#pragma unroll
-        for (int i = 0; i < W; ++i) {
-            const int col = c * W + i;  // uniform
-            if (col == j) {             // the multiplier replaces column j
-                if (act) {
-                    re[i] = lre;
-                    im[i] = lim;
-                }
-            } else if (col > j) {
-                // complex64 factors: rows that take no update have a zero
-                // multiplier, so the update needs no per-row branch (a
-                // non-finite pivot row then spreads to finished rows, and the
-                // refinement of such factors fails over to FP64 factors);
-                // complex128 factors keep LAPACK's untouched finished rows
-                if (sizeof(T) == 4 || act) {
-                    const V u = s_u[col];
-                    re[i] -= lre * u.x - lim * u.y;
-                    im[i] -= lre * u.y + lim * u.x;
-                }
-                if (col == j + 1) {
-                    nxr = re[i];
-                    nxi = im[i];
-                }
-            }
-            // keep the scheduler from hoisting every column's pivot-row load at once
-            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-        }
+    }
+    if (c == TPR - 1 && act) {  // the last column's multipliers
+        re[W - 1] = lre;
+        im[W - 1] = lim;
     }
 
     // each row to its final position
@@ -378,6 +615,8 @@ __global__ __launch_bounds__(256, 3) void k_panel(PanelArgs<T> a)
     // workgroup 0 keeps slot t and slot NB + t in lane t (NB is the wave
     // width), so each interchange is a ballot and two lane reads.
     __syncthreads();  // s_piv complete
+    if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
+    if (w == 0 && tid == 0 && zero >= 0 && a.info[b] == 0) a.info[b] = zero + 1;
     if (w == 0 && wave == 0) {
         static_assert(NB == 64, "one slot pair per lane");
         const int rlo = k + lane;
@@ -428,7 +667,7 @@ __global__ __launch_bounds__(256, 3) void k_panel(PanelArgs<T> a)
 //   [ntl+ntr, ...)     columns [c_sw0, n): interchanges only (columns whose
 //                      rows k..k+NB-1 still await earlier panels' updates)
 struct SwapArgs {
-    int n, k, pmax, ntl, ntr, c_tr0, c_tr1, c_sw0, do_swap;
+    int n, k, slots, ntl, ntr, c_tr0, c_tr1, c_sw0, do_swap;
     const int *nmem;  // per matrix index: its own size (identity beyond), or null
 };
 
@@ -444,7 +683,7 @@ __global__ __launch_bounds__(256) void k_swap_trsm(typename CT<T>::V *A, int lda
     const int b = bidx ? bidx[bl] : bl;
     const int n = a.n, k = a.k;
     V *Ab = A + (size_t)b * strideA;
-    const XLayout<V> X(a.pmax);
+    const XLayout<V> X(a.slots);
     char *xm = xbuf + (size_t)bl * X.mat_bytes;
 
     const bool trsm = tile >= a.ntl && tile < a.ntl + a.ntr;
@@ -1078,7 +1317,7 @@ int occupancy_panel(int *blocks_per_cu)
 // tall panels go in several launches and short ones in one, and each member
 // has its own exchange buffer.
 struct GetrfPlan {
-    int pmax = 0, resident = 0, per_launch = 0;
+    int pmax = 0, slots = 0, resident = 0, per_launch = 0;
     size_t xbytes = 0;
 };
 
@@ -1103,7 +1342,8 @@ int getrf_plan(wm_ctx *ctx, int n, int batch, GetrfPlan *pl)
     pl->pmax = pmax;
     pl->resident = resident;
     pl->per_launch = std::min(batch, resident / pmax);
-    pl->xbytes = (size_t)batch * XLayout<V>(pmax).mat_bytes;
+    pl->slots = pmax * (RW / 64);
+    pl->xbytes = (size_t)batch * XLayout<V>(pl->slots).mat_bytes;
     return WM_OK;
 }
 
@@ -1117,8 +1357,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
     using V = typename CT<T>::V;
     constexpr int RW = 256 / TPR;
     constexpr int CB = (sizeof(T) == 8) ? 16 : 32;
-    const int pmax = pl.pmax;
-    const XLayout<V> X(pmax);
+    const XLayout<V> X(pl.slots);
     char *xbase = (char *)ctx->ws_lu.ptr;
     const double esz = 2.0 * sizeof(T);
     const int kPanelClass = sizeof(T) == 8 ? K_PANEL : K_PANEL32;
@@ -1146,7 +1385,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
             PanelArgs<T> pa;
             pa.A = G.bidx ? G.Ab : G.Ab + (size_t)b0 * strideA;
             pa.lda = lda; pa.strideA = strideA; pa.n = n; pa.k = c;
-            pa.P = P; pa.pmax = pmax;
+            pa.P = P; pa.slots = pl.slots;
             pa.ipiv = G.bidx ? G.ipb : G.ipb + (size_t)b0 * strideP;
             pa.strideP = strideP;
             pa.info = G.bidx ? G.infob : G.infob + b0;
@@ -1165,7 +1404,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
     // interchanges of the panel at c left of c; solve for [tr0, tr1); interchanges only for [tr1, n)
     auto swap = [&](const Grp &G, int c, int tr1, int do_swap, int tr0) {
         SwapArgs sa;
-        sa.n = n; sa.k = c; sa.pmax = pmax; sa.do_swap = do_swap;
+        sa.n = n; sa.k = c; sa.slots = pl.slots; sa.do_swap = do_swap;
         sa.nmem = d_nmem;
         sa.ntl = do_swap ? (c + CB - 1) / CB : 0;
         sa.c_tr0 = tr0; sa.c_tr1 = tr1;
@@ -1244,8 +1483,8 @@ int getrf_width(wm_ctx *ctx, int prec, int n)
 {
     int bpc = 0;
     const bool f64 = prec == WM_PREC_F64;  // complex64 factors (FP32, BF16X3) share the FP32 panel
-    if ((f64 ? occupancy_panel<double, 2>(&bpc) : occupancy_panel<float, kTprF32>(&bpc)) != WM_OK || bpc <= 0) return 1;
-    const int RW = f64 ? 128 : 256 / kTprF32;
+    if ((f64 ? occupancy_panel<double, kTprF64>(&bpc) : occupancy_panel<float, kTprF32>(&bpc)) != WM_OK || bpc <= 0) return 1;
+    const int RW = 256 / (f64 ? kTprF64 : kTprF32);
     const int pmax = (n + RW - 1) / RW;
     return std::max(1, bpc * ctx->num_cu / std::max(1, ctx->panel_share) / pmax);
 }
@@ -1343,7 +1582,7 @@ int getrf_batched(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t stride
         return WM_ERR_ARG;
     }
     if (prec == WM_PREC_F64)
-        return getrf_run<double, 2>(ctx, prec, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, 8, d_nmem);
+        return getrf_run<double, kTprF64>(ctx, prec, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, 8, d_nmem);
     if (prec == WM_PREC_F32)
         return getrf_run<float, kTprF32>(ctx, prec, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, 4,
                                          d_nmem);
@@ -1431,26 +1670,26 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         using T = decltype(tag);
         using V = typename CT<T>::V;
         const int RW = 256 / TPRv;
-        const int pmax = (n + RW - 1) / RW;
-        const XLayout<V> X(pmax);
+        const int slots = (n + RW - 1) / RW * (RW / 64);
+        const XLayout<V> X(slots);
         WM_TRY(prepare_xbuf(ctx, X.mat_bytes, (uint64_t)n, ctx->stream));
         char *xbuf = (char *)ctx->ws_lu.ptr;
         hipLaunchKernelGGL(k_tag_bump, dim3(1), dim3(64), 0, ctx->stream, ctx->d_tag, (uint32_t)n);
         ctx->panel_tag += (uint64_t)n;
         PanelArgs<T> pa;
         pa.A = (V *)Ap; pa.lda = n; pa.strideA = 0; pa.n = n; pa.k = k;
-        pa.P = (n - k + RW - 1) / RW; pa.pmax = pmax;
+        pa.P = (n - k + RW - 1) / RW; pa.slots = slots;
         pa.ipiv = ipiv; pa.strideP = 0; pa.info = info;
         pa.err = ctx->d_err; pa.xbuf = xbuf; pa.bidx = nullptr; pa.tagp = ctx->d_tag; pa.toff = (uint32_t)k;
         pa.nmem = nullptr;
         constexpr int CB = (sizeof(T) == 8) ? 16 : 32;
         if (sizeof(T) == 8)
-            hipLaunchKernelGGL((k_panel<double, 2>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<double> *)&pa);
+            hipLaunchKernelGGL((k_panel<double, kTprF64>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<double> *)&pa);
         else
             hipLaunchKernelGGL((k_panel<float, kTprF32>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<float> *)&pa);
         if (do_swap) {
             SwapArgs sa;
-            sa.n = n; sa.k = k; sa.pmax = pmax; sa.do_swap = 1; sa.nmem = nullptr;
+            sa.n = n; sa.k = k; sa.slots = slots; sa.do_swap = 1; sa.nmem = nullptr;
             sa.ntl = (k + CB - 1) / CB;
             sa.ntr = (n - k - NB + CB - 1) / CB;
             sa.c_tr0 = k + NB; sa.c_tr1 = n; sa.c_sw0 = n;
@@ -1460,7 +1699,7 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         }
         return WM_OK;
     };
-    int rc = (prec == WM_PREC_F64) ? run(double(0), (double2 *)A, 2) : run(float(0), (float2 *)A, kTprF32);
+    int rc = (prec == WM_PREC_F64) ? run(double(0), (double2 *)A, kTprF64) : run(float(0), (float2 *)A, kTprF32);
     WM_HIP_TRY(hipStreamSynchronize(ctx->stream));
     (void)hipFree(info);
     if (rc != WM_OK) return rc;

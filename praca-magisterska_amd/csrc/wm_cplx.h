@@ -46,30 +46,9 @@ __device__ inline bool spin_give_up(long &it, int *err)
     return false;
 }
 
-// Reciprocal of a complex number, conj(z) / |z|^2 on z scaled by a power of two
-// to a largest part in [1/2, 1): |z|^2 and its rounding error in two words, one
-// hardware reciprocal refined by Newton steps, its remainder and the products'
-// rounding errors folded into one last addition per part: within 0.51 ulp of
-// the exact value (Smith's algorithm, three chained divisions: 1.4 ulp) in
-// about a quarter of the dependent steps.  Zero and non-finite numbers take
-// Smith's (1962) path.
+// Smith (1962) reciprocal of a complex number.
 __device__ inline double2 crecip(double re, double im)
 {
-    const double big = fmax(fabs(re), fabs(im));
-    if (big > 0.0 && big < __builtin_inf() && re == re && im == im) {
-        const int e = -__builtin_amdgcn_frexp_exp(big);
-        const double a = __builtin_amdgcn_ldexp(re, e), b = __builtin_amdgcn_ldexp(im, e);
-        const double aa = a * a, bb = b * b, d = aa + bb;
-        const double lo = fmin(aa, bb) - (d - fmax(aa, bb));
-        const double de = lo + (__builtin_fma(a, a, -aa) + __builtin_fma(b, b, -bb));
-        double r = __builtin_amdgcn_rcp(d);
-        r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-        r = __builtin_fma(r, __builtin_fma(-de, r, __builtin_fma(-d, r, 1.0)), r);
-        const double q = __builtin_fma(-de, r, __builtin_fma(-d, r, 1.0));
-        const double x = a * r, y = -b * r;
-        return make_double2(__builtin_amdgcn_ldexp(x + __builtin_fma(x, q, __builtin_fma(a, r, -x)), e),
-                            __builtin_amdgcn_ldexp(y + __builtin_fma(y, q, __builtin_fma(-b, r, -y)), e));
-    }
     if (fabs(re) >= fabs(im)) {
         const double t = im / re, d = re + im * t;
         return make_double2(1.0 / d, -t / d);

@@ -204,8 +204,15 @@ template <typename T>
 __device__ inline T sub_mul_im(T im, T lr, T li, T ur, T ui)
 {
 #pragma clang fp contract(off)
-    const T p = li * ur;
-    return im - fma_t(lr, ui, p);
+    const T p = lr * ui;
+    return im - fma_t(li, ur, p);
+}
+// (ar, ai) * (br, bi), rounded alike
+__device__ inline double2 mul_c(double ar, double ai, double br, double bi)
+{
+#pragma clang fp contract(off)
+    const double p = ai * bi, q = ar * bi;
+    return make_double2(fma_t(ar, br, -p), fma_t(ai, br, q));
 }
 
 // GEPP of the (n-k) x NB panel at column k for one matrix per blockIdx.y.
@@ -401,7 +408,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
                 const V u = s_u[par ^ 1][col];
                 if (upd) {
                     // sub_mul_re or sub_mul_im
-                    x = sub_mul_im(x, wlr, imag ? wli : -wli, imag ? u.x : u.y, imag ? u.y : u.x);
+                    x = sub_mul_im(x, imag ? wlr : -wli, imag ? wli : wlr, u.x, u.y);
                 }
                 if (lane < NE && col >= j) {
                     if (solo) {
@@ -588,8 +595,9 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         act = gv != 0.0 && valid && lr > pr;
         lre = lim = 0;
         if (act) {
-            lre = (T)((double)nxr * rinv.x - (double)nxi * rinv.y);
-            lim = (T)((double)nxr * rinv.y + (double)nxi * rinv.x);
+            const double2 l = mul_c((double)nxr, (double)nxi, rinv.x, rinv.y);
+            lre = (T)l.x;
+            lim = (T)l.y;
         }
         nxr = xr;
         nxi = xi;

@@ -434,6 +434,72 @@ int wm_memcpy_d2d(wm_ctx *c, void *dst, const void *src, size_t bytes)
 }
 
 // ---- geometry -------------------------------------------------------------------
+namespace {
+
+// The fill's row tables (wm_geom): rows 0..ld-1 cut into runs of at most 64 rows
+// with at most 64 distinct observation points (equal coordinates and segment key).
+struct FillRows {
+    std::vector<int> wrow, pkey, slots;
+    std::vector<double> pts;
+};
+
+void fill_rows(const std::vector<double> &obs, const std::vector<int> &okey, int npls, int ld, FillRows &t)
+{
+    struct Pt {
+        double r[3];
+        int key;
+    };
+    std::vector<Pt> cur;
+    t.slots.assign(ld, 0);
+    t.wrow.assign(1, 0);
+    auto point = [&](int m, int h) {
+        Pt p;
+        for (int d = 0; d < 3; ++d) p.r[d] = obs[(size_t)(6 * h + d) * ld + m];
+        p.key = okey[(size_t)h * ld + m];
+        return p;
+    };
+    auto find = [&](const Pt &p) {  // the newest points first: a row shares one with the row before it
+        for (int i = (int)cur.size() - 1; i >= 0; --i)
+            if (cur[i].key == p.key && std::memcmp(cur[i].r, p.r, sizeof p.r) == 0) return i;
+        return -1;
+    };
+    auto close = [&](int row_end) {
+        const size_t w = t.wrow.size() - 1;
+        t.pts.resize((w + 1) * 3 * 64);
+        t.pkey.resize((w + 1) * 64);
+        for (int l = 0; l < 64; ++l) {  // lanes without a point repeat one, with no segment's key
+            const bool own = l < (int)cur.size();
+            const Pt p = own ? cur[l] : cur.empty() ? point(0, 0) : cur[0];
+            for (int d = 0; d < 3; ++d) t.pts[(w * 3 + d) * 64 + l] = p.r[d];
+            t.pkey[w * 64 + l] = own ? p.key : -1;
+        }
+        t.wrow.push_back(row_end);
+        cur.clear();
+    };
+    for (int m = 0; m < ld; ++m) {
+        int slot[2] = {0, 0};
+        for (int pass = 0; pass < 2; ++pass) {  // pass 1: the row opens a new run
+            const size_t had = cur.size();
+            if (m < npls)
+                for (int h = 0; h < 2; ++h) {
+                    const Pt p = point(m, h);
+                    slot[h] = find(p);
+                    if (slot[h] < 0) {
+                        slot[h] = (int)cur.size();
+                        cur.push_back(p);
+                    }
+                }
+            if (cur.size() <= 64 && m - t.wrow.back() < 64) break;
+            cur.resize(had);
+            close(m);
+        }
+        t.slots[m] = slot[0] | slot[1] << 8;
+    }
+    close(ld);
+}
+
+}  // namespace
+
 int wm_geom_create(wm_ctx *c, const float *x, const float *y, const float *z, const float *rad, const int *ipc,
                    const int *ips, const int *ise, int nsmax, int npls, wm_geom **out)
 {
@@ -456,7 +522,7 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
     (void)hipSetDevice(c->device);
     const int ld = round_up(npls, 128);
     std::vector<double> obs((size_t)12 * ld, 0.0), src((size_t)16 * ld, 0.0), img;
-    std::vector<int> okey((size_t)2 * ld, -1), skey((size_t)2 * ld, -2), ikey;
+    std::vector<int> okey((size_t)2 * ld, -1), skey((size_t)4 * ld, -2), ikey;
     const bool pec = ienv == 2;
     if (pec) {
         img.assign((size_t)16 * ld, 0.0);
@@ -496,8 +562,8 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
         const int k1 = seg_key(s1), k2 = seg_key(s2);
         okey[p] = k1;
         okey[ld + p] = k2;
-        skey[2 * p] = k1;
-        skey[2 * p + 1] = k2;
+        skey[4 * p] = k1;
+        skey[4 * p + 1] = k2;
         // source half 1: first node of s1 -> peak; half 2: peak -> second node of s2
         double *r = &src[(size_t)p * 16];
         const double *A[2] = {F1, P}, *B[2] = {P, F2};
@@ -526,7 +592,7 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
                 q[8 * g + 6] = r[8 * g + 6];
                 q[8 * g + 7] = r[8 * g + 7];
                 const int s = segs[g], na = ise[s - 1], nb = ise[s - 1 + nsmax];
-                if ((double)z[na - 1] < 1.e-6 && (double)z[nb - 1] < 1.e-6) ikey[2 * p + g] = skey[2 * p + g];
+                if ((double)z[na - 1] < 1.e-6 && (double)z[nb - 1] < 1.e-6) ikey[2 * p + g] = skey[4 * p + g];
             }
         }
     }
@@ -539,6 +605,19 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
         }
         for (int d = 0; d < 12; ++d) obs[(size_t)d * ld + p] = 1.0e3;
     }
+    // first halves that are not the previous basis's second half (same record,
+    // key and image): along a wire the fill evaluates each segment once
+    for (int p = 0; p < ld; ++p) {
+        bool same = p > 0 && p < npls && skey[4 * p] == skey[4 * (p - 1) + 1] &&
+                    std::memcmp(&src[(size_t)p * 16], &src[(size_t)(p - 1) * 16 + 8], 8 * sizeof(double)) == 0;
+        if (pec && same)
+            same = ikey[2 * p] == ikey[2 * (p - 1) + 1] &&
+                   std::memcmp(&img[(size_t)p * 16], &img[(size_t)(p - 1) * 16 + 8], 8 * sizeof(double)) == 0;
+        skey[4 * p + 2] = same ? 0 : 1;
+        skey[4 * p + 3] = 0;
+    }
+    FillRows fr;
+    fill_rows(obs, okey, npls, ld, fr);
     // diameter of the structure (with its image over the PEC ground): the
     // bounding-box diagonal of every source half
     double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
@@ -564,7 +643,10 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
     g->sgnenv = (double)sgnenv;
     if (hipMalloc(&g->d_obs, obs.size() * sizeof(double)) != hipSuccess ||
         hipMalloc(&g->d_src, src.size() * sizeof(double)) != hipSuccess ||
-        hipMalloc(&g->d_obs_key, okey.size() * sizeof(int)) != hipSuccess ||
+        hipMalloc(&g->d_wrow, fr.wrow.size() * sizeof(int)) != hipSuccess ||
+        hipMalloc(&g->d_pts, fr.pts.size() * sizeof(double)) != hipSuccess ||
+        hipMalloc(&g->d_pkey, fr.pkey.size() * sizeof(int)) != hipSuccess ||
+        hipMalloc(&g->d_slots, fr.slots.size() * sizeof(int)) != hipSuccess ||
         hipMalloc(&g->d_src_key, skey.size() * sizeof(int)) != hipSuccess ||
         (pec && (hipMalloc(&g->d_img, img.size() * sizeof(double)) != hipSuccess ||
                  hipMalloc(&g->d_img_key, ikey.size() * sizeof(int)) != hipSuccess))) {
@@ -578,7 +660,11 @@ int wm_geom_create_env(wm_ctx *c, const float *x, const float *y, const float *z
     }
     WM_HIP_TRY(hipMemcpy(g->d_obs, obs.data(), obs.size() * sizeof(double), hipMemcpyHostToDevice));
     WM_HIP_TRY(hipMemcpy(g->d_src, src.data(), src.size() * sizeof(double), hipMemcpyHostToDevice));
-    WM_HIP_TRY(hipMemcpy(g->d_obs_key, okey.data(), okey.size() * sizeof(int), hipMemcpyHostToDevice));
+    g->nwaves = (int)fr.wrow.size() - 1;
+    WM_HIP_TRY(hipMemcpy(g->d_wrow, fr.wrow.data(), fr.wrow.size() * sizeof(int), hipMemcpyHostToDevice));
+    WM_HIP_TRY(hipMemcpy(g->d_pts, fr.pts.data(), fr.pts.size() * sizeof(double), hipMemcpyHostToDevice));
+    WM_HIP_TRY(hipMemcpy(g->d_pkey, fr.pkey.data(), fr.pkey.size() * sizeof(int), hipMemcpyHostToDevice));
+    WM_HIP_TRY(hipMemcpy(g->d_slots, fr.slots.data(), fr.slots.size() * sizeof(int), hipMemcpyHostToDevice));
     WM_HIP_TRY(hipMemcpy(g->d_src_key, skey.data(), skey.size() * sizeof(int), hipMemcpyHostToDevice));
     *out = g;
     return WM_OK;
@@ -626,7 +712,10 @@ int wm_geom_destroy(wm_geom *g)
     if (!g) return WM_OK;
     if (g->d_obs) (void)hipFree(g->d_obs);
     if (g->d_src) (void)hipFree(g->d_src);
-    if (g->d_obs_key) (void)hipFree(g->d_obs_key);
+    if (g->d_wrow) (void)hipFree(g->d_wrow);
+    if (g->d_pts) (void)hipFree(g->d_pts);
+    if (g->d_pkey) (void)hipFree(g->d_pkey);
+    if (g->d_slots) (void)hipFree(g->d_slots);
     if (g->d_src_key) (void)hipFree(g->d_src_key);
     if (g->d_img) (void)hipFree(g->d_img);
     if (g->d_img_key) (void)hipFree(g->d_img_key);

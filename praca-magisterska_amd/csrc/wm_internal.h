@@ -132,9 +132,16 @@ struct wm_geom {
     int ld = 0;       // padded size (multiple of 128)
     double diam = 0;  // bounding-box diagonal of the structure (with its image over the PEC ground), m
     double *d_obs = nullptr;   // 12 arrays of ld doubles: rc1xyz, lm1xyz, rc2xyz, lm2xyz
-    int *d_obs_key = nullptr;  // 2 arrays of ld ints: segment key of obs half 1, 2
+    // fill: runs of rows ("waves") whose observation points (segment centres)
+    // are at most 64 distinct ones, padding rows included
+    int nwaves = 0;
+    int *d_wrow = nullptr;    // nwaves + 1 first rows
+    double *d_pts = nullptr;  // per wave 3 x 64 doubles: its points' x, y, z (unused lanes repeat one)
+    int *d_pkey = nullptr;    // per wave 64 ints: their segment keys
+    int *d_slots = nullptr;   // ld ints: lanes of a row's two points in its wave, first | second << 8
     double *d_src = nullptr;   // ld records of 16 doubles: rs1[3] dc1[3] dl1 an1 rs2[3] dc2[3] dl2 an2
-    int *d_src_key = nullptr;  // ld records of 2 ints
+    int *d_src_key = nullptr;  // ld records of 4 ints: segment keys of the halves, 1 if half 1 differs from the
+                               // previous basis's half 2, 0
     // PEC ground (ienv 2): image records (coordinates and directions scaled by
     // sgnx, sgny, sgnz) laid out as d_src, image terms weighted by sgnenv; an
     // image half's key is its segment key when the self rule applies to it

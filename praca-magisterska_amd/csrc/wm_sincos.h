@@ -5,8 +5,11 @@
 // pi/2 split into three parts, P1 and P2 of 33 significant bits (so n P1 and
 // n P2 are exact for n < 2^20) and P3 the remainder, each subtracted with a
 // fused multiply-add; then sin r and cos r on |r| <= pi/4 (a little beyond
-// after rounding n) from their Taylor series, through r^17 and r^16 (the
-// first omitted terms are below 1e-19 and 3e-18), and the quadrant n mod 4.
+// after rounding n) from minimax polynomials (this project's own fit: weighted
+// least squares in 80-bit arithmetic, reweighted to a level error; truncation
+// errors relative to the result 1.86e-20 and 5.7e-20, where the Taylor sums through r^17
+// and r^16 used before leave 1e-19 and 3e-18 with two more terms), and the
+// quadrant n mod 4.
 // Every rounding is written out, so host and device builds give the same bits.
 #pragma once
 
@@ -22,33 +25,38 @@ namespace wm {
 
 constexpr double kSinCosMax = 1.6e6;  // below 2^20 pi/2: n P1 and n P2 stay exact
 
-WM_HD inline void sincos_phase(double x, double &s, double &c)
+// The constants, as values that a kernel can keep in registers of its choice.
+struct SinCosConsts {
+    double two_over_pi = 0.6366197723675814;
+    double p1 = 1.5707963267341256, p2 = 6.077100506303966e-11, p3 = 2.0222662487959506e-21;
+    // sin r = r + r^3 (s[6] + r^2 (s[5] + ...)),  cos r = 1 + r^2 (-1/2 + r^2 (c[5] + r^2 (c[4] + ...)))
+    double s[7] = {-7.5786380750307477e-13,
+                   1.6058359290223325e-10,
+                   -2.5052104800183583e-08,
+                   2.7557319213547918e-06,
+                   -0.00019841269841253486,
+                   0.0083333333333333211,
+                   -0.16666666666666666};
+    double c[6] = {-1.1358412519525422e-11,
+                   2.0875698350458964e-09,
+                   -2.7557314160173976e-07,
+                   2.4801587288782315e-05,
+                   -0.0013888888888872939,
+                   0.041666666666666595};
+};
+
+WM_HD inline void sincos_phase(double x, double &s, double &c, const SinCosConsts &k = SinCosConsts())
 {
-    constexpr double kTwoOverPi = 0.6366197723675814;
-    constexpr double kP1 = 1.5707963267341256, kP2 = 6.077100506303966e-11, kP3 = 2.0222662487959506e-21;
-    const double n = rint(x * kTwoOverPi);
-    double r = fma(-n, kP1, x);
-    r = fma(-n, kP2, r);
-    r = fma(-n, kP3, r);
+    const double n = rint(x * k.two_over_pi);
+    double r = fma(-n, k.p1, x);
+    r = fma(-n, k.p2, r);
+    r = fma(-n, k.p3, r);
     const double r2 = r * r;
-    // sin r = r + r^3 (-1/3! + r^2 (1/5! - ...)),  cos r = 1 + r^2 (-1/2! + r^2 (1/4! - ...))
-    double ps = 2.8114572543455206e-15;                 // 1/17!
-    ps = fma(ps, r2, -7.647163731819816e-13);           // -1/15!
-    ps = fma(ps, r2, 1.6059043836821613e-10);           // 1/13!
-    ps = fma(ps, r2, -2.505210838544172e-08);           // -1/11!
-    ps = fma(ps, r2, 2.7557319223985893e-06);           // 1/9!
-    ps = fma(ps, r2, -0.0001984126984126984);           // -1/7!
-    ps = fma(ps, r2, 0.008333333333333333);             // 1/5!
-    ps = fma(ps, r2, -0.16666666666666666);             // -1/3!
+    double ps = k.s[0], pc = k.c[0];
+    for (int i = 1; i < 7; ++i) ps = fma(ps, r2, k.s[i]);
+    for (int i = 1; i < 6; ++i) pc = fma(pc, r2, k.c[i]);
+    pc = fma(pc, r2, -0.5);
     const double sr = fma(r * r2, ps, r);
-    double pc = 4.779477332387385e-14;                  // 1/16!
-    pc = fma(pc, r2, -1.1470745597729725e-11);          // -1/14!
-    pc = fma(pc, r2, 2.08767569878681e-09);             // 1/12!
-    pc = fma(pc, r2, -2.755731922398589e-07);           // -1/10!
-    pc = fma(pc, r2, 2.48015873015873e-05);             // 1/8!
-    pc = fma(pc, r2, -0.001388888888888889);            // -1/6!
-    pc = fma(pc, r2, 0.041666666666666664);             // 1/4!
-    pc = fma(pc, r2, -0.5);                             // -1/2!
     const double cr = fma(r2, pc, 1.0);
     // quadrant q: (sin, cos) = (s, c), (c, -s), (-s, -c), (-c, s) for q = 0..3
     const int q = (int)n & 3;

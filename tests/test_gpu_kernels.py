@@ -44,3 +44,36 @@ def test_panel_non_finite_entries(wm, ctx, n):
     assert list(info) == [n, 1]
     P = piv.download()
     assert np.all(P >= np.arange(1, n + 1)) and np.all(P <= n)
+
+
+@pytest.mark.parametrize("ienv", [1, 2])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 700])
+def test_fill_row_runs(wm, geometries, oracle, ctx, geo_dir, n, ienv):
+    """Fills whose rows end inside, at and just beyond a run of 64 observation points and
+    the padded size, for chains of segments (a dipole or monopole) and, at 700, a mesh
+    with junctions: every entry against the oracle, the padding the identity."""
+    import os
+    p = os.path.join(geo_dir, f"runs_{n}_{ienv}.geo")
+    if n >= 700:
+        # with the ground each of the four rods gains a basis at its foot
+        geometries.lightning(p, n - 4 if ienv == 2 else n, depth=0.0 if ienv == 2 else 0.5, ring=ienv == 1)
+    elif ienv == 2:
+        geometries.monopole(p, n)
+    else:
+        geometries.dipole(p, n + 1, 1.0, 0.2 / (n + 1))
+    g = wm.Geometry.load(ctx, p, ienv=ienv)
+    assert g.npls == n
+    f = [5.0, 150.0]
+    Z = g.fill(f)
+    t = oracle.load(p, ienv=ienv)
+    for i in range(2):
+        ref = oracle.zmatrix(t, wm.wavenumber(f[i]), ienv=ienv)
+        assert np.abs(Z[i] - ref).max() <= 1e-12 * np.abs(ref).max()
+    import ctypes as C
+    ka = np.array([wm.wavenumber(x) for x in f])
+    D = wm.DeviceArray(ctx, np.full((2, g.ld, g.ld), np.nan, np.complex128))
+    assert wm.lib().wm_zfill(ctx.h, g.h, 2, ka.ctypes.data_as(C.POINTER(C.c_double)), D.ptr, g.ld ** 2, None, 0) == 0
+    full = D.download().transpose(0, 2, 1)
+    assert np.array_equal(full[:, :n, :n], Z)
+    eye = np.eye(g.ld)
+    assert np.array_equal(full[:, n:], np.stack([eye[n:]] * 2)) and np.array_equal(full[:, :, n:], np.stack([eye[:, n:]] * 2))

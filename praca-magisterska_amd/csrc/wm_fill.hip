@@ -39,7 +39,7 @@
 // the reference takes a square root and divides ("wersja referencyjna/
 // Zmatrix.cpp":679-688); the results differ from its by about an ulp.
 // cos kR and sin kR come from sincos_phase (wm_sincos.h: Cody-Waite reduction
-// and Taylor polynomials, within about 1.5 ulp of the exact values for kR up
+// and minimax polynomials, within about 1.5 ulp of the exact values for kR up
 // to 100 and 2.5 ulp up to its limit), which needs a fraction of the
 // operations and registers of a general-purpose sincos.
 //

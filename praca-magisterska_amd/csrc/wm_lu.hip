@@ -679,15 +679,27 @@ struct SwapArgs {
     const int *nmem;  // per matrix index: its own size (identity beyond), or null
 };
 
+// A wave owns CB / 4 columns, lane = row slot: slots t < NB are rows k + t (one
+// contiguous run per column: coalesced), the others the rows from below the
+// panel that take part; a column's loads all come before its stores in the same
+// wave, so no barrier separates them.  Interchange-only tiles move the slots
+// that change; solved tiles keep the new top rows in registers and solve there:
+// step j broadcasts x_j by lane reads and takes column j of L11 from LDS (packed
+// by columns: consecutive lanes, consecutive entries), without barriers, and
+// the rows are stored once.  The arithmetic and its order are a forward
+// substitution's.  What a small launch costs is this chain of 63 steps and the
+// memory latencies before and after it, a large one moving the rows.  Against
+// tiles solved with a barrier per step, per launch: 28 -> 14 us (N = 512), 64 ->
+// 35 us (12 x 4096), 37 -> 20 us (2 x 8192), 135 -> 65 us (16 x 8192), pivots near
+// the diagonal; 346 -> 302 us (16 x 8192, random pivots).
 template <typename T, int CB>
 __global__ __launch_bounds__(256) void k_swap_trsm(typename CT<T>::V *A, int lda, int64_t strideA, SwapArgs a,
                                                    char *xbuf, const int *bidx)
 {
     using V = typename CT<T>::V;
-    constexpr int RG = 256 / CB;        // row groups for the triangular solve
-    constexpr int RPT = NB / RG;        // rows per thread in the solve
-    constexpr int EPT = 2 * NB * CB / 256;  // permuted elements per thread (max)
-    const int bl = blockIdx.y, tile = blockIdx.x, tid = threadIdx.x;
+    constexpr int CW = CB / 4;  // columns per wave
+    const int bl = blockIdx.y, tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = bidx ? bidx[bl] : bl;
     const int n = a.n, k = a.k;
     V *Ab = A + (size_t)b * strideA;
@@ -702,86 +714,60 @@ __global__ __launch_bounds__(256) void k_swap_trsm(typename CT<T>::V *A, int lda
     // identity) and zero blocks right of it (their solve changes nothing)
     if (a.nmem && (k >= a.nmem[b] || c0 >= a.nmem[b])) return;
 
-    // gather the old contents of the touched rows, keep the new top block
-    // (rows k..k+NB-1) of solved columns in LDS, then scatter.  Consecutive
-    // lanes take consecutive row slots of one column: the NB rows k..k+NB-1,
-    // source or target of most moves, are then one contiguous run per column
-    // (coalesced in column-major storage); s_top is kept column by column,
-    // padded so the solve's reads across columns spread over the LDS banks.
-    __shared__ V s_top[CB][NB + 1];
+    int src0 = k + lane, src1 = 0, dst1 = 0;
+    bool ex = false;
     if (a.do_swap) {
-        __shared__ int s_rows[2 * NB], s_src[2 * NB];
-        __shared__ int s_cnt;
         const int *pm = X.perm(xm);
-        if (tid == 0) s_cnt = pm[0];
-        if (tid < 2 * NB) { s_rows[tid] = pm[1 + tid]; s_src[tid] = pm[1 + 2 * NB + tid]; }
-        __syncthreads();
-        const int tcnt = s_cnt;
-        V val[EPT];
+        const int *rows = pm + 1, *src = pm + 1 + 2 * NB;
+        ex = NB + lane < pm[0];
+        src0 = src[lane];
+        if (ex) {
+            src1 = src[NB + lane];
+            dst1 = rows[NB + lane];
+        }
+    }
+    const bool move0 = trsm || src0 != k + lane;
+    V top[CW], ext[CW];
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) {
-            const int idx = tid + 256 * e;
-            const int t = idx % (2 * NB), cc = idx / (2 * NB), col = c0 + cc;
-            val[e] = V{0, 0};
-            if (t < tcnt && col < cend) {
-                val[e] = Ab[s_src[t] + (size_t)col * lda];
-                if (trsm && t < NB) s_top[cc][t] = val[e];
-            }
-        }
-        __syncthreads();
+    for (int q = 0; q < CW; ++q) {
+        const int col = c0 + wave * CW + q;
+        const V *Ac = Ab + (size_t)col * lda;
+        top[q] = ext[q] = V{0, 0};
+        if (col < cend && move0) top[q] = Ac[src0];
+        if (col < cend && ex) ext[q] = Ac[src1];
+    }
+    __shared__ V s_l[NB * (NB - 1) / 2];  // strictly lower part of L11, column by column
+    auto lidx = [](int i, int j) { return j * (2 * NB - 1 - j) / 2 + (i - j - 1); };
+    if (trsm) {
+        for (int j = wave; j < NB - 1; j += 4)
+            if (lane > j) s_l[lidx(lane, j)] = Ab[(k + lane) + (size_t)(k + j) * lda];
+    }
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) {
-            const int idx = tid + 256 * e;
-            const int t = idx % (2 * NB), col = c0 + idx / (2 * NB);
-            if (t < tcnt && col < cend) Ab[s_rows[t] + (size_t)col * lda] = val[e];
-        }
-    } else if (trsm) {
-        for (int idx = tid; idx < NB * CB; idx += 256) {
-            const int t = idx % NB, cc = idx / NB, col = c0 + cc;
-            if (col < cend) s_top[cc][t] = Ab[(k + t) + (size_t)col * lda];
-        }
+    for (int q = 0; q < CW; ++q) {
+        const int col = c0 + wave * CW + q;
+        V *Ac = Ab + (size_t)col * lda;
+        if (col < cend && ex) Ac[dst1] = ext[q];
+        if (col < cend && !trsm && move0) Ac[k + lane] = top[q];
     }
     if (!trsm) return;
-
-    // forward substitution with the unit lower L11 (strictly lower part in LDS)
-    __shared__ V s_l[NB * (NB - 1) / 2];
-    __shared__ V s_x[2][CB];
-    for (int e = tid; e < NB * NB; e += 256) {
-        const int i = e % NB, jj = e / NB;
-        if (i > jj) s_l[i * (i - 1) / 2 + jj] = Ab[(k + i) + (size_t)(k + jj) * lda];
-    }
     __syncthreads();
-    const int c = tid % CB, rg = tid / CB;
-    const bool cok = (c0 + c) < cend;
-    T xr[RPT], xi[RPT];
+#pragma unroll 8
+    for (int j = 0; j < NB - 1; ++j) {
+        V xj[CW];
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        const V v = cok ? s_top[c][rg + q * RG] : V{0, 0};
-        xr[q] = v.x;
-        xi[q] = v.y;
-    }
-    for (int jj = 0; jj < NB; ++jj) {
-        const int par = jj & 1;
-        if (rg == jj % RG) {
+        for (int q = 0; q < CW; ++q) xj[q] = V{readlane_t(top[q].x, j), readlane_t(top[q].y, j)};
+        if (lane > j) {
+            const V l = s_l[lidx(lane, j)];
 #pragma unroll
-            for (int q = 0; q < RPT; ++q)
-                if (q == jj / RG) s_x[par][c] = V{xr[q], xi[q]};
-        }
-        __syncthreads();
-        const V xj = s_x[par][c];
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int i = rg + q * RG;
-            if (i > jj) {
-                const V l = s_l[i * (i - 1) / 2 + jj];
-                xr[q] -= l.x * xj.x - l.y * xj.y;
-                xi[q] -= l.x * xj.y + l.y * xj.x;
-            }
+            for (int q = 0; q < CW; ++q)
+                top[q] = V{sub_mul_re(top[q].x, xj[q].x, xj[q].y, l.x, l.y),
+                           sub_mul_im(top[q].y, xj[q].x, xj[q].y, l.x, l.y)};
         }
     }
-    if (cok) {
 #pragma unroll
-        for (int q = 0; q < RPT; ++q) Ab[(k + rg + q * RG) + (size_t)(c0 + c) * lda] = V{xr[q], xi[q]};
+    for (int q = 0; q < CW; ++q) {
+        const int col = c0 + wave * CW + q;
+        if (col < cend) Ab[(k + lane) + (size_t)col * lda] = top[q];
     }
 }
 
@@ -1231,6 +1217,32 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b3(float2 *Abase, int lda, int6
             }
 }
 
+// Launches the interchanges and solves of one panel for m matrices; sa without
+// its tile counts.  Tiles of 8 columns (two per wave) shorten the chain of a
+// launch that leaves the device idle, tiles of 16 read L11 half as often: 14.4
+// against 17.5 us per launch at N = 512, 20.3 against 22.7 at 2 x 8192 (512 wide
+// tiles and fewer per matrix), 75 against 65 at 16 x 8192.
+template <typename T>
+void launch_swap(const wm_ctx *ctx, SwapArgs sa, typename CT<T>::V *A, int lda, int64_t strideA, char *xbuf,
+                 const int *bidx, int m, hipStream_t s)
+{
+    const int left = sa.do_swap ? sa.k : 0, solve = std::max(0, sa.c_tr1 - sa.c_tr0),
+              right = sa.do_swap ? std::max(0, sa.n - sa.c_sw0) : 0;
+    auto tiles = [&](int cb) {
+        sa.ntl = (left + cb - 1) / cb;
+        sa.ntr = (solve + cb - 1) / cb;
+        return sa.ntl + sa.ntr + (right + cb - 1) / cb;
+    };
+    const int wide = tiles(16);
+    if (wide == 0) return;
+    if ((int64_t)wide * m <= 4 * ctx->num_cu) {
+        const int t = tiles(8);
+        hipLaunchKernelGGL((k_swap_trsm<T, 8>), dim3(t, m), dim3(256), 0, s, A, lda, strideA, sa, xbuf, bidx);
+    } else {
+        hipLaunchKernelGGL((k_swap_trsm<T, 16>), dim3(wide, m), dim3(256), 0, s, A, lda, strideA, sa, xbuf, bidx);
+    }
+}
+
 // Launches C -= L U for nb_ matrices, C = A[r0.., c0..] (mrows x ncols),
 // L = A[r0.., kk..kk+K), U = A[kk..kk+K, c0..).  gk: 8 complex128, 4 complex64,
 // 2 complex64 with split-BF16x3 products.
@@ -1364,7 +1376,6 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
 {
     using V = typename CT<T>::V;
     constexpr int RW = 256 / TPR;
-    constexpr int CB = (sizeof(T) == 8) ? 16 : 32;
     const XLayout<V> X(pl.slots);
     char *xbase = (char *)ctx->ws_lu.ptr;
     const double esz = 2.0 * sizeof(T);
@@ -1414,15 +1425,11 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
         SwapArgs sa;
         sa.n = n; sa.k = c; sa.slots = pl.slots; sa.do_swap = do_swap;
         sa.nmem = d_nmem;
-        sa.ntl = do_swap ? (c + CB - 1) / CB : 0;
         sa.c_tr0 = tr0; sa.c_tr1 = tr1;
-        sa.ntr = tr1 > tr0 ? (tr1 - tr0 + CB - 1) / CB : 0;
         sa.c_sw0 = tr1;
-        const int nsw = do_swap && n > tr1 ? (n - tr1 + CB - 1) / CB : 0;
-        if (sa.ntl + sa.ntr + nsw == 0) return;
+        if (!do_swap && tr1 <= tr0) return;
         prof_begin(ctx, kSwapClass, G.st);
-        hipLaunchKernelGGL((k_swap_trsm<T, CB>), dim3(sa.ntl + sa.ntr + nsw, G.m), dim3(256), 0, G.st, G.Ab, lda,
-                           strideA, sa, G.xbuf, G.bidx);
+        launch_swap<T>(ctx, sa, G.Ab, lda, strideA, G.xbuf, G.bidx, G.m, G.st);
         prof_end(ctx, kSwapClass, G.st, G.m * 4.0 * NB * NB * (tr1 - tr0), G.m * 4.0 * NB * n * esz);
     };
     auto gemm = [&](const Grp &G, int r0, int c0, int mrows, int ncols, int kk, int K) {
@@ -1690,7 +1697,6 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         pa.ipiv = ipiv; pa.strideP = 0; pa.info = info;
         pa.err = ctx->d_err; pa.xbuf = xbuf; pa.bidx = nullptr; pa.tagp = ctx->d_tag; pa.toff = (uint32_t)k;
         pa.nmem = nullptr;
-        constexpr int CB = (sizeof(T) == 8) ? 16 : 32;
         if (sizeof(T) == 8)
             hipLaunchKernelGGL((k_panel<double, kTprF64>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<double> *)&pa);
         else
@@ -1698,12 +1704,8 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         if (do_swap) {
             SwapArgs sa;
             sa.n = n; sa.k = k; sa.slots = slots; sa.do_swap = 1; sa.nmem = nullptr;
-            sa.ntl = (k + CB - 1) / CB;
-            sa.ntr = (n - k - NB + CB - 1) / CB;
             sa.c_tr0 = k + NB; sa.c_tr1 = n; sa.c_sw0 = n;
-            if (sa.ntl + sa.ntr > 0)
-                hipLaunchKernelGGL((k_swap_trsm<T, CB>), dim3(sa.ntl + sa.ntr, 1), dim3(256), 0, ctx->stream, (V *)Ap,
-                                   n, (int64_t)0, sa, xbuf, (const int *)nullptr);
+            launch_swap<T>(ctx, sa, (V *)Ap, n, 0, xbuf, nullptr, 1, ctx->stream);
         }
         return WM_OK;
     };

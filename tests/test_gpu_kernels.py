@@ -77,3 +77,19 @@ def test_fill_row_runs(wm, geometries, oracle, ctx, geo_dir, n, ienv):
     assert np.array_equal(full[:, :n, :n], Z)
     eye = np.eye(g.ld)
     assert np.array_equal(full[:, n:], np.stack([eye[n:]] * 2)) and np.array_equal(full[:, :, n:], np.stack([eye[:, n:]] * 2))
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n,batch", [(320, 70), (64, 5)])
+def test_wide_batch_equals_single(wm, ctx, prec, n, batch):
+    """A batch wide enough for the launches' larger tiles gives each member's factors and
+    pivots bit for bit as factored alone (smaller tiles)."""
+    rng = np.random.RandomState(n + batch)
+    A = rng.randn(batch, n, n) + 1j * rng.randn(batch, n, n)
+    dev, piv, info = wm.getrf_batched(ctx, A, prec)
+    LU, P = dev.download(), piv.download()
+    assert not info.any()
+    for b in (0, batch // 2, batch - 1):
+        d1, p1, _ = wm.getrf_batched(ctx, A[b], prec)
+        assert np.array_equal(p1.download()[0], P[b])
+        assert np.array_equal(d1.download()[0], LU[b])

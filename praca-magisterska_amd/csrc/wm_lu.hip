@@ -946,6 +946,92 @@ __global__ __launch_bounds__(256, 3) void k_gemm_f64(double2 *Abase, int lda, in
             }
 }
 
+// The complex128 update of launches with too few 64 x 64 tiles to fill the device
+// (small matrices, the narrow updates inside an outer block): the same products
+// in the same order (the same bits) on tiles of 32 x 32, one 16 x 16 tile per wave,
+// so four times as many workgroups share the work.  Such a launch is a chain of
+// latencies: both operands' first two chunks of 32 (all of K = 64) and the C tile
+// are loaded at once at the start, and a chunk needs one barrier.
+constexpr int GS_B = 32, GS_KC = 32;
+
+__global__ __launch_bounds__(256, 2) void k_gemm_f64_small(double2 *Abase, int lda, int64_t strideA, GemmArgs g,
+                                                           const int *bidx, int TI, int TJ)
+{
+    const int t = xcd_tile(blockIdx.x, TI * TJ);
+    if (t >= TI * TJ) return;
+    const int b = bidx ? bidx[blockIdx.z] : (int)blockIdx.z;
+    double2 *M = Abase + (size_t)b * strideA;
+    const int mrows = g.mrows, ncols = g.ncols, K = g.K;
+    int ti, tj;
+    tile_coords(t, TI, TJ, ti, tj);
+    const int i0 = ti * GS_B, j0 = tj * GS_B;
+    if (g.nmem && (g.r0 + i0 >= g.nmem[b] || g.c0 + j0 >= g.nmem[b])) return;
+    const double2 *A = M + g.r0 + (size_t)g.kk * lda;  // L block
+    const double2 *B = M + g.kk + (size_t)g.c0 * lda;  // U block
+    double2 *C = M + g.r0 + (size_t)g.c0 * lda;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wi = (wave & 1) * 16, wj = (wave >> 1) * 16;
+
+    // two buffers: a chunk is staged while the other is still read
+    __shared__ double2 sA[2][GS_KC][GS_B + 1];
+    __shared__ double2 sB[2][GS_KC][GS_B + 1];
+    double2 pa[2][4], pb[2][4];
+    // chunk elements moved by this thread: L row ai, k = ak + 8e; U k = bk, columns bj + 8e
+    const int ai = tid % GS_B, ak = tid / GS_B, bk = tid % GS_KC, bj = tid / GS_KC;
+    const bool arow = i0 + ai < mrows;
+    auto fetch = [&](int kc, double2 *a, double2 *u) {
+        const double2 *pA = A + (i0 + ai) + (size_t)(kc + ak) * lda;
+        const double2 *pB = B + (kc + bk) + (size_t)(j0 + bj) * lda;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = arow ? pA[(size_t)(8 * e) * lda] : double2{0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[e] = (j0 + bj + 8 * e < ncols) ? pB[(size_t)(8 * e) * lda] : double2{0.0, 0.0};
+    };
+    auto stash = [&](int buf, const double2 *a, const double2 *u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sA[buf][ak + 8 * e][ai] = a[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sB[buf][bk][bj + 8 * e] = u[e];
+    };
+    fetch(0, pa[0], pb[0]);
+    if (GS_KC < K) fetch(GS_KC, pa[1], pb[1]);
+    const int gi = i0 + wi + lane % 16, gj = j0 + wj + lane / 16;
+    double2 c[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        c[v] = gi < mrows && gj + 4 * v < ncols ? C[gi + (size_t)(gj + 4 * v) * lda] : double2{0.0, 0.0};
+
+    v4d P = v4d{0, 0, 0, 0}, Q = P, S = P;
+    auto compute = [&](int buf) {
+#pragma unroll
+        for (int ks = 0; ks < GS_KC; ks += 4) {
+            const int kk = ks + lane / 16;
+            const double2 bv = sB[buf][kk][wj + lane % 16], av = sA[buf][kk][wi + lane % 16];
+            P = __builtin_amdgcn_mfma_f64_16x16x4f64(bv.x, av.x, P, 0, 0, 0);
+            Q = __builtin_amdgcn_mfma_f64_16x16x4f64(bv.y, av.y, Q, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f64_16x16x4f64(bv.x + bv.y, av.x + av.y, S, 0, 0, 0);
+        }
+    };
+    // K is a multiple of two chunks; a buffer is written again only after the
+    // barrier that follows its last reads
+    for (int kc = 0; kc < K; kc += 2 * GS_KC) {
+        stash(0, pa[0], pb[0]);
+        if (kc + 2 * GS_KC < K) fetch(kc + 2 * GS_KC, pa[0], pb[0]);
+        __syncthreads();
+        compute(0);
+        stash(1, pa[1], pb[1]);
+        if (kc + 3 * GS_KC < K) fetch(kc + 3 * GS_KC, pa[1], pb[1]);
+        __syncthreads();
+        compute(1);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (gi < mrows && gj + 4 * v < ncols) {
+            const double p = P[v], q = Q[v];
+            C[gi + (size_t)(gj + 4 * v) * lda] = double2{c[v].x - (p - q), c[v].y - (S[v] - p - q)};
+        }
+}
+
 // complex64 with three real products per complex product, as k_gemm_f64:
 // P = sum Br Ar, Q = sum Bi Ai, S = sum (Br + Bi)(Ar + Ai).  Workgroup tile
 // 128 x 64, four waves of 64 x 32 (2 x 1 tiles of v_mfma_f32_32x32x2f32).
@@ -1243,6 +1329,11 @@ void launch_swap(const wm_ctx *ctx, SwapArgs sa, typename CT<T>::V *A, int lda, 
     }
 }
 
+// Most 64 x 64 tiles of a complex128 update that runs on tiles of 32 x 32: 14 -> 6 us
+// with 49 tiles, 24.5 -> 22.0 with 361, 31.0 -> 30.9 with 529 (K = 64); 36 -> 12 us with
+// 16, 41.7 -> 37.4 with 256, 62.5 -> 61.5 with 400 (K = 256).
+constexpr int64_t kSmallTiles = 512;
+
 // Launches C -= L U for nb_ matrices, C = A[r0.., c0..] (mrows x ncols),
 // L = A[r0.., kk..kk+K), U = A[kk..kk+K, c0..).  gk: 8 complex128, 4 complex64,
 // 2 complex64 with split-BF16x3 products.
@@ -1251,7 +1342,14 @@ void launch_gemm(int gk, void *A, int lda, int64_t strideA, const GemmArgs &g, i
 {
     if (g.mrows <= 0 || g.ncols <= 0 || g.K <= 0) return;
     if (gk == 8) {
-        const int TI = (g.mrows + GZ_BM - 1) / GZ_BM, TJ = (g.ncols + GZ_BN - 1) / GZ_BN;
+        int TI = (g.mrows + GZ_BM - 1) / GZ_BM, TJ = (g.ncols + GZ_BN - 1) / GZ_BN;
+        if ((int64_t)TI * TJ * nb_ <= kSmallTiles) {
+            TI = (g.mrows + GS_B - 1) / GS_B;
+            TJ = (g.ncols + GS_B - 1) / GS_B;
+            hipLaunchKernelGGL(k_gemm_f64_small, dim3(xcd_grid(TI * TJ), 1, nb_), dim3(256), 0, s, (double2 *)A, lda,
+                               strideA, g, bidx, TI, TJ);
+            return;
+        }
         hipLaunchKernelGGL(k_gemm_f64, dim3(xcd_grid(TI * TJ), 1, nb_), dim3(256), 0, s, (double2 *)A, lda, strideA,
                            g, bidx, TI, TJ);
     } else if (gk == 4) {

@@ -303,6 +303,7 @@ int wm_shutdown(wm_ctx *c)
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     if (c->aux) (void)hipStreamSynchronize(c->aux);
+    if (c->lu_side) (void)hipStreamSynchronize(c->lu_side);
     drop_graphs(c);
     c->ws_info.release();
     c->ws_fill.release();
@@ -322,6 +323,9 @@ int wm_shutdown(wm_ctx *c)
     for (auto e : c->aux_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->aux) (void)hipStreamDestroy(c->aux);
+    for (auto e : c->lu_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->lu_side) (void)hipStreamDestroy(c->lu_side);
     (void)hipStreamDestroy(c->stream);
     if (c == g_default_ctx) g_default_ctx = nullptr;
     delete c;

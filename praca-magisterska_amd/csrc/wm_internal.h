@@ -122,6 +122,10 @@ struct wm_ctx {
     hipStream_t aux = nullptr;
     hipEvent_t aux_ev[2] = {nullptr, nullptr};  // launch stream -> aux, aux -> launch stream
     wm::DevBuf ws_fill2;
+    // look-ahead of factorizations: the rest of a block's update runs on this
+    // stream while the next block's panels are factored; created on first use
+    hipStream_t lu_side = nullptr;
+    hipEvent_t lu_ev[2] = {nullptr, nullptr};  // launch stream -> lu_side, lu_side -> launch stream
 };
 
 // Geometry as the fill kernel reads it.  Observation data per basis (SoA,

@@ -72,7 +72,9 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 //   cand [slots][NWS]: each candidate's row (NW 32-bit words, per chunk the low
 //                     or real halves of its 32 values, then the high or
 //                     imaginary ones) and the reciprocal of its pivot (4 words)
-// followed by the panel permutation: cnt, rows[2NB], src[2NB].
+// followed by kPermSlots panel permutations (one per panel of an outer block):
+// cnt, rows[2NB], src[2NB].
+constexpr int kPermSlots = 16;  // panels per outer block at most
 template <typename V>
 struct XLayout {
     static constexpr int NW = NB * (int)sizeof(V) / 4;  // 32-bit words per panel row
@@ -85,12 +87,12 @@ struct XLayout {
         par_bytes = (size_t)slots * (SLS + NWS) * sizeof(uint64_t);
         par_bytes = (par_bytes + 255) & ~(size_t)255;
         perm_off = 2 * par_bytes;
-        mat_bytes = perm_off + (1 + 4 * NB) * sizeof(int);
+        mat_bytes = perm_off + kPermSlots * (1 + 4 * NB) * sizeof(int);
         mat_bytes = (mat_bytes + 255) & ~(size_t)255;
     }
     __device__ uint64_t *slot(char *m, int par) const { return (uint64_t *)(m + par * par_bytes); }
     __device__ uint64_t *cand(char *m, int par) const { return slot(m, par) + (size_t)slots * SLS; }
-    __device__ int *perm(char *m) const { return (int *)(m + perm_off); }
+    __device__ int *perm(char *m, int slot) const { return (int *)(m + perm_off) + slot * (1 + 4 * NB); }
 };
 
 // Columns of the panel updated together, and workgroups per CU that the
@@ -104,6 +106,7 @@ struct PanelArgs {
     int lda;
     int64_t strideA;
     int n, k, P, slots;
+    int pslot;  // where the panel's permutation goes
     int *ipiv;
     int64_t strideP;
     int *info;
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         // the member's own matrix ends above this panel: an identity panel, no
         // interchanges (pivots k+1 .. k+NB) and an empty permutation
         if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = k + tid + 1;
-        if (w == 0 && tid == 0) X.perm(xm)[0] = 0;
+        if (w == 0 && tid == 0) X.perm(xm, a.pslot)[0] = 0;
         return;
     }
 
@@ -654,7 +657,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
                 shi = sj;
             }
         }
-        int *pm = X.perm(xm);
+        int *pm = X.perm(xm, a.pslot);
         int *rows = pm + 1, *src = pm + 1 + 2 * NB;
         rows[lane] = rlo;
         src[lane] = slo;
@@ -669,13 +672,13 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
 // ---------------------------------------------------------------------------
 // Row interchanges outside the panel and U12 = L11^{-1} A12.  Tiles of CB
 // columns, three kinds by tile index:
-//   [0, ntl)           columns [tile*CB, k): interchanges only (L to the left)
+//   [0, ntl)           columns [c_l0, c_l1): interchanges only (to the left)
 //   [ntl, ntl+ntr)     columns [c_tr0, c_tr1): interchanges (if do_swap) and
 //                      the triangular solve of rows k..k+NB-1
 //   [ntl+ntr, ...)     columns [c_sw0, n): interchanges only (columns whose
 //                      rows k..k+NB-1 still await earlier panels' updates)
 struct SwapArgs {
-    int n, k, slots, ntl, ntr, c_tr0, c_tr1, c_sw0, do_swap;
+    int n, k, slots, pslot, c_l0, c_l1, ntl, ntr, c_tr0, c_tr1, c_sw0, do_swap;
     const int *nmem;  // per matrix index: its own size (identity beyond), or null
 };
 
@@ -707,9 +710,9 @@ __global__ __launch_bounds__(256) void k_swap_trsm(typename CT<T>::V *A, int lda
     char *xm = xbuf + (size_t)bl * X.mat_bytes;
 
     const bool trsm = tile >= a.ntl && tile < a.ntl + a.ntr;
-    const int c0 = tile < a.ntl ? tile * CB : trsm ? a.c_tr0 + (tile - a.ntl) * CB
+    const int c0 = tile < a.ntl ? a.c_l0 + tile * CB : trsm ? a.c_tr0 + (tile - a.ntl) * CB
                                                    : a.c_sw0 + (tile - a.ntl - a.ntr) * CB;
-    const int cend = tile < a.ntl ? k : trsm ? a.c_tr1 : n;
+    const int cend = tile < a.ntl ? a.c_l1 : trsm ? a.c_tr1 : n;
     // beyond the member's own size: no interchanges (its panel was the
     // identity) and zero blocks right of it (their solve changes nothing)
     if (a.nmem && (k >= a.nmem[b] || c0 >= a.nmem[b])) return;
@@ -717,7 +720,7 @@ __global__ __launch_bounds__(256) void k_swap_trsm(typename CT<T>::V *A, int lda
     int src0 = k + lane, src1 = 0, dst1 = 0;
     bool ex = false;
     if (a.do_swap) {
-        const int *pm = X.perm(xm);
+        const int *pm = X.perm(xm, a.pslot);
         const int *rows = pm + 1, *src = pm + 1 + 2 * NB;
         ex = NB + lane < pm[0];
         src0 = src[lane];
@@ -1312,7 +1315,7 @@ template <typename T>
 void launch_swap(const wm_ctx *ctx, SwapArgs sa, typename CT<T>::V *A, int lda, int64_t strideA, char *xbuf,
                  const int *bidx, int m, hipStream_t s)
 {
-    const int left = sa.do_swap ? sa.k : 0, solve = std::max(0, sa.c_tr1 - sa.c_tr0),
+    const int left = sa.do_swap ? std::max(0, sa.c_l1 - sa.c_l0) : 0, solve = std::max(0, sa.c_tr1 - sa.c_tr0),
               right = sa.do_swap ? std::max(0, sa.n - sa.c_sw0) : 0;
     auto tiles = [&](int cb) {
         sa.ntl = (left + cb - 1) / cb;
@@ -1470,7 +1473,7 @@ int getrf_plan(wm_ctx *ctx, int n, int batch, GetrfPlan *pl)
 template <typename T, int TPR>
 int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, int lda, int64_t strideA, int *ipiv,
                int64_t strideP, int batch, int *d_info, const int *d_bidx, hipStream_t s, int gk, int kSub,
-               const int *d_nmem)
+               const int *d_nmem, hipStream_t side)
 {
     using V = typename CT<T>::V;
     constexpr int RW = 256 / TPR;
@@ -1493,7 +1496,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
     // panel at column c for every member, in launches of as many members as
     // keep their clusters co-resident; members b0.. of a launch use exchange
     // buffers b0.. (the interchange kernel reads member b's permutation there)
-    auto panel = [&](const Grp &G, int c) {
+    auto panel = [&](const Grp &G, int c, int pslot) {
         const int P = (n - c + RW - 1) / RW;
         const int per = std::max(1, std::min(G.m, pl.resident / P));
         const double mr = n - c;
@@ -1502,7 +1505,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
             PanelArgs<T> pa;
             pa.A = G.bidx ? G.Ab : G.Ab + (size_t)b0 * strideA;
             pa.lda = lda; pa.strideA = strideA; pa.n = n; pa.k = c;
-            pa.P = P; pa.slots = pl.slots;
+            pa.P = P; pa.slots = pl.slots; pa.pslot = pslot;
             pa.ipiv = G.bidx ? G.ipb : G.ipb + (size_t)b0 * strideP;
             pa.strideP = strideP;
             pa.info = G.bidx ? G.infob : G.infob + b0;
@@ -1518,17 +1521,18 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
                      m * 2.0 * mr * NB * esz);
         }
     };
-    // interchanges of the panel at c left of c; solve for [tr0, tr1); interchanges only for [tr1, n)
-    auto swap = [&](const Grp &G, int c, int tr1, int do_swap, int tr0) {
+    // interchanges of the panel at c (permutation slot ps) in columns [l0, l1),
+    // solve for [tr0, tr1) with (do_swap) or without them, interchanges in [sw0, n)
+    auto swap = [&](const Grp &G, int c, int ps, int l0, int l1, int tr0, int tr1, int sw0, int do_swap) {
         SwapArgs sa;
-        sa.n = n; sa.k = c; sa.slots = pl.slots; sa.do_swap = do_swap;
+        sa.n = n; sa.k = c; sa.slots = pl.slots; sa.pslot = ps; sa.do_swap = do_swap;
         sa.nmem = d_nmem;
+        sa.c_l0 = l0; sa.c_l1 = l1;
         sa.c_tr0 = tr0; sa.c_tr1 = tr1;
-        sa.c_sw0 = tr1;
-        if (!do_swap && tr1 <= tr0) return;
+        sa.c_sw0 = sw0;
         prof_begin(ctx, kSwapClass, G.st);
         launch_swap<T>(ctx, sa, G.Ab, lda, strideA, G.xbuf, G.bidx, G.m, G.st);
-        prof_end(ctx, kSwapClass, G.st, G.m * 4.0 * NB * NB * (tr1 - tr0), G.m * 4.0 * NB * n * esz);
+        prof_end(ctx, kSwapClass, G.st, G.m * 4.0 * NB * NB * std::max(0, tr1 - tr0), G.m * 4.0 * NB * n * esz);
     };
     auto gemm = [&](const Grp &G, int r0, int c0, int mrows, int ncols, int kk, int K) {
         if (mrows <= 0 || ncols <= 0) return;
@@ -1559,22 +1563,60 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
         // their interchanges at once and their update from the whole block in
         // one product with K = kSub * NB (rows of the later panels' solves are
         // updated first by a short product).
-        for (int k = 0; k < n; k += kSub * NB) {
+        for (int k = 0; k < n && !side; k += kSub * NB) {
             const int kend = (n - k < kSub * NB) ? n : k + kSub * NB;
             for (int c = k; c < kend; c += NB) {
                 if (c > k) gemm(G, c, c, n - c, kend - c, c - NB, NB);
-                panel(G, c);
+                panel(G, c, 0);
                 if (c == k) {
-                    swap(G, c, n, 1, c + NB);
+                    swap(G, c, 0, 0, c, c + NB, n, n, 1);
                 } else {
-                    swap(G, c, kend, 1, c + NB);
+                    swap(G, c, 0, 0, c, c + NB, kend, kend, 1);
                     if (kend < n) {
                         gemm(G, c, kend, NB, n - kend, k, c - k);
-                        swap(G, c, n, 0, kend);
+                        swap(G, c, 0, 0, 0, kend, n, n, 0);
                     }
                 }
             }
             gemm(G, kend, kend, n - kend, n - kend, k, kend - k);
+        }
+        // Look-ahead: a block's update goes to the next block's columns first; the
+        // rest of it runs on the side stream while the next block's panels (which
+        // leave most of the device idle) are factored inside their own columns.
+        // Their interchanges and solves of the other columns wait for both.  Every
+        // entry takes the same operations in the same order: the same bits.
+        Grp H = G;
+        H.st = side;
+        bool pending = false;
+        for (int k = 0; k < n && side; k += kSub * NB) {
+            const int kend = std::min(n, k + kSub * NB), kend2 = std::min(n, kend + kSub * NB);
+            for (int c = k; c < kend; c += NB) {
+                if (c > k) gemm(G, c, c, n - c, kend - c, c - NB, NB);
+                panel(G, c, (c - k) / NB);
+                swap(G, c, (c - k) / NB, k, c, c + NB, kend, n, 1);
+            }
+            if (pending) WM_HIP_TRY(hipStreamWaitEvent(s, ctx->lu_ev[1], 0));
+            pending = false;
+            for (int c = k; c < kend; c += NB) {
+                const int ps = (c - k) / NB;
+                if (c == k) {
+                    swap(G, c, ps, 0, k, kend, n, n, 1);
+                } else {
+                    swap(G, c, ps, 0, k, 0, 0, kend, 1);
+                    if (kend < n) {
+                        gemm(G, c, kend, NB, n - kend, k, c - k);
+                        swap(G, c, ps, 0, 0, kend, n, n, 0);
+                    }
+                }
+            }
+            if (kend2 < n) {
+                WM_HIP_TRY(hipEventRecord(ctx->lu_ev[0], s));
+                WM_HIP_TRY(hipStreamWaitEvent(side, ctx->lu_ev[0], 0));
+                gemm(H, kend, kend2, n - kend, n - kend2, k, kend - k);
+                WM_HIP_TRY(hipEventRecord(ctx->lu_ev[1], side));
+                pending = true;
+            }
+            gemm(G, kend, kend, n - kend, kend2 - kend, k, kend - k);
         }
         WM_HIP_TRY(hipGetLastError());
     }
@@ -1608,12 +1650,34 @@ namespace {
 template <typename T, int TPR>
 int getrf_enqueue(wm_ctx *ctx, const GetrfPlan &pl, int n, void *A, int lda, int64_t strideA, int *ipiv,
                   int64_t strideP, int batch, int *d_info, const int *d_bidx, hipStream_t s, int gk, int ks,
-                  const int *d_nmem)
+                  const int *d_nmem, hipStream_t side)
 {
     if (!d_bidx) hipLaunchKernelGGL(k_zero_int, dim3((batch + 255) / 256), dim3(256), 0, s, d_info, batch);
     else hipLaunchKernelGGL(k_zero_idx, dim3((batch + 255) / 256), dim3(256), 0, s, d_info, d_bidx, batch);
     return getrf_impl<T, TPR>(ctx, pl, n, (typename CT<T>::V *)A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx,
-                              s, gk, ks, d_nmem);
+                              s, gk, ks, d_nmem, side);
+}
+
+// Look-ahead stream of a factorization, or null for one that runs on one stream.
+// The side stream pays once its updates are long enough against the launches and
+// events it adds (1 x 4096: 14.1 -> 14.4 ms, 4 x 4096: 21.9 -> 21.6, 12 x 4096: 44.4 ->
+// 43.8, 2 x 8192: 63.8 -> 61.4, 2 x 14336: 246 -> 236; split-BF16x3 12 x 8192: 117 ->
+// 110 ms) and while the panels of the batch go in one launch, which leaves CUs
+// idle; a batch of several such launches keeps the device busy by itself (16 x
+// 8192: 347 -> 360 ms).  The profiler keeps every launch on one stream.
+constexpr int64_t kSideMinEntries = (int64_t)1 << 26;
+int getrf_side(wm_ctx *ctx, const GetrfPlan &pl, int n, int batch, int ks, hipStream_t *side)
+{
+    *side = nullptr;
+    if (ctx->prof.on || batch > pl.per_launch || n <= 2 * ks * NB || (int64_t)n * n * batch < kSideMinEntries)
+        return WM_OK;
+    if (!ctx->lu_side) {  // events first, the stream last: lu_side set means all exist
+        for (auto &e : ctx->lu_ev)
+            if (!e) WM_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        WM_HIP_TRY(hipStreamCreateWithFlags(&ctx->lu_side, hipStreamNonBlocking));
+    }
+    *side = ctx->lu_side;
+    return WM_OK;
 }
 
 template <typename T, int TPR>
@@ -1625,9 +1689,11 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
     WM_TRY((getrf_plan<T, TPR>(ctx, n, batch, &pl)));
     const uint64_t ntags = (uint64_t)n;
     WM_TRY(prepare_xbuf(ctx, pl.xbytes, ntags, s));
+    hipStream_t side = nullptr;
+    WM_TRY(getrf_side(ctx, pl, n, batch, ks, &side));
     if (!ctx->use_graphs || ctx->prof.on) {
         WM_TRY((getrf_enqueue<T, TPR>(ctx, pl, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, gk, ks,
-                                      d_nmem)));
+                                      d_nmem, side)));
     } else {
         // Replay a captured factorization of the same shape and buffers, or
         // capture one.  Its kernels read their tags from the device counter, so
@@ -1640,7 +1706,7 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
         if (!exec) {
             WM_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             const int rc = getrf_enqueue<T, TPR>(ctx, pl, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s,
-                                                 gk, ks, d_nmem);
+                                                 gk, ks, d_nmem, side);
             hipGraph_t graph = nullptr;
             const hipError_t ec = hipStreamEndCapture(s, &graph);
             if (rc != WM_OK) {
@@ -1791,7 +1857,7 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         ctx->panel_tag += (uint64_t)n;
         PanelArgs<T> pa;
         pa.A = (V *)Ap; pa.lda = n; pa.strideA = 0; pa.n = n; pa.k = k;
-        pa.P = (n - k + RW - 1) / RW; pa.slots = slots;
+        pa.P = (n - k + RW - 1) / RW; pa.slots = slots; pa.pslot = 0;
         pa.ipiv = ipiv; pa.strideP = 0; pa.info = info;
         pa.err = ctx->d_err; pa.xbuf = xbuf; pa.bidx = nullptr; pa.tagp = ctx->d_tag; pa.toff = (uint32_t)k;
         pa.nmem = nullptr;
@@ -1802,6 +1868,7 @@ extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, 
         if (do_swap) {
             SwapArgs sa;
             sa.n = n; sa.k = k; sa.slots = slots; sa.do_swap = 1; sa.nmem = nullptr;
+            sa.pslot = 0; sa.c_l0 = 0; sa.c_l1 = k;
             sa.c_tr0 = k + NB; sa.c_tr1 = n; sa.c_sw0 = n;
             launch_swap<T>(ctx, sa, (V *)Ap, n, 0, xbuf, nullptr, 1, ctx->stream);
         }

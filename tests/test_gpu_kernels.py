@@ -93,3 +93,40 @@ def test_wide_batch_equals_single(wm, ctx, prec, n, batch):
         d1, p1, _ = wm.getrf_batched(ctx, A[b], prec)
         assert np.array_equal(p1.download()[0], P[b])
         assert np.array_equal(d1.download()[0], LU[b])
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16x3"])
+@pytest.mark.parametrize("n,batch", [(8192, 1), (4160, 4)])
+def test_lookahead_matches_one_stream(wm, ctx, prec, n, batch):
+    """Factorizations large enough for the look-ahead stream, captured and launched directly,
+    give the factors and pivots of the one-stream order (which the profiler keeps) bit for bit;
+    captures are replayed with other work and synchronizations in between."""
+    rng = np.random.RandomState(n)
+    A = np.empty((batch, n, n), np.complex64 if prec != "f64" else np.complex128)
+    for b in range(batch):
+        A[b].real = rng.standard_normal((n, n))
+        A[b].imag = rng.standard_normal((n, n))
+    host = np.ascontiguousarray(A.transpose(0, 2, 1))
+    dev, piv, _ = wm.getrf_batched(ctx, A, prec)
+
+    def factor():
+        import ctypes as C
+        dev.upload(host)
+        info = np.zeros(batch, np.int32)
+        rc = wm.lib().wm_getrf_batched(ctx.h, wm.PREC_NAMES[prec], n, dev.ptr, n, n * n, piv.ptr, n, batch,
+                                       info.ctypes.data_as(C.POINTER(C.c_int)))
+        assert rc == 0
+        return dev.download(), piv.download()
+
+    ctx.prof_enable(True)
+    ref = factor()
+    ctx.prof_enable(False)
+    for _ in range(2):  # replays
+        got = factor()
+        assert np.array_equal(got[1], ref[1]) and np.array_equal(got[0], ref[0])
+    ctx.set_graphs(False)
+    try:
+        got = factor()
+    finally:
+        ctx.set_graphs(True)
+    assert np.array_equal(got[1], ref[1]) and np.array_equal(got[0], ref[0])

@@ -823,6 +823,20 @@ int solve_items(wm_ctx *c, const wm_solve_opts &o, WorkItem *items, int count, h
         WM_TRY(copy_d2h(hnorm.data(), mx, count * sizeof(unsigned long long), s));
     }
 
+    // condition estimates of the listed items with the factors they have now
+    std::vector<double> cond(count, 0.0), anorm(count, 0.0);
+    for (int b = 0; b < count; ++b) std::memcpy(&anorm[b], &hnorm[b], 8);
+    auto estimate = [&](const std::vector<int> &lst, int f64) -> int {
+        if (lst.empty()) return WM_OK;
+        std::vector<int> np(lst.size());
+        for (size_t i = 0; i < lst.size(); ++i) np[i] = items[lst[i]].g->npls;
+        std::vector<double> est;
+        WM_TRY(inv_norm1_estimate(c, f64 ? WM_PREC_F64 : WM_PREC_F32, n, f64 ? (const void *)Z : (const void *)Z32, sZ,
+                                  perm, D, sV, lst, np, dact, s, est));
+        for (size_t i = 0; i < lst.size(); ++i) cond[lst[i]] = anorm[lst[i]] * est[i];
+        return WM_OK;
+    };
+
     std::vector<int> hinfo(count, 0), iters(count, 0), fell(count, 0);
     std::vector<double> dxr(count, 0.0), berr(count, 0.0);
     int noconv = 0;
@@ -849,6 +863,7 @@ int solve_items(wm_ctx *c, const wm_solve_opts &o, WorkItem *items, int count, h
         };
         if (!own.empty()) WM_TRY(factor_solve(own));
         for (int b : own) items[b].anchor_used = b;
+        if (o.cond_est) WM_TRY(estimate(own, 1));  // before the factors in use become preconditioners
         WM_TRY(aux_join.join());  // the other items' matrices are filled
         // the others: FP64 GMRES refinement preconditioned by the anchor's factors
         // (an anchor with a zero pivot preconditions nothing: its dependents are factored)
@@ -860,7 +875,7 @@ int solve_items(wm_ctx *c, const wm_solve_opts &o, WorkItem *items, int count, h
         if (!gdeps.empty()) {
             GmresArgs ga;
             ga.n = n; ga.nr = nr; ga.m = gm; ga.count = count;
-            ga.Z = Z; ga.sZ = sZ; ga.F = Z; ga.fprec = WM_PREC_F64; ga.sF = sZ; ga.perm = perm;
+            ga.Z = Z; ga.sZ = sZ; ga.F = Z; ga.sF = sZ; ga.perm = perm;
             ga.B = B; ga.X = X; ga.R = R; ga.D = D; ga.sV = sV;
             ga.K = Kry; ga.red = red; ga.dact = dact; ga.dfac = dfac; ga.mx = mx; ga.mx2 = mx2;
             ga.np = 0;
@@ -884,6 +899,7 @@ int solve_items(wm_ctx *c, const wm_solve_opts &o, WorkItem *items, int count, h
                 fell[b] = 1;
                 items[b].anchor_used = b;
             }
+            if (o.cond_est) WM_TRY(estimate(redo, 1));
         }
         for (int b = 0; b < count; ++b) items[b].fprec = WM_PREC_F64;
     } else if (!mixed) {
@@ -1016,28 +1032,15 @@ int solve_items(wm_ctx *c, const wm_solve_opts &o, WorkItem *items, int count, h
         }
     }
 
-    // condition estimates with the final factors of every item
-    std::vector<double> cond(count, 0.0), anorm(count, 0.0);
-    if (o.cond_est) {
-        for (int b = 0; b < count; ++b) {
-            unsigned long long bits = hnorm[b];
-            std::memcpy(&anorm[b], &bits, 8);
-        }
+    // condition estimates with the final factors of every item (a recycled
+    // batch has taken its anchors' while their factors stood)
+    if (o.cond_est && !recycle)
         for (int f64 = 0; f64 < 2; ++f64) {
             std::vector<int> lst;
-            for (int b = 0; b < count; ++b) {
-                if (recycle && items[b].anchor_used != b) continue;  // solved with another item's factors
+            for (int b = 0; b < count; ++b)
                 if ((mixed ? items[b].fprec == WM_PREC_F64 : true) == (f64 == 1)) lst.push_back(b);
-            }
-            if (lst.empty()) continue;
-            std::vector<int> np(lst.size());
-            for (size_t i = 0; i < lst.size(); ++i) np[i] = items[lst[i]].g->npls;
-            std::vector<double> est;
-            WM_TRY(inv_norm1_estimate(c, f64 ? WM_PREC_F64 : WM_PREC_F32, n, f64 ? (const void *)Z : (const void *)Z32,
-                                      sZ, perm, D, sV, lst, np, dact, s, est));
-            for (size_t i = 0; i < lst.size(); ++i) cond[lst[i]] = anorm[lst[i]] * est[i];
+            WM_TRY(estimate(lst, f64));
         }
-    }
 
     std::vector<double2> hX((size_t)sV * count);
     WM_TRY(check_device_error(c, s));
@@ -1090,13 +1093,4 @@ extern "C" int wmx_refine_decide(int nrhs, const double *dm, const double *xm, d
 {
     if (nrhs <= 0 || !dm || !xm || !prev || !first || !rate || !worst) return -100;
     return wm::refine_decide(nrhs, dm, xm, prev, it, tol, max_iter, *first, *rate, *worst);
-}
-
-// Internal hook: right-hand sides per launch member of the GMRES
-// preconditioner's grouped solves (1, 2, 4 or 8).
-extern "C" int wmx_set_group_cols(wm_ctx *ctx, int w)
-{
-    if (!ctx || (w != 1 && w != 2 && w != 4 && w != 8)) return WM_ERR_ARG;
-    ctx->group_cols = w;
-    return WM_OK;
 }

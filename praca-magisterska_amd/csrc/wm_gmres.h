@@ -15,8 +15,7 @@ struct GmresArgs {
     int count = 0;                 // items in the batch (the Krylov sets hold count members each)
     const double2 *Z = nullptr;    // complex128 matrices of the items
     int64_t sZ = 0;
-    const void *F = nullptr;       // LU factors: complex128 for fprec WM_PREC_F64, complex64 otherwise
-    int fprec = WM_PREC_F64;
+    double2 *F = nullptr;          // complex128 LU factors; those in use are rewritten (precond_prepare)
     int64_t sF = 0;
     const int *perm = nullptr;     // row permutation of each factor, n ints per factor
     const double2 *B = nullptr;    // right-hand sides

@@ -233,9 +233,9 @@ int gmres_ir(wm_ctx *c, const wm_solve_opts &o, const GmresArgs &a, const std::v
     std::vector<unsigned long long> hm((size_t)2 * cnt * nr);
     std::vector<double2> hred;
 
-    // the inverted diagonal blocks of every factor in use: the preconditioner
-    // applies them as products (its solves need not be backward stable; the
-    // FP64 residuals decide the result)
+    // every factor in use goes to the form of the preconditioner's solves, in
+    // place (its solves need not be backward stable; the FP64 residuals decide
+    // the result)
     std::vector<int> facs, slot_of;
     for (int f : fac) {
         if (f < 0) continue;
@@ -245,9 +245,9 @@ int gmres_ir(wm_ctx *c, const wm_solve_opts &o, const GmresArgs &a, const std::v
             facs.push_back(f);
         }
     }
-    WM_TRY(c->ws_dinv.ensure(diag_inv_bytes(n, std::max<int>(1, (int)facs.size()))));
+    WM_TRY(c->ws_dinv.ensure(precond_bytes(n, std::max<int>(1, (int)facs.size()))));
     double2 *dinv = (double2 *)c->ws_dinv.ptr;
-    WM_TRY(diag_inv_batched(c, a.fprec, n, a.F, n, a.sF, facs, dinv, s));
+    WM_TRY(precond_prepare(c, WM_PREC_F64, n, a.F, n, a.sF, facs, a.F, dinv, s));
 
     std::vector<int> uploaded;  // the list a.dact (and a.dfac) hold
     auto upload_idx = [&](const std::vector<int> &lst) -> int {
@@ -320,8 +320,7 @@ int gmres_ir(wm_ctx *c, const wm_solve_opts &o, const GmresArgs &a, const std::v
             hipLaunchKernelGGL(k_copy_set, dim3((unsigned)((sV + 255) / 256), nl), blk, 0, s, zk, vk, sV, a.dact);
             std::vector<int> fl(lst.size());
             for (size_t q = 0; q < lst.size(); ++q) fl[q] = facOf[lst[q]];
-            WM_TRY(getrs_grouped(c, a.fprec, n, nr, a.F, n, a.sF, a.perm, n, zk, sV, lst, fl, s, dinv, &slot_of,
-                                 c->group_cols));
+            WM_TRY(precond_solve(c, n, nr, a.F, n, a.sF, a.perm, n, dinv, slot_of, zk, sV, lst, fl, s));
             WM_TRY(residual_batched(c, n, nr, a.Z, n, a.sZ, zk, nullptr, n, sV, w, nl, s, a.dact,
                                     outer == 0 && k == 0 ? a.mx2 : nullptr, a.np));
             // classical Gram-Schmidt, twice; the coefficients stay on the device

@@ -118,7 +118,6 @@ struct wm_ctx {
     // second stream of recycled sweeps (wm_set_fill_overlap): the GMRES items'
     // fills, with their own self-term workspace; created on first use
     bool overlap_fill = true;
-    int group_cols = 4;  // preconditioner solves: right-hand sides per launch member (1, 2, 4 or 8)
     hipStream_t aux = nullptr;
     hipEvent_t aux_ev[2] = {nullptr, nullptr};  // launch stream -> aux, aux -> launch stream
     wm::DevBuf ws_fill2;
@@ -197,26 +196,25 @@ int getrs_perm_batched(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, in
 // Solves with shared factors: column r < nr of item items[q] (at V + items[q] *
 // strideV + r * n) is solved in place with the factors and permutation of
 // index fac[q].  The columns of items that share a factor are the right-hand
-// sides of one launch member (up to max_w per member), so each factor is read
-// once per member rather than once per column; a column's arithmetic is the
-// same whatever it is grouped with.  A triangular solve's time per 64-row
-// block grows with its right-hand sides while its chain of blocks is
-// latency-bound, so members of a few columns each run faster than one wide
-// member (kGroupCols).
-// With dinv (the inverted diagonal blocks of diag_inv_batched, factor f in slot
-// (*slot_of)[f]) each diagonal block is applied as a product instead of a
-// substitution: not backward stable like the substitution, for preconditioner
-// applications only.
-constexpr int kGroupCols = 4;
+// sides of one launch member (up to max_w <= 8 per member); a column's
+// arithmetic is the same whatever it is grouped with.
 int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, int64_t strideF, const int *perm,
                   int64_t strideQ, double2 *V, int64_t strideV, const std::vector<int> &items,
-                  const std::vector<int> &fac, hipStream_t s, const double2 *dinv = nullptr,
-                  const std::vector<int> *slot_of = nullptr, int max_w = kGroupCols);
-// Inverses of the 64 x 64 diagonal blocks of the factors of index factors[z]
-// into slot z of Dinv (diag_inv_bytes(n, factors.size()) bytes), FP64.
-size_t diag_inv_bytes(int n, int nfac);
-int diag_inv_batched(wm_ctx *ctx, int prec, int n, const void *F, int lda, int64_t strideF,
-                     const std::vector<int> &factors, double2 *Dinv, hipStream_t s);
+                  const std::vector<int> &fac, hipStream_t s, int max_w);
+// Preconditioner solves with shared factors, grouped likewise in members of up
+// to 16 columns.  precond_prepare takes the factors of the listed indices
+// (complex128 for WM_PREC_F64, complex64 otherwise) to the form the solves use:
+// the inverses of their 64 x 64 diagonal blocks in slot z of Dinv
+// (precond_bytes(n, factors.size()) bytes), and every row block times its
+// inverse in Fs (complex128, same layout and stride; may be the factors
+// themselves, whose off-diagonal blocks it then replaces).  Not backward stable
+// like substitution: for preconditioner applications only.
+size_t precond_bytes(int n, int nfac);
+int precond_prepare(wm_ctx *ctx, int prec, int n, const void *F, int lda, int64_t strideF,
+                    const std::vector<int> &factors, double2 *Fs, double2 *Dinv, hipStream_t s);
+int precond_solve(wm_ctx *ctx, int n, int nr, const double2 *Fs, int lda, int64_t strideF, const int *perm,
+                  int64_t strideQ, const double2 *Dinv, const std::vector<int> &slot_of, double2 *V, int64_t strideV,
+                  const std::vector<int> &items, const std::vector<int> &fac, hipStream_t s);
 // Solves A^H X = B with the same factors and permutation (A = P^T L U, so
 // X = P^T L^-H U^-H B); used by the condition estimate.
 int getrsh_perm_batched(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int lda, int64_t strideA,

@@ -89,8 +89,6 @@ struct TrsvArgs {
     int *err;
     const int *bidx;      // launch member -> matrix index of B and Y (null: identity)
     const int *aidx;      // launch member -> matrix index of the factors and permutation (null: as bidx)
-    const double2 *dinv;  // inverted diagonal blocks (k_diag_inv), used instead of substitution, or null
-    const int *dslot;     // launch member -> slot of its factors' blocks in dinv
 };
 
 // Packed entries of one 64 x 64 triangle with its diagonal.
@@ -131,7 +129,7 @@ __device__ inline int du_idx(int i, int j) { return j * (j + 1) / 2 + i; }
 // right-hand sides as staged (no gather), the upper pass L^H (upper, unit
 // diagonal) in place; element (i, j) of the triangle is conj(A(j, i)).  The
 // caller scatters the result through the permutation (x = P^T w).
-template <typename T, int NR, bool UPPER, bool TRANS, bool INV = false>
+template <typename T, int NR, bool UPPER, bool TRANS>
 __global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
 {
     // no contraction: a right-hand side's arithmetic is the same in every
@@ -160,11 +158,7 @@ __global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
     // diagonal block to LDS (independent of other blocks, so before any wait)
     __shared__ double2 s_d[kPack];
     __shared__ double2 s_rd[TB];
-    if (INV) {
-        const double2 *D = a.dinv + (((size_t)a.dslot[bl] * 2 + (UPPER ? 1 : 0)) * nblk + bi) * kPack;
-        for (int e = tid; e < kPack; e += 256) s_d[e] = D[e];
-    }
-    for (int e = tid; !INV && e < TB * TB; e += 256) {
+    for (int e = tid; e < TB * TB; e += 256) {
         // consecutive threads walk down a column of the stored factor
         const int i = TRANS ? e / TB : e % TB, j = TRANS ? e % TB : e / TB;
         if (!UPPER && i > j) s_d[dl_idx(i, j)] = elem(A, r0 + i, r0 + j);
@@ -255,29 +249,7 @@ __global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
                 for (int p = 1; p < 4; ++p) { x[k].x += s_acc[p][row][r].x; x[k].y += s_acc[p][row][r].y; }
             }
         }
-        if (INV) {
-            // x = D^-1 a with the inverted diagonal block: a product instead of
-            // a 64-step substitution (the wave's sums go through its own LDS
-            // entries; the block of L^-1 has a unit diagonal)
-#pragma unroll
-            for (int k = 0; k < RW; ++k)
-                if (part + 4 * k < NR) s_acc[0][row][part + 4 * k] = x[k];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-            for (int k = 0; k < RW; ++k) {
-                const int r = part + 4 * k;
-                if (r >= NR) break;
-                double2 v = UPPER ? make_double2(0.0, 0.0) : x[k];
-#pragma unroll
-                for (int j = 0; j < TB; ++j) {
-                    if (UPPER ? j >= row : j < row)
-                        cfma(v, s_d[UPPER ? du_idx(row, j) : dl_idx(row, j)], s_acc[0][j][r]);
-                }
-                x[k] = v;
-            }
-        } else if (!UPPER) {
+        if (!UPPER) {
         // the substitution is the launch's critical path: unrolled, so each
         // step's LDS read of the block is issued ahead of the step
 #pragma unroll
@@ -437,11 +409,6 @@ template <typename T, int NR, bool TRANS>
 void launch_trsv(const TrsvArgs &a, int batch, int r_off, bool upper, hipStream_t s)
 {
     const dim3 grid(batch, a.n / TB);
-    if (a.dinv && !TRANS) {
-        if (upper) hipLaunchKernelGGL((k_trsv<T, NR, true, false, true>), grid, dim3(256), 0, s, a, r_off);
-        else hipLaunchKernelGGL((k_trsv<T, NR, false, false, true>), grid, dim3(256), 0, s, a, r_off);
-        return;
-    }
     if (upper) hipLaunchKernelGGL((k_trsv<T, NR, true, TRANS>), grid, dim3(256), 0, s, a, r_off);
     else hipLaunchKernelGGL((k_trsv<T, NR, false, TRANS>), grid, dim3(256), 0, s, a, r_off);
 }
@@ -450,8 +417,7 @@ void launch_trsv(const TrsvArgs &a, int batch, int r_off, bool upper, hipStream_
 // blockIdx = (block, triangle 0 = L (unit lower) / 1 = U, slot); slot z
 // takes the factors of index fidx[z].  Lane j solves for column j of the
 // inverse by substitution against the block staged in LDS; the inverse is
-// stored packed as the triangular solve stages it (strictly lower part of
-// L^-1, upper part of U^-1 with its diagonal), kPack entries per block.
+// stored whole, column by column, zeros in its other triangle.
 template <typename T>
 __global__ __launch_bounds__(64) void k_diag_inv(const void *F, int lda, int64_t strideF, const int *fidx, int nblk,
                                                  double2 *Dinv)
@@ -486,12 +452,281 @@ __global__ __launch_bounds__(64) void k_diag_inv(const void *F, int lda, int64_t
         }
     }
     __syncthreads();
-    double2 *D = Dinv + (((size_t)blockIdx.z * 2 + upper) * nblk + bi) * kPack;
+    double2 *D = Dinv + (((size_t)blockIdx.z * 2 + upper) * nblk + bi) * TB * TB;
     for (int e = j; e < TB * TB; e += TB) {
         const int i = e % TB, k = e / TB;
-        if (!upper && i > k) D[dl_idx(i, k)] = s_x[i][k];
-        if (upper && i <= k) D[du_idx(i, k)] = s_x[i][k];
+        D[e] = (upper ? i <= k : i >= k) ? s_x[i][k] : make_double2(0.0, 0.0);
     }
+}
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// Preconditioner factors: every row block of L and U times the inverse of its
+// diagonal block, L' = diag(L_ii)^-1 L and U' = diag(U_ii)^-1 U, so that a solve
+// needs no work on the diagonal between one block's values and the next's.
+// blockIdx = (column block, row block, slot); row block bi of factor fidx[z],
+// column block cb (left of the diagonal: L, right of it: U) is multiplied by
+// its inverse on the matrix cores (three real products per complex product,
+// lanes as in k_psolve) and written to dst, which may be the factors themselves.
+template <typename T>
+__global__ __launch_bounds__(256) void k_scale_blocks(const void *F, double2 *dst, int lda, int64_t strideF,
+                                                      const int *fidx, int nblk, const double2 *Dinv)
+{
+    using V = typename CT<T>::V;
+    const int cb = blockIdx.x, bi = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (cb == bi) return;
+    const int upper = cb > bi;
+    const size_t base = (size_t)fidx[blockIdx.z] * strideF + (size_t)bi * TB + (size_t)cb * TB * lda;
+    const V *A = (const V *)F + base;
+    const double2 *D = Dinv + (((size_t)blockIdx.z * 2 + upper) * nblk + bi) * TB * TB;
+    __shared__ double2 s_t[TB][TB];  // s_t[k][(column + k) % TB]: both sides free of bank conflicts
+    for (int e = tid; e < TB * TB; e += 256) {
+        // consecutive lanes walk down a column
+        s_t[e % TB][(e / TB + e % TB) % TB] = ld2<T>(A + e % TB + (size_t)(e / TB) * lda);
+    }
+    __syncthreads();
+    v4d P[4], Q[4], S[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) P[c] = Q[c] = S[c] = v4d{0, 0, 0, 0};
+    for (int k = lane / 16; k < TB; k += 4) {
+        const double2 d = D[(size_t)k * TB + wave * 16 + lane % 16];
+        const double ds = d.x + d.y;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const double2 t = s_t[k][(c * 16 + lane % 16 + k) % TB];
+            P[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x, d.x, P[c], 0, 0, 0);
+            Q[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.y, d.y, Q[c], 0, 0, 0);
+            S[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.x + t.y, ds, S[c], 0, 0, 0);
+        }
+    }
+    double2 *O = dst + base + wave * 16 + lane % 16;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            O[(size_t)(c * 16 + lane / 16 + 4 * v) * lda] =
+                make_double2(P[c][v] - Q[c][v], S[c][v] - P[c][v] - Q[c][v]);
+}
+
+// Preconditioner solve L' y = diag(L_ii)^-1 P b (UPPER: U' x = diag(U_ii)^-1 y) for up
+// to kPsW right-hand sides per launch member, one launch.  Workgroup (member,
+// g) owns row block bi (lower: g, upper: nblk-1-g): c = D_ii^-1 b, then c minus
+// the products with the solved blocks as their values arrive, on the matrix
+// cores (wave w < 4: rows 16 w ..; three real products per complex product; a
+// right-hand side is a column of the products, so its values do not depend on
+// its neighbours).  Values of a block travel as plain 8-byte words: a member's
+// blocks are filled with kPsEmpty, a NaN pattern no arithmetic produces, before
+// the launch, and a reader polls its words until they hold something else.
+// Four more waves do the polling: a wave's loads complete in order, so a poll
+// behind the next block's factor entries would wait for HBM in every step.
+// Waits only on blocks of workgroups with smaller ids (dispatched earlier).
+//
+// What bounds it: the chain of n / 64 blocks, 2.0 us each with up to 4 columns and
+// 3.6 us with 16 (0.5 us for the values to cross, the rest the product of the
+// newest block: 48 4x4x4 products per wave for 4 columns, 96 for 8, 48 16x16x4,
+// at four times the cycles each, above).  The 4x4x4 form spends nothing on
+// columns that are not there and rounds like the 16x16x4 one: a column has the
+// same bits in every width.  Per triangle at N = 8192, against substitution by
+// inverted diagonal blocks on the vector units, four columns per member:
+//   1 factor, 3 columns    258 us instead of 1004
+//   2 factors, 16 columns  466 us instead of 1245 (factors read once, not 4 times)
+//   N = 512, 3 columns      18 us instead of 65
+// One polling wave instead of four: 470 us for 1 x 3 before the 4x4x4 form, 355
+// with four; real and imaginary words apart (whole lines per store): 470 us
+// instead of 628 for 2 x 16.
+constexpr int kPsW = 16;
+constexpr int kPsPoll = 4;
+constexpr uint64_t kPsEmpty = 0x7ff8b10c5e7afe55ull;
+
+struct PsolveArgs {
+    const double2 *F;       // scaled factors
+    int lda;
+    int64_t strideF;
+    int n;
+    const double2 *dinv;
+    const double *in;       // right-hand sides, [member][block][kPsW][re, im][TB]
+    uint64_t *pub;          // solved values, the same layout
+    const int *fac, *slot, *width;  // per member: factor, its slot in dinv, its right-hand sides
+    int *err;
+};
+
+template <bool UPPER>
+__global__ __launch_bounds__(256 + 64 * kPsPoll) void k_psolve(PsolveArgs a)
+{
+    const int bl = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nblk = a.n / TB;
+    const int bi = UPPER ? nblk - 1 - (int)blockIdx.y : (int)blockIdx.y, r0 = bi * TB;
+    const int w = a.width[bl];
+    uint64_t *pub = a.pub + (size_t)bl * a.n * kPsW * 2;
+    const int noff = UPPER ? nblk - 1 - bi : bi;
+    auto blk = [&](int q) { return UPPER ? nblk - 1 - q : q; };
+    // two buffers: a block's values are staged while the previous ones are read
+    __shared__ double2 s_y[2][kPsW][TB + 1];
+
+    if (wave >= 4) {  // the values of the other blocks: lane = row, wave 4 + j has columns j, j + kPsPoll, ...
+        constexpr int kE = kPsW / kPsPoll;
+        const int j0 = wave - 4;
+        __syncthreads();
+        for (int q = 0; q < noff; ++q) {
+            const uint64_t *py = pub + (((size_t)blk(q) * kPsW + j0) * 2) * TB + lane;
+            uint64_t yx[kE], yy[kE];
+            long it = 0;
+            for (;;) {
+#pragma unroll
+                for (int e = 0; e < kE; ++e) {
+                    yx[e] = yy[e] = 0;
+                    if (j0 + kPsPoll * e < w) {
+                        yx[e] = ld_pkt(py + 2 * kPsPoll * TB * e);
+                        yy[e] = ld_pkt(py + 2 * kPsPoll * TB * e + TB);
+                    }
+                }
+                bool got = true;
+#pragma unroll
+                for (int e = 0; e < kE; ++e) got = got & (yx[e] != kPsEmpty) & (yy[e] != kPsEmpty);
+                if (__all(got)) break;
+                if (spin_give_up(it, a.err)) break;
+            }
+#pragma unroll
+            for (int e = 0; e < kE; ++e)
+                if (j0 + kPsPoll * e < w)
+                    s_y[(q + 1) & 1][j0 + kPsPoll * e][lane] = make_double2(
+                        __longlong_as_double((long long)yx[e]), __longlong_as_double((long long)yy[e]));
+            __syncthreads();
+        }
+        return;
+    }
+
+    const double2 *A = a.F + (size_t)a.fac[bl] * a.strideF;
+    const double2 *D = a.dinv + (((size_t)a.slot[bl] * 2 + (UPPER ? 1 : 0)) * nblk + bi) * TB * TB;
+    const int row = wave * 16 + lane % 16, kq = lane / 16, rhs = lane % 16;
+    double2 lcur[16], lnext[16];  // this lane's factor entries: row, columns kq + 4 t of a block
+    auto load_block = [&](int q, double2 *l) {
+        const double2 *p = A + r0 + row + (size_t)(q * TB + kq) * a.lda;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) l[t] = p[(size_t)(4 * t) * a.lda];
+    };
+    v4d P, Q, S;
+    auto product = [&](const double2 *l, int buf) {
+        P = Q = S = v4d{0, 0, 0, 0};
+        if (w <= 4) {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                const double2 y = s_y[buf][lane % 4][4 * t + kq];
+                P[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, l[t].x, P[0], 0, 0, 0);
+                Q[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, l[t].y, Q[0], 0, 0, 0);
+                S[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x + y.y, l[t].x + l[t].y, S[0], 0, 0, 0);
+            }
+            return;
+        }
+        if (w <= 8) {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const double2 y = s_y[buf][4 * g + lane % 4][4 * t + kq];
+                    P[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, l[t].x, P[g], 0, 0, 0);
+                    Q[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, l[t].y, Q[g], 0, 0, 0);
+                    S[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x + y.y, l[t].x + l[t].y, S[g], 0, 0, 0);
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const double2 y = s_y[buf][rhs][4 * t + kq];
+            P = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, l[t].x, P, 0, 0, 0);
+            Q = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, l[t].y, Q, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x + y.y, l[t].x + l[t].y, S, 0, 0, 0);
+        }
+    };
+
+    // c = D^-1 b (this lane: row `row`, right-hand sides kq + 4 v)
+    const double *in = a.in + (((size_t)bl * nblk + bi) * kPsW + wave) * 2 * TB + lane;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_y[0][wave + 4 * e][lane] = make_double2(in[8 * TB * e], in[8 * TB * e + TB]);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) lcur[t] = D[row + (size_t)(4 * t + kq) * TB];
+    __syncthreads();
+    product(lcur, 0);
+    double cr[4], ci[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        cr[v] = P[v] - Q[v];
+        ci[v] = S[v] - P[v] - Q[v];
+    }
+    auto subtract = [&]() {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            cr[v] -= P[v] - Q[v];
+            ci[v] -= S[v] - P[v] - Q[v];
+        }
+    };
+    // Two blocks per turn, loads without a condition (past the end: the last
+    // block once more), so that a product's wait counts leave the next block's
+    // loads in flight; an odd block goes first.
+    int q = noff & 1;
+    if (q) {
+        load_block(blk(0), lnext);
+        load_block(blk(min(1, noff - 1)), lcur);
+        __syncthreads();
+        product(lnext, 1);
+        subtract();
+    } else if (noff > 0) {
+        load_block(blk(0), lcur);
+    }
+    for (; q < noff; q += 2) {
+        load_block(blk(q + 1), lnext);
+        __syncthreads();
+        product(lcur, (q + 1) & 1);
+        subtract();
+        load_block(blk(min(q + 2, noff - 1)), lcur);
+        __syncthreads();
+        product(lnext, q & 1);
+        subtract();
+    }
+    auto word = [](double x) {
+        const uint64_t u = (uint64_t)__double_as_longlong(x);
+        return u == kPsEmpty ? 0x7ff8000000000000ull : u;
+    };
+    uint64_t *o = pub + (size_t)bi * kPsW * 2 * TB + row;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (kq + 4 * v < w) {
+            uint64_t *ov = o + (kq + 4 * v) * 2 * TB;
+            __hip_atomic_store(ov, word(cr[v]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(ov + TB, word(ci[v]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+}
+
+// Right-hand sides of a preconditioner solve, [member][block][kPsW][re, im][TB]:
+// rows through perm of column cols[member * kPsW + j] of V (element offset; -1:
+// zero), and both triangles' values marked empty (pub, pub + members * n *
+// kPsW complex words).
+__global__ void k_ps_gather(const double2 *V, int n, const int64_t *cols, const int *fac, const int *perm,
+                            int64_t strideQ, double *in, uint64_t *pub, int members)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
+    if (t >= n * kPsW) return;
+    const int row = t / (TB * kPsW) * TB + t % TB, j = t / TB % kPsW;
+    const int64_t c = cols[(size_t)m * kPsW + j];
+    const size_t o = (size_t)m * n * kPsW * 2 + (size_t)(t / TB) * 2 * TB + t % TB;
+    const double2 v = c >= 0 ? V[c + perm[(size_t)fac[m] * strideQ + row]] : make_double2(0.0, 0.0);
+    in[o] = v.x;
+    in[o + TB] = v.y;
+    const size_t half = (size_t)members * n * kPsW * 2;
+    pub[o] = pub[o + TB] = pub[half + o] = pub[half + o + TB] = kPsEmpty;
+}
+
+// The solved columns back to V.
+__global__ void k_ps_scatter(const double *pub, int n, const int64_t *cols, double2 *V)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
+    if (t >= n * kPsW) return;
+    const int row = t / (TB * kPsW) * TB + t % TB, j = t / TB % kPsW;
+    const int64_t c = cols[(size_t)m * kPsW + j];
+    const double *p = pub + (size_t)m * n * kPsW * 2 + (size_t)(t / TB) * 2 * TB + t % TB;
+    if (c >= 0) V[c + row] = make_double2(p[0], p[TB]);
 }
 
 // Right-hand sides handled by one pass starting at r_off: 8, 4, 2 or 1.
@@ -578,8 +813,7 @@ size_t solve_pkts(int n, int nrhs, int batch) { return 2 * (size_t)batch * (n / 
 // (nothing allocated, no profiler events).
 int getrs_any(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int lda, int64_t strideA, const int *perm,
               int64_t strideQ, void *B, int ldb, int64_t strideB, int batch, hipStream_t s, const int *d_bidx,
-              bool trans, const int *d_aidx, SolveBufs *ext = nullptr, const double2 *dinv = nullptr,
-              const int *d_dslot = nullptr)
+              bool trans, const int *d_aidx, SolveBufs *ext = nullptr)
 {
     if (n <= 0 || n % TB != 0 || nrhs <= 0 || batch <= 0 || ldb < n) {
         set_error("getrs: bad arguments (n=%d multiple of %d, nrhs=%d, batch=%d)", n, TB, nrhs, batch);
@@ -625,8 +859,6 @@ int getrs_any(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int lda, in
         a.perm = perm; a.strideQ = strideQ; a.ldb = ldb; a.strideB = strideB; a.err = ctx->d_err;
         a.bidx = d_bidx;
         a.aidx = d_aidx;
-        a.dinv = trans ? nullptr : dinv;
-        a.dslot = d_dslot;
         a.Bin = Ystage; a.Y = (double2 *)B; a.pkt = pkt;
         a.epoch = ++*epoch;
         const int nr = rhs_chunk(nrhs - r0);
@@ -695,38 +927,40 @@ __global__ void k_scatter_cols(const double2 *S, int n, const int64_t *cols, dou
 
 }  // namespace
 
-size_t diag_inv_bytes(int n, int nfac) { return (size_t)nfac * 2 * (n / TB) * kPack * sizeof(double2); }
+size_t precond_bytes(int n, int nfac) { return (size_t)nfac * 2 * n * TB * sizeof(double2); }
 
-int diag_inv_batched(wm_ctx *ctx, int prec, int n, const void *F, int lda, int64_t strideF,
-                     const std::vector<int> &factors, double2 *Dinv, hipStream_t s)
+int precond_prepare(wm_ctx *ctx, int prec, int n, const void *F, int lda, int64_t strideF,
+                    const std::vector<int> &factors, double2 *Fs, double2 *Dinv, hipStream_t s)
 {
     if (factors.empty()) return WM_OK;
     if (n % TB != 0) {
-        set_error("diag_inv: n=%d not a multiple of %d", n, TB);
+        set_error("precond_prepare: n=%d not a multiple of %d", n, TB);
         return WM_ERR_ARG;
     }
     WM_TRY(ctx->ws_dinv_idx.ensure(factors.size() * sizeof(int)));
     WM_TRY(copy_h2d(ctx->ws_dinv_idx.ptr, factors.data(), factors.size() * sizeof(int), s));
-    const dim3 grid((unsigned)(n / TB), 2, (unsigned)factors.size());
+    const unsigned nblk = (unsigned)(n / TB), nf = (unsigned)factors.size();
     const int *fidx = (const int *)ctx->ws_dinv_idx.ptr;
-    if (prec == WM_PREC_F64)
-        hipLaunchKernelGGL(k_diag_inv<double>, grid, dim3(TB), 0, s, F, lda, strideF, fidx, n / TB, Dinv);
-    else
-        hipLaunchKernelGGL(k_diag_inv<float>, grid, dim3(TB), 0, s, F, lda, strideF, fidx, n / TB, Dinv);
+    if (prec == WM_PREC_F64) {
+        hipLaunchKernelGGL(k_diag_inv<double>, dim3(nblk, 2, nf), dim3(TB), 0, s, F, lda, strideF, fidx, n / TB, Dinv);
+        hipLaunchKernelGGL(k_scale_blocks<double>, dim3(nblk, nblk, nf), dim3(256), 0, s, F, Fs, lda, strideF, fidx,
+                           n / TB, (const double2 *)Dinv);
+    } else {
+        hipLaunchKernelGGL(k_diag_inv<float>, dim3(nblk, 2, nf), dim3(TB), 0, s, F, lda, strideF, fidx, n / TB, Dinv);
+        hipLaunchKernelGGL(k_scale_blocks<float>, dim3(nblk, nblk, nf), dim3(256), 0, s, F, Fs, lda, strideF, fidx,
+                           n / TB, (const double2 *)Dinv);
+    }
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
 }
 
-int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, int64_t strideF, const int *perm,
-                  int64_t strideQ, double2 *V, int64_t strideV, const std::vector<int> &items,
-                  const std::vector<int> &fac, hipStream_t s, const double2 *dinv, const std::vector<int> *slot_of,
-                  int max_w)
+namespace {
+
+// Columns of items that share a factor, cut into members of up to max_w: the
+// factor of each member and W column offsets (-1: none) per member.
+int group_columns(int n, int nr, int64_t strideV, const std::vector<int> &items, const std::vector<int> &fac,
+                  int max_w, std::vector<int> &member_fac, std::vector<int64_t> &cols, int &W)
 {
-    if (items.empty()) return WM_OK;
-    if (items.size() != fac.size() || nr <= 0 || strideV < (int64_t)n * nr) {
-        set_error("getrs_grouped: bad arguments");
-        return WM_ERR_ARG;
-    }
     // the columns of each factor, factors in the order of their first item
     std::vector<int> order;
     std::vector<std::vector<int64_t>> cols_of;
@@ -734,7 +968,7 @@ int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, 
     for (size_t q = 0; q < items.size(); ++q) {
         const int f = fac[q];
         if (f < 0) {
-            set_error("getrs_grouped: item %d has no factors", items[q]);
+            set_error("grouped solve: item %d has no factors", items[q]);
             return WM_ERR_ARG;
         }
         if ((size_t)f >= pos_of.size()) pos_of.resize((size_t)f + 1, -1);
@@ -747,46 +981,114 @@ int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, 
     }
     size_t widest = 0;
     for (const auto &c : cols_of) widest = std::max(widest, c.size());
-    int W = 1;  // right-hand sides per launch member: a power of two, at most max_w (<= 8)
-    while (W < std::min(max_w, 8) && (size_t)W < widest) W *= 2;
-    std::vector<int> aidx;
-    std::vector<int64_t> cols;
+    W = 1;  // right-hand sides per launch member: a power of two, at most max_w
+    while (W < max_w && (size_t)W < widest) W *= 2;
+    if (max_w == kPsW) W = kPsW;
     for (size_t g = 0; g < order.size(); ++g)
         for (size_t j0 = 0; j0 < cols_of[g].size(); j0 += W) {
-            aidx.push_back(order[g]);
+            member_fac.push_back(order[g]);
             for (int j = 0; j < W; ++j)
                 cols.push_back(j0 + j < cols_of[g].size() ? cols_of[g][j0 + j] : (int64_t)-1);
         }
-    const int members = (int)aidx.size();
-    std::vector<int> dslot(members, 0);
-    if (dinv) {
-        for (int m = 0; m < members; ++m) {
-            const int f = aidx[m];
-            if (!slot_of || f >= (int)slot_of->size() || (*slot_of)[f] < 0) {
-                set_error("getrs_grouped: factor %d has no inverted diagonal blocks", f);
-                return WM_ERR_ARG;
-            }
-            dslot[m] = (*slot_of)[f];
-        }
+    return WM_OK;
+}
+
+}  // namespace
+
+int precond_solve(wm_ctx *ctx, int n, int nr, const double2 *Fs, int lda, int64_t strideF, const int *perm,
+                  int64_t strideQ, const double2 *Dinv, const std::vector<int> &slot_of, double2 *V, int64_t strideV,
+                  const std::vector<int> &items, const std::vector<int> &fac, hipStream_t s)
+{
+    if (items.empty()) return WM_OK;
+    if (items.size() != fac.size() || nr <= 0 || strideV < (int64_t)n * nr || n % TB != 0) {
+        set_error("precond_solve: bad arguments");
+        return WM_ERR_ARG;
     }
+    std::vector<int> mf;
+    std::vector<int64_t> cols;
+    int W = kPsW;
+    WM_TRY(group_columns(n, nr, strideV, items, fac, kPsW, mf, cols, W));
+    const int members = (int)mf.size();
+    // tables: factor, slot, width per member, then the columns
+    std::vector<int> tab(3 * (size_t)members);
+    for (int m = 0; m < members; ++m) {
+        const int f = mf[m];
+        if (f >= (int)slot_of.size() || slot_of[f] < 0) {
+            set_error("precond_solve: factor %d was not prepared", f);
+            return WM_ERR_ARG;
+        }
+        tab[m] = f;
+        tab[members + m] = slot_of[f];
+        int w = 0;
+        while (w < kPsW && cols[(size_t)m * kPsW + w] >= 0) ++w;
+        tab[2 * members + m] = w;
+    }
+    const size_t tab_b = (tab.size() * sizeof(int) + 255) & ~(size_t)255;
+    const size_t cols_b = (cols.size() * sizeof(int64_t) + 255) & ~(size_t)255;
+    const size_t vec_b = (size_t)members * n * kPsW * sizeof(double2);
+    WM_TRY(ctx->ws_group.ensure(tab_b + cols_b + 3 * vec_b));
+    char *base = (char *)ctx->ws_group.ptr;
+    std::vector<char> host(tab_b + cols_b, 0);
+    std::memcpy(host.data(), tab.data(), tab.size() * sizeof(int));
+    std::memcpy(host.data() + tab_b, cols.data(), cols.size() * sizeof(int64_t));
+    WM_TRY(copy_h2d(base, host.data(), host.size(), s));
+    const int *d_tab = (const int *)base;
+    const int64_t *d_cols = (const int64_t *)(base + tab_b);
+    double *in = (double *)(base + tab_b + cols_b);
+    uint64_t *pub = (uint64_t *)(base + tab_b + cols_b + vec_b);
+    uint64_t *pub2 = pub + (size_t)members * n * kPsW * 2;
+    const dim3 grid((unsigned)members, (unsigned)(n / TB)), vgrid((unsigned)(n * kPsW / 256), (unsigned)members);
+    const double fl = 4.0 * (double)n * n * items.size() * nr, by = members * 8.0 * (double)n * n;
+    hipLaunchKernelGGL(k_ps_gather, vgrid, dim3(256), 0, s,
+                       (const double2 *)V, n, d_cols, d_tab, perm, strideQ, in, pub, members);
+    PsolveArgs a;
+    a.F = Fs; a.lda = lda; a.strideF = strideF; a.n = n; a.dinv = Dinv;
+    a.fac = d_tab; a.slot = d_tab + members; a.width = d_tab + 2 * members;
+    a.err = ctx->d_err;
+    a.in = in; a.pub = pub;
+    prof_begin(ctx, K_TRSV, s);
+    hipLaunchKernelGGL(k_psolve<false>, grid, dim3(256 + 64 * kPsPoll), 0, s, a);
+    prof_end(ctx, K_TRSV, s, fl, by);
+    a.in = (const double *)pub; a.pub = pub2;  // the lower triangle's values are the upper one's right-hand sides
+    prof_begin(ctx, K_TRSV, s);
+    hipLaunchKernelGGL(k_psolve<true>, grid, dim3(256 + 64 * kPsPoll), 0, s, a);
+    prof_end(ctx, K_TRSV, s, fl, by);
+    hipLaunchKernelGGL(k_ps_scatter, vgrid, dim3(256), 0, s,
+                       (const double *)pub2, n, d_cols, V);
+    WM_HIP_TRY(hipGetLastError());
+    return WM_OK;
+}
+
+int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, int64_t strideF, const int *perm,
+                  int64_t strideQ, double2 *V, int64_t strideV, const std::vector<int> &items,
+                  const std::vector<int> &fac, hipStream_t s, int max_w)
+{
+    if (items.empty()) return WM_OK;
+    if (items.size() != fac.size() || nr <= 0 || strideV < (int64_t)n * nr) {
+        set_error("getrs_grouped: bad arguments");
+        return WM_ERR_ARG;
+    }
+    std::vector<int> aidx;
+    std::vector<int64_t> cols;
+    int W = 1;
+    WM_TRY(group_columns(n, nr, strideV, items, fac, std::min(max_w, 8), aidx, cols, W));
+    const int members = (int)aidx.size();
     const size_t aidx_b = ((size_t)members * sizeof(int) + 255) & ~(size_t)255;
     const size_t cols_b = ((size_t)members * W * sizeof(int64_t) + 255) & ~(size_t)255;
     const size_t stage_b = (size_t)members * W * n * sizeof(double2);
-    WM_TRY(ctx->ws_group.ensure(2 * aidx_b + cols_b + stage_b));
+    WM_TRY(ctx->ws_group.ensure(aidx_b + cols_b + stage_b));
     char *base = (char *)ctx->ws_group.ptr;
-    std::vector<char> host(2 * aidx_b + cols_b, 0);
+    std::vector<char> host(aidx_b + cols_b, 0);
     std::memcpy(host.data(), aidx.data(), aidx.size() * sizeof(int));
-    std::memcpy(host.data() + aidx_b, dslot.data(), dslot.size() * sizeof(int));
-    std::memcpy(host.data() + 2 * aidx_b, cols.data(), cols.size() * sizeof(int64_t));
+    std::memcpy(host.data() + aidx_b, cols.data(), cols.size() * sizeof(int64_t));
     WM_TRY(copy_h2d(base, host.data(), host.size(), s));
     const int *d_aidx = (const int *)base;
-    const int *d_dslot = (const int *)(base + aidx_b);
-    const int64_t *d_cols = (const int64_t *)(base + 2 * aidx_b);
-    double2 *S = (double2 *)(base + 2 * aidx_b + cols_b);
+    const int64_t *d_cols = (const int64_t *)(base + aidx_b);
+    double2 *S = (double2 *)(base + aidx_b + cols_b);
     const dim3 grid((unsigned)((n + 255) / 256), (unsigned)(members * W));
     hipLaunchKernelGGL(k_gather_cols, grid, dim3(256), 0, s, (const double2 *)V, n, d_cols, S);
     WM_TRY(getrs_any(ctx, prec, n, W, F, lda, strideF, perm, strideQ, S, n, (int64_t)W * n, members, s, nullptr,
-                     false, d_aidx, nullptr, dinv, dinv ? d_dslot : nullptr));
+                     false, d_aidx));
     hipLaunchKernelGGL(k_scatter_cols, grid, dim3(256), 0, s, (const double2 *)S, n, d_cols, V);
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
@@ -941,18 +1243,26 @@ extern "C" int wmx_getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const voi
     WM_TRY(ctx->ws_perm.ensure((size_t)nfac * n * sizeof(int)));
     int *perm = (int *)ctx->ws_perm.ptr;
     WM_TRY(perm_batched(ctx, n, ipiv, n, perm, n, nfac, ctx->stream));
-    const double2 *dinv = nullptr;
-    std::vector<int> facs(nfac), slot(nfac);
-    for (int f = 0; f < nfac; ++f) facs[f] = slot[f] = f;
-    if (inv) {
-        WM_TRY(ctx->ws_dinv.ensure(diag_inv_bytes(n, nfac)));
-        dinv = (const double2 *)ctx->ws_dinv.ptr;
-        WM_TRY(diag_inv_batched(ctx, prec, n, A, n, (int64_t)n * n, facs, (double2 *)dinv, ctx->stream));
+    const std::vector<int> its(items, items + nitems), fs(fac, fac + nitems);
+    if (!inv) {
+        WM_TRY(getrs_grouped(ctx, prec, n, nr, A, n, (int64_t)n * n, perm, n, (double2 *)V, strideV, its, fs,
+                             ctx->stream, max_w > 0 ? max_w : 8));
+        return check_device_error(ctx, ctx->stream);
     }
-    WM_TRY(getrs_grouped(ctx, prec, n, nr, A, n, (int64_t)n * n, perm, n, (double2 *)V, strideV,
-                         std::vector<int>(items, items + nitems), std::vector<int>(fac, fac + nitems), ctx->stream,
-                         dinv, inv ? &slot : nullptr, max_w > 0 ? max_w : kGroupCols));
-    return check_device_error(ctx, ctx->stream);
+    // the preconditioner's solves, on a scaled copy of the factors
+    std::vector<int> slot(nfac);
+    for (int f = 0; f < nfac; ++f) slot[f] = f;
+    WM_TRY(ctx->ws_dinv.ensure(precond_bytes(n, nfac)));
+    double2 *dinv = (double2 *)ctx->ws_dinv.ptr, *copy = nullptr;
+    WM_HIP_TRY(hipMalloc(&copy, (size_t)nfac * n * n * sizeof(double2)));
+    int rc = precond_prepare(ctx, prec, n, A, n, (int64_t)n * n, slot, copy, dinv, ctx->stream);
+    if (rc == WM_OK)
+        rc = precond_solve(ctx, n, nr, copy, n, (int64_t)n * n, perm, n, dinv, slot, (double2 *)V, strideV, its, fs,
+                           ctx->stream);
+    if (rc == WM_OK) rc = check_device_error(ctx, ctx->stream);
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(copy);
+    return rc;
 }
 
 // Internal test hook (not part of include/wiremom.h): solves A^H X = B with the

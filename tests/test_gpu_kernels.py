@@ -1,5 +1,7 @@
 """Single kernels of the library at the sizes where their tilings and splits can
 go wrong, against LAPACK (scipy / the oracle) or plain numpy."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -130,3 +132,46 @@ def test_lookahead_matches_one_stream(wm, ctx, prec, n, batch):
     finally:
         ctx.set_graphs(True)
     assert np.array_equal(got[1], ref[1]) and np.array_equal(got[0], ref[0])
+
+
+@pytest.mark.parametrize("n", [64, 128, 192, 1024])
+def test_preconditioner_solve_widths(wm, ctx, n):
+    """The preconditioner's solves at every way their products are formed (up to
+    4, up to 8 and up to 16 columns, then a second member), from one row block
+    up.  Diagonally dominant matrices: 1e-12 of numpy's solution; a column has
+    the same bits in every width; a column of NaN and one of infinities leave
+    their neighbours alone."""
+    L = wm.lib()
+    L.wmx_getrs_grouped.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_void_p,
+                                    C.c_void_p, C.c_int64, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int]
+    rng = np.random.RandomState(n)
+    A = rng.randn(1, n, n) + 1j * rng.randn(1, n, n) + 4 * n ** 0.5 * np.eye(n)
+    V = rng.randn(17, n) + 1j * rng.randn(17, n)
+    dev, piv, info = wm.getrf_batched(ctx, A, "f64")
+    assert not info.any()
+
+    def solve(V, cols):
+        Vd = wm.DeviceArray(ctx, np.ascontiguousarray(V))
+        it, fac = np.array(cols, np.int32), np.zeros(len(cols), np.int32)
+        assert L.wmx_getrs_grouped(ctx.h, wm.PREC_F64, n, 1, dev.ptr, 1, piv.ptr, Vd.ptr, n, len(it),
+                                   it.ctypes.data, fac.ctypes.data, 1, 0) == 0
+        out = Vd.download()
+        Vd.free()
+        return out
+
+    ref = solve(V, range(17))
+    x = np.linalg.solve(A[0], V.T).T
+    assert np.abs(ref - x).max() <= 1e-12 * np.abs(x).max()
+    for w in (1, 3, 4, 5, 8, 9, 16):
+        got = solve(V, range(w))
+        assert np.array_equal(got[:w].view(np.uint64), ref[:w].view(np.uint64)), w
+        assert np.array_equal(got[w:].view(np.uint64), V[w:].view(np.uint64)), w
+    for w in (4, 8, 16):
+        bad = V.copy()
+        bad[0, n // 2] = np.nan
+        bad[w - 1, 0] = np.inf
+        got = solve(bad, range(w))
+        assert np.array_equal(got[1:w - 1].view(np.uint64), ref[1:w - 1].view(np.uint64)), w
+        assert not np.isfinite(got[0]).all() and not np.isfinite(got[w - 1]).all()
+    dev.free()
+    piv.free()

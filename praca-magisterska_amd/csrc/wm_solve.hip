@@ -6,9 +6,9 @@
 //
 // Each triangular solve is one launch.  Workgroup i owns row block i (64
 // rows).  It subtracts the contributions of the blocks already solved, as
-// each one becomes ready (its values arrive as tagged packets, written by the
-// block's workgroup after its solve), and then solves its diagonal block
-// inside one wave with lane broadcasts.  A workgroup only ever waits on
+// each one becomes ready (its values arrive in words that were marked empty
+// before, written by the block's workgroup after its solve), and then solves
+// its diagonal block, a column per wave, with lane broadcasts.  A workgroup only ever waits on
 // blocks owned by workgroups with a smaller id in the same grid, which are
 // dispatched before it, so the chain always makes progress; every wait is
 // bounded.  Arithmetic is FP64; complex64 factors are widened on load.
@@ -16,6 +16,7 @@
 #include <cfloat>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "wm_cplx.h"
@@ -74,24 +75,6 @@ __global__ __launch_bounds__(256) void k_perm(const int *ipiv, int64_t strideP, 
     if (t < n) perm[(size_t)b * strideQ + t] = row;
 }
 
-struct TrsvArgs {
-    const void *A;
-    int lda;
-    int64_t strideA;
-    int n, nrhs;
-    const int *perm;
-    int64_t strideQ;
-    const double2 *Bin;   // lower solve: right-hand sides (gathered through perm), per launch member
-    int ldb;
-    int64_t strideB;
-    double2 *Y;           // output (lower: y, upper: x in place of y)
-    uint64_t *pkt;        // solved values as tagged packets: per member [block][rhs][row][4 words]
-    int epoch;            // packet tag of this launch
-    int *err;
-    const int *bidx;      // launch member -> matrix index of B and Y (null: identity)
-    const int *aidx;      // launch member -> matrix index of the factors and permutation (null: as bidx)
-};
-
 // Packed entries of one 64 x 64 triangle with its diagonal.
 constexpr int kPack = TB * (TB + 1) / 2;
 
@@ -103,13 +86,6 @@ __device__ inline double bcast(double v, int lane)  // value of `lane` to the wh
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// The double whose low and high words lanes `l` and `l + 1` hold, to the whole wave.
-__device__ inline double word_pair(uint32_t w, int l)
-{
-    const unsigned lo = __builtin_amdgcn_readlane(w, l), hi = __builtin_amdgcn_readlane(w, l + 1);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 // Packed index of element (i, j) of the 64 x 64 diagonal block, column by
 // column (so the lanes of a wave, one row each, read consecutive entries of
 // a column: no LDS bank conflicts): strictly lower part for L (i > j), upper
@@ -117,176 +93,349 @@ __device__ inline double word_pair(uint32_t w, int l)
 __device__ inline int dl_idx(int i, int j) { return j * (2 * TB - 1 - j) / 2 + (i - j - 1); }
 __device__ inline int du_idx(int i, int j) { return j * (j + 1) / 2 + i; }
 
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// Right-hand sides in one pass of a triangular solve: kPsW per launch member
+// (columns of the matrix products), kPassCols per matrix.
+constexpr int kPsW = 16;
+constexpr int kPassCols = 32;
+constexpr int kPsPoll = 4;  // polling waves
+constexpr uint64_t kPsEmpty = 0x7ff8b10c5e7afe55ull;
+
+// Values of a pass are kept as [item][block][column][re, im][TB].
+struct TrsvArgs {
+    const void *A;
+    int lda;
+    int64_t strideA;
+    int n;
+    int ncols;         // columns per item
+    int chunks;        // launch members per item: member m has columns m % chunks * cw ... of item m / chunks
+    int cw;
+    const int *bidx;   // item -> matrix (null: identity)
+    const int *aidx;   // item -> factors (null: as bidx)
+    const int *width;  // SCALED: item -> its columns in use
+    const double2 *dinv;  // SCALED: inverted diagonal blocks
+    const int *slot;      // SCALED: item -> its factors' blocks in dinv
+    uint64_t *in;      // right-hand sides; the lower solve leaves them marked empty, for the upper solve's values
+    uint64_t *pub;     // solved values
+    int *err;
+};
+
 // Triangular solve, one launch.  Workgroup (member, g) owns row block bi of
 // that launch member (lower: g, upper: nblk-1-g); lower solves L y = P b,
-// upper solves U x = y in place, and also publishes each solved value as four
-// tagged packets for the later blocks.  The grid is (members, blocks), so
-// workgroup ids run over the members first: the resident workgroups hold the
-// leading blocks of every member and all members' chains advance together.
-// Waits only on blocks of workgroups with smaller ids (dispatched earlier).
+// upper solves U x = y.  The grid is (members, blocks), so workgroup ids run
+// over the members first: the resident workgroups hold the leading blocks of
+// every member and all members' chains advance together.  Waits only on blocks
+// of workgroups with smaller ids (dispatched earlier).
+//
+// Four waves (wave w: rows 16 w ..) subtract the products with the solved blocks
+// as their values arrive, on the matrix cores; a right-hand side is a column of
+// the products, so its values do not depend on its neighbours, and the 4x4x4
+// form (up to 8 columns) rounds like the 16x16x4 one.  Then all eight waves
+// substitute through the diagonal block, a column each.  Values of a block
+// travel as plain 8-byte words: they are marked empty (kPsEmpty, a NaN pattern
+// no arithmetic produces) before the launch, and a reader polls its words until
+// they hold something else.  The other four waves do the polling: a wave's
+// loads complete in order, so a poll behind the next block's factor entries
+// would wait for HBM in every step.
 //
 // TRANS solves with the conjugate transposes of the factors (A^H = U^H L^H P):
 // the lower pass takes U^H (lower, non-unit diagonal conj(u_ii)) on the
-// right-hand sides as staged (no gather), the upper pass L^H (upper, unit
-// diagonal) in place; element (i, j) of the triangle is conj(A(j, i)).  The
-// caller scatters the result through the permutation (x = P^T w).
-template <typename T, int NR, bool UPPER, bool TRANS>
-__global__ __launch_bounds__(256) void k_trsv(TrsvArgs a, int r_off)
+// right-hand sides as they are (no gather), the upper pass L^H (upper, unit
+// diagonal); element (i, j) of the triangle is conj(A(j, i)).  The results
+// leave through the permutation (x = P^T w).
+//
+// SCALED solves with factors whose row blocks are multiplied by the inverses of
+// their diagonal blocks (k_scale_blocks): c = D_ii^-1 b at the start instead of
+// the substitution, and three real products per complex product instead of
+// four.  For preconditioners.
+//
+// What bounds it: the chain of n / 64 blocks.  SCALED: 2.0 us each with up to 4
+// columns and 3.6 us with 16 (0.5 us for the values to cross, the rest the
+// product of the newest block: 48 4x4x4 products per wave for 4 columns, 96 for
+// 8, 48 16x16x4, at four times the cycles each, above).  Per triangle at N =
+// 8192, against substitution by inverted diagonal blocks on the vector units,
+// four columns per member:
+//   1 factor, 3 columns    258 us instead of 1004
+//   2 factors, 16 columns  466 us instead of 1245 (factors read once, not 4 times)
+//   N = 512, 3 columns      18 us instead of 65
+// One polling wave instead of four: 470 us for 1 x 3 before the 4x4x4 form, 355
+// with four; real and imaginary words apart (whole lines per store): 470 us
+// instead of 628 for 2 x 16.
+// Not SCALED: 4.4 us a block lower and 8.7 us upper with 8 columns in two matrices of
+// N = 8192, of which the substitution is about 2.3 and 4 us (76 and 110 cycles a
+// step) and the product 1; 843 us per triangle instead of 1930 with the poll, the
+// products (values broadcast by lane reads) and a column per wave substitution in
+// the same four waves, eight columns at most per pass.
+template <typename T, bool UPPER, bool TRANS, bool SCALED>
+__global__ __launch_bounds__(256 + 64 * kPsPoll) void k_trsv(TrsvArgs a)
 {
-    // no contraction: a right-hand side's arithmetic is the same in every
-    // instantiation (NR), so grouping columns never changes their values
+    // no contraction: a right-hand side's arithmetic is the same in every form
 #pragma clang fp contract(off)
     using V = typename CT<T>::V;
     constexpr bool UNIT = TRANS ? UPPER : !UPPER;  // unit diagonal (L or L^H)
-    // element (i, j) of the triangle being solved
-    auto elem = [&](const V *A, int i, int j) -> double2 {
+    const int item = blockIdx.x / a.chunks, c0 = blockIdx.x % a.chunks * a.cw;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nblk = a.n / TB;
+    const int bi = UPPER ? nblk - 1 - (int)blockIdx.y : (int)blockIdx.y, r0 = bi * TB;
+    const int w = SCALED ? a.width[item] : min(a.cw, a.ncols - c0);
+    const int fb = a.aidx ? a.aidx[item] : a.bidx ? a.bidx[item] : item;
+    const V *A = (const V *)a.A + (size_t)fb * a.strideA;
+    const double2 *D = a.dinv;
+    if (SCALED) D += (((size_t)a.slot[item] * 2 + (UPPER ? 1 : 0)) * nblk + bi) * TB * TB;
+    // this member's columns of block q of the item's values
+    auto cols_of = [&](uint64_t *v, int q) { return v + (((size_t)item * nblk + q) * a.ncols + c0) * 2 * TB; };
+    auto elem = [&](int i, int j) -> double2 {  // element (i, j) of the triangle being solved
         if (!TRANS) return ld2<T>(A + i + (size_t)j * a.lda);
         const double2 v = ld2<T>(A + j + (size_t)i * a.lda);
         return make_double2(v.x, -v.y);
     };
-    const int bl = blockIdx.x, tid = threadIdx.x, row = tid & 63;
-    const int b = a.bidx ? a.bidx[bl] : bl;
-    const int fb = a.aidx ? a.aidx[bl] : b;  // factors (and their permutation) of this member
-    const int part = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nblk = a.n / TB;
-    const int bi = UPPER ? nblk - 1 - (int)blockIdx.y : (int)blockIdx.y, r0 = bi * TB;
-    const V *A = (const V *)a.A + (size_t)fb * a.strideA;
-    double2 *Y = a.Y + (size_t)b * a.strideB + (size_t)r_off * a.ldb;
-    uint64_t *pk = a.pkt + (size_t)bl * nblk * NR * 256;
-    const uint32_t tag = (uint32_t)a.epoch;
-    const int nr = a.nrhs - r_off;
-
-    // diagonal block to LDS (independent of other blocks, so before any wait)
-    constexpr int kPad = 1;  // dl_idx(0, 0) is -1
-    __shared__ double2 s_d[kPad + kPack];
-    __shared__ double2 s_rd[TB];
-    for (int e = tid; e < TB * TB; e += 256) {
-        // consecutive threads walk down a column of the stored factor
-        const int i = TRANS ? e / TB : e % TB, j = TRANS ? e % TB : e / TB;
-        if (!UPPER && i > j) s_d[kPad + dl_idx(i, j)] = elem(A, r0 + i, r0 + j);
-        if (UPPER && i < j) s_d[kPad + du_idx(i, j)] = elem(A, r0 + i, r0 + j);
-        if (!UNIT && i == j) {
-            const double2 u = elem(A, r0 + i, r0 + j);
-            s_rd[i] = crecip(u.x, u.y);
-        }
-    }
-
-    double2 acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = make_double2(0.0, 0.0);
-    if (part == 0) {
-        const int src = (UPPER || TRANS) ? r0 + row : a.perm[(size_t)fb * a.strideQ + r0 + row];
-        const double2 *in = UPPER ? Y : a.Bin + (size_t)bl * a.strideB + (size_t)r_off * a.ldb;
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-            if (r < nr) acc[r] = in[src + (size_t)r * a.ldb];
-    }
-
-    // off-diagonal blocks in dependency order, next block prefetched
-    const int nb_off = UPPER ? nblk - 1 - bi : bi;
+    auto put = [](uint64_t *o, double x) {
+        const uint64_t u = (uint64_t)__double_as_longlong(x);
+        __hip_atomic_store(o, u == kPsEmpty ? 0x7ff8000000000000ull : u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const int noff = UPPER ? nblk - 1 - bi : bi;
     auto blk = [&](int q) { return UPPER ? nblk - 1 - q : q; };
-    double2 lcur[16], lnext[16];
-    if (nb_off > 0) {
-        const int c0 = blk(0) * TB + part * 16;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) lcur[c] = elem(A, r0 + row, c0 + c);
-    }
-    for (int q = 0; q < nb_off; ++q) {
-        // The part's 16 solved values of block q: 64 packets per right-hand
-        // side, one per lane, polled until the block's workgroup has tagged
-        // them (a value and its readiness in one memory round trip), and all
-        // loaded before the next block's L prefetch.
-        const uint64_t *pq = pk + (size_t)blk(q) * NR * 256 + part * 64 + row;
-        uint32_t yw[NR];
-        long it = 0;
-        for (;;) {
-            bool got = true;
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                yw[r] = 0u;
-                if (r < nr) {
-                    const uint64_t v = ld_pkt(pq + r * 256);
-                    yw[r] = (uint32_t)v;
-                    got = got && (uint32_t)(v >> 32) == tag;
+    // two buffers: a block's values are staged while the previous ones are read
+    __shared__ double2 s_y[2][kPsW][TB + 1];
+    constexpr int kPad = 1;  // dl_idx(0, 0) is -1
+    __shared__ double2 s_d[SCALED ? 1 : kPad + kPack];
+    __shared__ double2 s_rd[SCALED ? 1 : TB];
+
+    if (wave >= 4) {
+        if (!SCALED) {
+            for (int e = tid - 256; e < TB * TB; e += 64 * kPsPoll) {
+                // consecutive threads walk down a column of the stored factor
+                const int i = TRANS ? e / TB : e % TB, j = TRANS ? e % TB : e / TB;
+                if (!UPPER && i > j) s_d[kPad + dl_idx(i, j)] = elem(r0 + i, r0 + j);
+                if (UPPER && i < j) s_d[kPad + du_idx(i, j)] = elem(r0 + i, r0 + j);
+                if (!UNIT && i == j) {
+                    const double2 u = elem(r0 + i, r0 + j);
+                    s_rd[i] = crecip(u.x, u.y);
                 }
             }
-            if (__all(got)) break;
-            if (spin_give_up(it, a.err)) break;
+        } else {
+            __syncthreads();  // the right-hand sides are staged
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (q + 1 < nb_off) {
-            const int c1 = blk(q + 1) * TB + part * 16;
+        // the values of the other blocks: lane = row, wave 4 + j has columns j, j + kPsPoll, ...
+        constexpr int kE = kPsW / kPsPoll;
+        const int j0 = wave - 4;
+        for (int q = 0; q < noff; ++q) {
+            const uint64_t *py = cols_of(a.pub, blk(q)) + j0 * 2 * TB + lane;
+            uint64_t yx[kE], yy[kE];
+            long it = 0;
+            for (;;) {
 #pragma unroll
-            for (int c = 0; c < 16; ++c) lnext[c] = elem(A, r0 + row, c1 + c);
+                for (int e = 0; e < kE; ++e) {
+                    yx[e] = yy[e] = 0;
+                    if (j0 + kPsPoll * e < w) {
+                        yx[e] = ld_pkt(py + 2 * kPsPoll * TB * e);
+                        yy[e] = ld_pkt(py + 2 * kPsPoll * TB * e + TB);
+                    }
+                }
+                bool got = true;
+#pragma unroll
+                for (int e = 0; e < kE; ++e) got = got & (yx[e] != kPsEmpty) & (yy[e] != kPsEmpty);
+                if (__all(got)) break;
+                if (spin_give_up(it, a.err)) break;
+            }
+#pragma unroll
+            for (int e = 0; e < kE; ++e)
+                if (j0 + kPsPoll * e < w)
+                    s_y[(q + 1) & 1][j0 + kPsPoll * e][lane] = make_double2(
+                        __longlong_as_double((long long)yx[e]), __longlong_as_double((long long)yy[e]));
+            __syncthreads();
         }
-        __builtin_amdgcn_sched_barrier(0);
+        if (SCALED) return;
+    } else {
+        const int row = wave * 16 + lane % 16, kq = lane / 16, rhs = lane % 16;
+        V lcur[16], lnext[16];  // this lane's factor entries: row, columns kq + 4 t of a block
+        auto load_block = [&](int q, V *l) {
+            const size_t step = TRANS ? 1 : (size_t)a.lda;
+            const V *p = TRANS ? A + (size_t)(r0 + row) * a.lda + q * TB + kq
+                               : A + r0 + row + (size_t)(q * TB + kq) * a.lda;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
+            for (int t = 0; t < 16; ++t) l[t] = p[4 * t * step];
+        };
+        // P + i R: the products of a block; SCALED: P, Q = re re, im im and R = (re + im)(re + im)
+        v4d P, Q, R;
+        auto product = [&](const V *l, int buf) {
+            P = Q = R = v4d{0, 0, 0, 0};
+            auto steps = [&](auto ng_c, auto mul) {
+                constexpr int NG = decltype(ng_c)::value;
 #pragma unroll
-            for (int r = 0; r < NR; ++r)
-                if (r < nr) cfms(acc[r], lcur[c], make_double2(word_pair(yw[r], 4 * c), word_pair(yw[r], 4 * c + 2)));
-        }
+                for (int t = 0; t < 16; ++t) {
+                    const double lx = l[t].x, ly = TRANS ? -l[t].y : l[t].y;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) lcur[c] = lnext[c];
-    }
+                    for (int g = 0; g < NG; ++g) mul(t, g, lx, ly);
+                }
+            };
+            auto small = [&](int t, int g, double lx, double ly) {
+                const double2 y = s_y[buf][4 * g + lane % 4][4 * t + kq];
+                if (SCALED) {
+                    P[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, lx, P[g], 0, 0, 0);
+                    Q[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, ly, Q[g], 0, 0, 0);
+                    R[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x + y.y, lx + ly, R[g], 0, 0, 0);
+                } else {
+                    P[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, lx, P[g], 0, 0, 0);
+                    R[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, lx, R[g], 0, 0, 0);
+                    P[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(-y.y, ly, P[g], 0, 0, 0);
+                    R[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, ly, R[g], 0, 0, 0);
+                }
+            };
+            if (w <= 4) {
+                steps(std::integral_constant<int, 1>{}, small);
+                return;
+            }
+            if (w <= 8) {
+                steps(std::integral_constant<int, 2>{}, small);
+                return;
+            }
+            steps(std::integral_constant<int, 1>{}, [&](int t, int, double lx, double ly) {
+                const double2 y = s_y[buf][rhs][4 * t + kq];
+                if (SCALED) {
+                    P = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, lx, P, 0, 0, 0);
+                    Q = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, ly, Q, 0, 0, 0);
+                    R = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x + y.y, lx + ly, R, 0, 0, 0);
+                } else {
+                    P = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, lx, P, 0, 0, 0);
+                    R = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, lx, R, 0, 0, 0);
+                    P = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.y, ly, P, 0, 0, 0);
+                    R = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, ly, R, 0, 0, 0);
+                }
+            });
+        };
 
-    // The four parts' sums meet in LDS; wave p then solves the right-hand
-    // sides p, p + 4, ... (each sum in the order part 0 + 1 + 2 + 3, so a
-    // value does not depend on NR or on which wave solves it).
-    __shared__ double2 s_acc[4][TB][NR];
+        // this lane: row `row`, columns kq + 4 v
+        double cr[4], ci[4];
+        uint64_t *in = cols_of(a.in, bi);
+        if (SCALED) {  // c = D^-1 b
 #pragma unroll
-    for (int r = 0; r < NR; ++r) s_acc[part][row][r] = acc[r];
-    __syncthreads();
-    constexpr int RW = (NR + 3) / 4;  // right-hand sides per wave
-    if (part < NR) {
-        double2 x[RW];
+            for (int e = 0; e < 4; ++e) {
+                uint64_t *p = in + (wave + 4 * e) * 2 * TB + lane;
+                s_y[0][wave + 4 * e][lane] =
+                    make_double2(__longlong_as_double((long long)p[0]), __longlong_as_double((long long)p[TB]));
+                if (!UPPER) p[0] = p[TB] = kPsEmpty;
+            }
 #pragma unroll
-        for (int k = 0; k < RW; ++k) {
-            const int r = part + 4 * k;
-            x[k] = make_double2(0.0, 0.0);
-            if (r < NR) {
-                x[k] = s_acc[0][row][r];
+            for (int t = 0; t < 16; ++t) {
+                const double2 d = D[row + (size_t)(4 * t + kq) * TB];
+                lcur[t].x = (T)d.x;
+                lcur[t].y = (T)d.y;
+            }
+            __syncthreads();
+            product(lcur, 0);
 #pragma unroll
-                for (int p = 1; p < 4; ++p) { x[k].x += s_acc[p][row][r].x; x[k].y += s_acc[p][row][r].y; }
+            for (int v = 0; v < 4; ++v) {
+                cr[v] = P[v] - Q[v];
+                ci[v] = R[v] - P[v] - Q[v];
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                cr[v] = ci[v] = 0.0;
+                if (kq + 4 * v < w) {
+                    uint64_t *p = in + (kq + 4 * v) * 2 * TB + row;
+                    cr[v] = __longlong_as_double((long long)p[0]);
+                    ci[v] = __longlong_as_double((long long)p[TB]);
+                    if (!UPPER) p[0] = p[TB] = kPsEmpty;
+                }
             }
         }
-        // The substitution is the launch's critical path: unrolled, and without
-        // branches.  A step broadcasts row j's value (every lane scales it by the
-        // diagonal's reciprocal), and the rows that it reaches take the
-        // difference by selection: the others read some entry of the packed
-        // block and drop the product, so a step's LDS reads need no mask and
-        // are issued ahead of it.
+        auto subtract = [&]() {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                cr[v] -= SCALED ? P[v] - Q[v] : P[v];
+                ci[v] -= SCALED ? R[v] - P[v] - Q[v] : R[v];
+            }
+        };
+        // Two blocks per turn, loads without a condition (past the end: the last
+        // block once more), so that a product's wait counts leave the next block's
+        // loads in flight; an odd block goes first.
+        int q = noff & 1;
+        if (q) {
+            load_block(blk(0), lnext);
+            load_block(blk(min(1, noff - 1)), lcur);
+            __syncthreads();
+            product(lnext, 1);
+            subtract();
+        } else if (noff > 0) {
+            load_block(blk(0), lcur);
+        }
+        for (; q < noff; q += 2) {
+            load_block(blk(q + 1), lnext);
+            __syncthreads();
+            product(lcur, (q + 1) & 1);
+            subtract();
+            load_block(blk(min(q + 2, noff - 1)), lcur);
+            __syncthreads();
+            product(lnext, q & 1);
+            subtract();
+        }
+        if (SCALED) {
+            uint64_t *o = cols_of(a.pub, bi) + row;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (kq + 4 * v < w) {
+                    put(o + (kq + 4 * v) * 2 * TB, cr[v]);
+                    put(o + (kq + 4 * v) * 2 * TB + TB, ci[v]);
+                }
+            return;
+        }
+        // into the buffer that no product reads any more
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s_y[(noff + 1) & 1][kq + 4 * v][row] = make_double2(cr[v], ci[v]);
+    }
+    if (SCALED) return;
+
+    // Diagonal block: lane = row, wave v has columns v and v + 8.  The
+    // substitution is the launch's critical path: unrolled, and without
+    // branches.  A step broadcasts row j's value (every lane scales it by the
+    // diagonal's reciprocal), and the rows that it reaches take the difference
+    // by selection: the others read some entry of the packed block and drop
+    // the product, so a step's LDS reads need no mask and are issued ahead.
+    // Solving four rows' own triangle in every lane to save broadcasts costs
+    // more instructions than the broadcasts: 1103 us per triangle of two
+    // matrices with 8 columns at N = 8192 instead of 896.
+    __syncthreads();
+    auto scaled = [](double2 c, double2 r) { return make_double2(c.x * r.x - c.y * r.y, c.x * r.y + c.y * r.x); };
+    auto substitute = [&](auto rw_c) {
+        constexpr int RW = decltype(rw_c)::value;
+        double2 x[RW];
+#pragma unroll
+        for (int k = 0; k < RW; ++k) x[k] = s_y[(noff + 1) & 1][wave + 8 * k][lane];
 #pragma unroll
         for (int jj = 0; jj < TB; ++jj) {
             const int j = UPPER ? TB - 1 - jj : jj;
-            const double2 l = s_d[kPad + (UPPER ? du_idx(row, j) : dl_idx(row, j))];
+            const double2 l = s_d[kPad + (UPPER ? du_idx(lane, j) : dl_idx(lane, j))];
             const double2 ri = UNIT ? make_double2(1.0, 0.0) : s_rd[j];
 #pragma unroll
             for (int k = 0; k < RW; ++k) {
-                if (part + 4 * k >= NR) break;
                 double2 xj = make_double2(bcast(x[k].x, j), bcast(x[k].y, j));
-                if (!UNIT) xj = make_double2(xj.x * ri.x - xj.y * ri.y, xj.x * ri.y + xj.y * ri.x);
+                if (!UNIT) xj = scaled(xj, ri);
                 double2 v = x[k];
                 cfms(v, l, xj);
-                const bool below = UPPER ? row < j : row > j;
-                x[k].x = below ? v.x : !UNIT && row == j ? xj.x : x[k].x;
-                x[k].y = below ? v.y : !UNIT && row == j ? xj.y : x[k].y;
+                const bool below = UPPER ? lane < j : lane > j;
+                x[k].x = below ? v.x : x[k].x;
+                x[k].y = below ? v.y : x[k].y;
             }
+        }
+        if (!UNIT) {  // the rows' own values, as their steps scaled them
+#pragma unroll
+            for (int k = 0; k < RW; ++k) x[k] = scaled(x[k], s_rd[lane]);
         }
 #pragma unroll
         for (int k = 0; k < RW; ++k) {
-            const int r = part + 4 * k;
-            if (r < nr) {
-                Y[(r0 + row) + (size_t)r * a.ldb] = x[k];
-                uint64_t *pw = pk + ((size_t)bi * NR + r) * 256 + row * 4;
-                const uint64_t xb = (uint64_t)__double_as_longlong(x[k].x), yb = (uint64_t)__double_as_longlong(x[k].y);
-                put_pkt(pw, tag, (uint32_t)xb);
-                put_pkt(pw + 1, tag, (uint32_t)(xb >> 32));
-                put_pkt(pw + 2, tag, (uint32_t)yb);
-                put_pkt(pw + 3, tag, (uint32_t)(yb >> 32));
-            }
+            const int r = wave + 8 * k;
+            if (r >= w) break;
+            uint64_t *o = cols_of(a.pub, bi) + r * 2 * TB + lane;
+            put(o, x[k].x);
+            put(o + TB, x[k].y);
         }
-    }
+    };
+    if (w > 8) substitute(std::integral_constant<int, 2>{});
+    else if (wave < w) substitute(std::integral_constant<int, 1>{});
 }
 
 // Partial products P[split][row][r] = sum_{j in split} Z[row][j] X[j][r].
@@ -392,14 +541,6 @@ __global__ void k_resid_final(const double2 *P, int nsplit, int n, int nrhs, con
     }
 }
 
-template <typename T, int NR, bool TRANS>
-void launch_trsv(const TrsvArgs &a, int batch, int r_off, bool upper, hipStream_t s)
-{
-    const dim3 grid(batch, a.n / TB);
-    if (upper) hipLaunchKernelGGL((k_trsv<T, NR, true, TRANS>), grid, dim3(256), 0, s, a, r_off);
-    else hipLaunchKernelGGL((k_trsv<T, NR, false, TRANS>), grid, dim3(256), 0, s, a, r_off);
-}
-
 // Inverses of the 64 x 64 diagonal blocks of LU factors, FP64 arithmetic:
 // blockIdx = (block, triangle 0 = L (unit lower) / 1 = U, slot); slot z
 // takes the factors of index fidx[z].  Lane j solves for column j of the
@@ -446,15 +587,13 @@ __global__ __launch_bounds__(64) void k_diag_inv(const void *F, int lda, int64_t
     }
 }
 
-typedef double v4d __attribute__((ext_vector_type(4)));
-
 // Preconditioner factors: every row block of L and U times the inverse of its
 // diagonal block, L' = diag(L_ii)^-1 L and U' = diag(U_ii)^-1 U, so that a solve
 // needs no work on the diagonal between one block's values and the next's.
 // blockIdx = (column block, row block, slot); row block bi of factor fidx[z],
 // column block cb (left of the diagonal: L, right of it: U) is multiplied by
 // its inverse on the matrix cores (three real products per complex product,
-// lanes as in k_psolve) and written to dst, which may be the factors themselves.
+// lanes as in k_trsv) and written to dst, which may be the factors themselves.
 template <typename T>
 __global__ __launch_bounds__(256) void k_scale_blocks(const void *F, double2 *dst, int lda, int64_t strideF,
                                                       const int *fidx, int nblk, const double2 *Dinv)
@@ -495,274 +634,49 @@ __global__ __launch_bounds__(256) void k_scale_blocks(const void *F, double2 *ds
                 make_double2(P[c][v] - Q[c][v], S[c][v] - P[c][v] - Q[c][v]);
 }
 
-// Preconditioner solve L' y = diag(L_ii)^-1 P b (UPPER: U' x = diag(U_ii)^-1 y) for up
-// to kPsW right-hand sides per launch member, one launch.  Workgroup (member,
-// g) owns row block bi (lower: g, upper: nblk-1-g): c = D_ii^-1 b, then c minus
-// the products with the solved blocks as their values arrive, on the matrix
-// cores (wave w < 4: rows 16 w ..; three real products per complex product; a
-// right-hand side is a column of the products, so its values do not depend on
-// its neighbours).  Values of a block travel as plain 8-byte words: a member's
-// blocks are filled with kPsEmpty, a NaN pattern no arithmetic produces, before
-// the launch, and a reader polls its words until they hold something else.
-// Four more waves do the polling: a wave's loads complete in order, so a poll
-// behind the next block's factor entries would wait for HBM in every step.
-// Waits only on blocks of workgroups with smaller ids (dispatched earlier).
-//
-// What bounds it: the chain of n / 64 blocks, 2.0 us each with up to 4 columns and
-// 3.6 us with 16 (0.5 us for the values to cross, the rest the product of the
-// newest block: 48 4x4x4 products per wave for 4 columns, 96 for 8, 48 16x16x4,
-// at four times the cycles each, above).  The 4x4x4 form spends nothing on
-// columns that are not there and rounds like the 16x16x4 one: a column has the
-// same bits in every width.  Per triangle at N = 8192, against substitution by
-// inverted diagonal blocks on the vector units, four columns per member:
-//   1 factor, 3 columns    258 us instead of 1004
-//   2 factors, 16 columns  466 us instead of 1245 (factors read once, not 4 times)
-//   N = 512, 3 columns      18 us instead of 65
-// One polling wave instead of four: 470 us for 1 x 3 before the 4x4x4 form, 355
-// with four; real and imaginary words apart (whole lines per store): 470 us
-// instead of 628 for 2 x 16.
-constexpr int kPsW = 16;
-constexpr int kPsPoll = 4;
-constexpr uint64_t kPsEmpty = 0x7ff8b10c5e7afe55ull;
-
-struct PsolveArgs {
-    const double2 *F;       // scaled factors
-    int lda;
-    int64_t strideF;
-    int n;
-    const double2 *dinv;
-    const double *in;       // right-hand sides, [member][block][kPsW][re, im][TB]
-    uint64_t *pub;          // solved values, the same layout
-    const int *fac, *slot, *width;  // per member: factor, its slot in dinv, its right-hand sides
-    int *err;
-};
-
-template <bool UPPER>
-__global__ __launch_bounds__(256 + 64 * kPsPoll) void k_psolve(PsolveArgs a)
-{
-    const int bl = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nblk = a.n / TB;
-    const int bi = UPPER ? nblk - 1 - (int)blockIdx.y : (int)blockIdx.y, r0 = bi * TB;
-    const int w = a.width[bl];
-    uint64_t *pub = a.pub + (size_t)bl * a.n * kPsW * 2;
-    const int noff = UPPER ? nblk - 1 - bi : bi;
-    auto blk = [&](int q) { return UPPER ? nblk - 1 - q : q; };
-    // two buffers: a block's values are staged while the previous ones are read
-    __shared__ double2 s_y[2][kPsW][TB + 1];
-
-    if (wave >= 4) {  // the values of the other blocks: lane = row, wave 4 + j has columns j, j + kPsPoll, ...
-        constexpr int kE = kPsW / kPsPoll;
-        const int j0 = wave - 4;
-        __syncthreads();
-        for (int q = 0; q < noff; ++q) {
-            const uint64_t *py = pub + (((size_t)blk(q) * kPsW + j0) * 2) * TB + lane;
-            uint64_t yx[kE], yy[kE];
-            long it = 0;
-            for (;;) {
-#pragma unroll
-                for (int e = 0; e < kE; ++e) {
-                    yx[e] = yy[e] = 0;
-                    if (j0 + kPsPoll * e < w) {
-                        yx[e] = ld_pkt(py + 2 * kPsPoll * TB * e);
-                        yy[e] = ld_pkt(py + 2 * kPsPoll * TB * e + TB);
-                    }
-                }
-                bool got = true;
-#pragma unroll
-                for (int e = 0; e < kE; ++e) got = got & (yx[e] != kPsEmpty) & (yy[e] != kPsEmpty);
-                if (__all(got)) break;
-                if (spin_give_up(it, a.err)) break;
-            }
-#pragma unroll
-            for (int e = 0; e < kE; ++e)
-                if (j0 + kPsPoll * e < w)
-                    s_y[(q + 1) & 1][j0 + kPsPoll * e][lane] = make_double2(
-                        __longlong_as_double((long long)yx[e]), __longlong_as_double((long long)yy[e]));
-            __syncthreads();
-        }
-        return;
-    }
-
-    const double2 *A = a.F + (size_t)a.fac[bl] * a.strideF;
-    const double2 *D = a.dinv + (((size_t)a.slot[bl] * 2 + (UPPER ? 1 : 0)) * nblk + bi) * TB * TB;
-    const int row = wave * 16 + lane % 16, kq = lane / 16, rhs = lane % 16;
-    double2 lcur[16], lnext[16];  // this lane's factor entries: row, columns kq + 4 t of a block
-    auto load_block = [&](int q, double2 *l) {
-        const double2 *p = A + r0 + row + (size_t)(q * TB + kq) * a.lda;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) l[t] = p[(size_t)(4 * t) * a.lda];
-    };
-    v4d P, Q, S;
-    auto product = [&](const double2 *l, int buf) {
-        P = Q = S = v4d{0, 0, 0, 0};
-        if (w <= 4) {
-#pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const double2 y = s_y[buf][lane % 4][4 * t + kq];
-                P[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, l[t].x, P[0], 0, 0, 0);
-                Q[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, l[t].y, Q[0], 0, 0, 0);
-                S[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x + y.y, l[t].x + l[t].y, S[0], 0, 0, 0);
-            }
-            return;
-        }
-        if (w <= 8) {
-#pragma unroll
-            for (int t = 0; t < 16; ++t) {
-#pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const double2 y = s_y[buf][4 * g + lane % 4][4 * t + kq];
-                    P[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x, l[t].x, P[g], 0, 0, 0);
-                    Q[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.y, l[t].y, Q[g], 0, 0, 0);
-                    S[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(y.x + y.y, l[t].x + l[t].y, S[g], 0, 0, 0);
-                }
-            }
-            return;
-        }
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            const double2 y = s_y[buf][rhs][4 * t + kq];
-            P = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, l[t].x, P, 0, 0, 0);
-            Q = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, l[t].y, Q, 0, 0, 0);
-            S = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x + y.y, l[t].x + l[t].y, S, 0, 0, 0);
-        }
-    };
-
-    // c = D^-1 b (this lane: row `row`, right-hand sides kq + 4 v)
-    const double *in = a.in + (((size_t)bl * nblk + bi) * kPsW + wave) * 2 * TB + lane;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s_y[0][wave + 4 * e][lane] = make_double2(in[8 * TB * e], in[8 * TB * e + TB]);
-#pragma unroll
-    for (int t = 0; t < 16; ++t) lcur[t] = D[row + (size_t)(4 * t + kq) * TB];
-    __syncthreads();
-    product(lcur, 0);
-    double cr[4], ci[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        cr[v] = P[v] - Q[v];
-        ci[v] = S[v] - P[v] - Q[v];
-    }
-    auto subtract = [&]() {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            cr[v] -= P[v] - Q[v];
-            ci[v] -= S[v] - P[v] - Q[v];
-        }
-    };
-    // Two blocks per turn, loads without a condition (past the end: the last
-    // block once more), so that a product's wait counts leave the next block's
-    // loads in flight; an odd block goes first.
-    int q = noff & 1;
-    if (q) {
-        load_block(blk(0), lnext);
-        load_block(blk(min(1, noff - 1)), lcur);
-        __syncthreads();
-        product(lnext, 1);
-        subtract();
-    } else if (noff > 0) {
-        load_block(blk(0), lcur);
-    }
-    for (; q < noff; q += 2) {
-        load_block(blk(q + 1), lnext);
-        __syncthreads();
-        product(lcur, (q + 1) & 1);
-        subtract();
-        load_block(blk(min(q + 2, noff - 1)), lcur);
-        __syncthreads();
-        product(lnext, q & 1);
-        subtract();
-    }
-    auto word = [](double x) {
-        const uint64_t u = (uint64_t)__double_as_longlong(x);
-        return u == kPsEmpty ? 0x7ff8000000000000ull : u;
-    };
-    uint64_t *o = pub + (size_t)bi * kPsW * 2 * TB + row;
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-        if (kq + 4 * v < w) {
-            uint64_t *ov = o + (kq + 4 * v) * 2 * TB;
-            __hip_atomic_store(ov, word(cr[v]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(ov + TB, word(ci[v]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-}
-
-// Right-hand sides of a preconditioner solve, [member][block][kPsW][re, im][TB]:
-// rows through perm of column cols[member * kPsW + j] of V (element offset; -1:
-// zero), and both triangles' values marked empty (pub, pub + members * n *
-// kPsW complex words).
-__global__ void k_ps_gather(const double2 *V, int n, const int64_t *cols, const int *fac, const int *perm,
-                            int64_t strideQ, double *in, uint64_t *pub, int members)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
-    if (t >= n * kPsW) return;
-    const int row = t / (TB * kPsW) * TB + t % TB, j = t / TB % kPsW;
-    const int64_t c = cols[(size_t)m * kPsW + j];
-    const size_t o = (size_t)m * n * kPsW * 2 + (size_t)(t / TB) * 2 * TB + t % TB;
-    const double2 v = c >= 0 ? V[c + perm[(size_t)fac[m] * strideQ + row]] : make_double2(0.0, 0.0);
-    in[o] = v.x;
-    in[o + TB] = v.y;
-    const size_t half = (size_t)members * n * kPsW * 2;
-    pub[o] = pub[o + TB] = pub[half + o] = pub[half + o + TB] = kPsEmpty;
-}
-
-// The solved columns back to V.
-__global__ void k_ps_scatter(const double *pub, int n, const int64_t *cols, double2 *V)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
-    if (t >= n * kPsW) return;
-    const int row = t / (TB * kPsW) * TB + t % TB, j = t / TB % kPsW;
-    const int64_t c = cols[(size_t)m * kPsW + j];
-    const double *p = pub + (size_t)m * n * kPsW * 2 + (size_t)(t / TB) * 2 * TB + t % TB;
-    if (c >= 0) V[c + row] = make_double2(p[0], p[TB]);
-}
-
-// Right-hand sides handled by one pass starting at r_off: 8, 4, 2 or 1.
+// Right-hand sides handled by one residual pass starting at r_off
 inline int rhs_chunk(int left) { return left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1; }
 
-template <typename T, bool TRANS = false>
-void trsv_dispatch(const TrsvArgs &a, int batch, int r_off, bool upper, hipStream_t s)
+// Right-hand sides of a pass into its layout: columns r_off ... of each item of B
+// (or the columns cols[item * ncols + j], element offsets; -1: zero), rows
+// through perm (or as they are), and the solved values' words marked empty.
+__global__ void k_rhs_in(const double2 *B, int n, int ldb, int64_t strideB, int r_off, int ncols, const int64_t *cols,
+                         const int *perm, int64_t strideQ, const int *bidx, const int *aidx, uint64_t *in,
+                         uint64_t *pub)
 {
-    switch (rhs_chunk(a.nrhs - r_off)) {
-        case 8: launch_trsv<T, 8, TRANS>(a, batch, r_off, upper, s); break;
-        case 4: launch_trsv<T, 4, TRANS>(a, batch, r_off, upper, s); break;
-        case 2: launch_trsv<T, 2, TRANS>(a, batch, r_off, upper, s); break;
-        default: launch_trsv<T, 1, TRANS>(a, batch, r_off, upper, s); break;
-    }
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)n * ncols) return;
+    const int item = blockIdx.y, j = (int)(t / TB % ncols), b = bidx ? bidx[item] : item;
+    const int row = (int)(t / ((int64_t)TB * ncols)) * TB + (int)(t % TB);
+    const int src = perm ? perm[(size_t)(aidx ? aidx[item] : b) * strideQ + row] : row;
+    const int64_t c = cols ? cols[(size_t)item * ncols + j] : (int64_t)b * strideB + (int64_t)(r_off + j) * ldb;
+    const size_t o = ((size_t)item * n * ncols + (size_t)(t / TB) * TB) * 2 + t % TB;
+    const double2 v = c >= 0 ? B[c + src] : make_double2(0.0, 0.0);
+    in[o] = (uint64_t)__double_as_longlong(v.x);
+    in[o + TB] = (uint64_t)__double_as_longlong(v.y);
+    pub[o] = pub[o + TB] = kPsEmpty;
 }
 
-// Bstage[member] = B[matrix] (n x nrhs columns with leading dimension ldb)
-__global__ void k_stage(const double2 *B, int ldb, int64_t strideB, int n, int nrhs, double2 *S, const int *bidx)
+// The solved values back to B, rows through perm (x = P^T w) or as they are.
+__global__ void k_rhs_out(const double *x, int n, int ldb, int64_t strideB, int r_off, int ncols, const int64_t *cols,
+                          const int *perm, int64_t strideQ, const int *bidx, const int *aidx, double2 *B)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, bl = blockIdx.y;
-    const int b = bidx ? bidx[bl] : bl;
-    if (i >= n) return;
-    for (int r = 0; r < nrhs; ++r) S[(size_t)bl * strideB + (size_t)r * ldb + i] = B[(size_t)b * strideB + (size_t)r * ldb + i];
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)n * ncols) return;
+    const int item = blockIdx.y, j = (int)(t / TB % ncols), b = bidx ? bidx[item] : item;
+    const int row = (int)(t / ((int64_t)TB * ncols)) * TB + (int)(t % TB);
+    const int dst = perm ? perm[(size_t)(aidx ? aidx[item] : b) * strideQ + row] : row;
+    const int64_t c = cols ? cols[(size_t)item * ncols + j] : (int64_t)b * strideB + (int64_t)(r_off + j) * ldb;
+    const size_t o = ((size_t)item * n * ncols + (size_t)(t / TB) * TB) * 2 + t % TB;
+    if (c >= 0) B[c + dst] = make_double2(x[o], x[o + TB]);
 }
 
-// S[member][perm[t]] = B[matrix][t] (the scatter x = P^T w of a transposed solve)
-__global__ void k_unperm(const double2 *B, int ldb, int64_t strideB, int n, int nrhs, const int *perm,
-                         int64_t strideQ, double2 *S, const int *bidx, const int *aidx)
+template <typename T, bool TRANS, bool SCALED>
+void launch_trsv(const TrsvArgs &a, int items, bool upper, hipStream_t s)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, bl = blockIdx.y;
-    const int b = bidx ? bidx[bl] : bl;
-    if (i >= n) return;
-    const int t = perm[(size_t)(aidx ? aidx[bl] : b) * strideQ + i];
-    for (int r = 0; r < nrhs; ++r) S[(size_t)bl * strideB + (size_t)r * ldb + t] = B[(size_t)b * strideB + (size_t)r * ldb + i];
-}
-
-// B[matrix] = S[member]
-__global__ void k_unstage(const double2 *S, int ldb, int64_t strideB, int n, int nrhs, double2 *B, const int *bidx)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, bl = blockIdx.y;
-    const int b = bidx ? bidx[bl] : bl;
-    if (i >= n) return;
-    for (int r = 0; r < nrhs; ++r) B[(size_t)b * strideB + (size_t)r * ldb + i] = S[(size_t)bl * strideB + (size_t)r * ldb + i];
-}
-
-__global__ void k_zero_words(int *p, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
+    const dim3 grid((unsigned)(items * a.chunks), (unsigned)(a.n / TB)), block(256 + 64 * kPsPoll);
+    if (upper) hipLaunchKernelGGL((k_trsv<T, true, TRANS, SCALED>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_trsv<T, false, TRANS, SCALED>), grid, block, 0, s, a);
 }
 
 }  // namespace
@@ -781,94 +695,60 @@ int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm
 
 namespace {
 
-// Buffers of a triangular solve supplied by the caller instead of the
-// context's (the allocation-free entry point): staging of B (batch * strideB
-// complex128) and the packets of both triangles, zeroed by the caller, whose
-// epochs then start at 1.
-struct SolveBufs {
-    double2 *stage = nullptr;
-    uint64_t *pkt = nullptr;
-    int epoch = 0;
-};
+// Bytes of a solve's right-hand sides and solved values, one pass of them.
+size_t solve_bytes(int n, int nrhs, int batch)
+{
+    return 2 * (size_t)batch * n * std::min(nrhs, kPassCols) * sizeof(double2);
+}
 
-// Packets of the two triangles of a batched solve.
-size_t solve_pkts(int n, int nrhs, int batch) { return 2 * (size_t)batch * (n / TB) * rhs_chunk(nrhs) * 256; }
-
-// Staging of B per launch member in ctx->ws_solve; the solved values'
-// packets in ctx->ws_pkt, per triangle and member nblk x NR x 256 packets.
-// trans: solve A^H X = B instead of A X = B.  ext: caller-supplied buffers
-// (nothing allocated, no profiler events).
+// Columns of each matrix in passes of up to kPassCols, in members of up to kPsW
+// columns (as even as possible).  trans: solve A^H X = B instead of A X = B.
+// ext: the buffer of solve_bytes, supplied by the caller instead of the
+// context's (nothing allocated, no profiler events).
 int getrs_any(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int lda, int64_t strideA, const int *perm,
               int64_t strideQ, void *B, int ldb, int64_t strideB, int batch, hipStream_t s, const int *d_bidx,
-              bool trans, const int *d_aidx, SolveBufs *ext = nullptr)
+              bool trans, const int *d_aidx, void *ext = nullptr)
 {
     if (n <= 0 || n % TB != 0 || nrhs <= 0 || batch <= 0 || ldb < n) {
         set_error("getrs: bad arguments (n=%d multiple of %d, nrhs=%d, batch=%d)", n, TB, nrhs, batch);
         return WM_ERR_ARG;
     }
-    const int nblk = n / TB;
-    const int nr_max = rhs_chunk(nrhs);
-    const size_t tri_pkts = (size_t)batch * nblk * nr_max * 256;  // packets per triangle
-    double2 *Ystage = nullptr;
-    uint64_t *pkt = nullptr;
-    int *epoch = nullptr;
-    if (ext) {
-        Ystage = ext->stage;
-        pkt = ext->pkt;
-        epoch = &ext->epoch;
-    } else {
-        WM_TRY(ctx->ws_solve.ensure((size_t)batch * strideB * sizeof(double2)));
-        Ystage = (double2 *)ctx->ws_solve.ptr;
-        // The packets live in their own buffer and only ever carry epoch tags of
-        // this context, so a wait can never be satisfied by stale data.  The
-        // buffer is zeroed whenever it is (re)allocated.
-        const size_t pkt_bytes = 2 * tri_pkts * sizeof(uint64_t);
-        if (ctx->ws_pkt.bytes < pkt_bytes || !ctx->ws_pkt.ptr) {
-            WM_TRY(ctx->ws_pkt.ensure(pkt_bytes));
-            const int64_t nf = (int64_t)(ctx->ws_pkt.bytes / sizeof(int));
-            hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, s, (int *)ctx->ws_pkt.ptr, nf);
-            ctx->solve_epoch = 0;
-        }
-        pkt = (uint64_t *)ctx->ws_pkt.ptr;
-        if (ctx->solve_epoch > (1 << 30)) {  // keep the tags unique: restart from a zeroed buffer
-            const int64_t nf = (int64_t)(ctx->ws_pkt.bytes / sizeof(int));
-            hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, s, (int *)pkt, nf);
-            ctx->solve_epoch = 0;
-        }
-        epoch = &ctx->solve_epoch;
+    uint64_t *in = (uint64_t *)ext;
+    if (!ext) {
+        WM_TRY(ctx->ws_solve.ensure(solve_bytes(n, nrhs, batch)));
+        in = (uint64_t *)ctx->ws_solve.ptr;
     }
-    // the lower solve reads B (staged per member) and writes y into B; the upper solves in place
-    hipLaunchKernelGGL(k_stage, dim3((n + 255) / 256, batch), dim3(256), 0, s, (const double2 *)B, ldb, strideB, n, nrhs,
-                       Ystage, d_bidx);
-    for (int r0 = 0; r0 < nrhs; r0 += rhs_chunk(nrhs - r0)) {
-        TrsvArgs a;
-        a.A = A; a.lda = lda; a.strideA = strideA; a.n = n; a.nrhs = nrhs;
-        a.perm = perm; a.strideQ = strideQ; a.ldb = ldb; a.strideB = strideB; a.err = ctx->d_err;
+    for (int r0 = 0; r0 < nrhs; r0 += kPassCols) {
+        const int nc = std::min(nrhs - r0, kPassCols);
+        uint64_t *pub = in + (size_t)batch * n * nc * 2;
+        const dim3 vgrid((unsigned)(((int64_t)n * nc + 255) / 256), (unsigned)batch);
+        hipLaunchKernelGGL(k_rhs_in, vgrid, dim3(256), 0, s, (const double2 *)B, n, ldb, strideB, r0, nc,
+                           (const int64_t *)nullptr, trans ? (const int *)nullptr : perm, strideQ, d_bidx, d_aidx, in,
+                           pub);
+        TrsvArgs a = {};
+        a.A = A; a.lda = lda; a.strideA = strideA; a.n = n; a.ncols = nc; a.err = ctx->d_err;
+        a.chunks = (nc + kPsW - 1) / kPsW;
+        a.cw = (nc + a.chunks - 1) / a.chunks;
         a.bidx = d_bidx;
         a.aidx = d_aidx;
-        a.Bin = Ystage; a.Y = (double2 *)B; a.pkt = pkt;
-        a.epoch = ++*epoch;
-        const int nr = rhs_chunk(nrhs - r0);
         const double esz = prec == WM_PREC_F64 ? 16.0 : 8.0;
-        const double fl = batch * 4.0 * (double)n * n * nr, by = batch * 0.5 * (double)n * n * esz;
+        const double fl = batch * 4.0 * (double)n * n * nc, by = batch * 0.5 * (double)n * n * esz;
         for (int up = 0; up < 2; ++up) {
-            if (up) { a.Bin = nullptr; a.pkt = pkt + tri_pkts; }
+            a.in = up ? pub : in;
+            a.pub = up ? in : pub;
             if (!ext) prof_begin(ctx, K_TRSV, s);
             if (prec == WM_PREC_F64) {
-                if (trans) trsv_dispatch<double, true>(a, batch, r0, up, s);
-                else trsv_dispatch<double>(a, batch, r0, up, s);
+                if (trans) launch_trsv<double, true, false>(a, batch, up, s);
+                else launch_trsv<double, false, false>(a, batch, up, s);
             } else {
-                if (trans) trsv_dispatch<float, true>(a, batch, r0, up, s);
-                else trsv_dispatch<float>(a, batch, r0, up, s);
+                if (trans) launch_trsv<float, true, false>(a, batch, up, s);
+                else launch_trsv<float, false, false>(a, batch, up, s);
             }
             if (!ext) prof_end(ctx, K_TRSV, s, fl, by);
         }
-    }
-    if (trans) {  // x = P^T w, through the staging buffer
-        hipLaunchKernelGGL(k_unperm, dim3((n + 255) / 256, batch), dim3(256), 0, s, (const double2 *)B, ldb, strideB, n,
-                           nrhs, perm, strideQ, Ystage, d_bidx, d_aidx);
-        hipLaunchKernelGGL(k_unstage, dim3((n + 255) / 256, batch), dim3(256), 0, s, (const double2 *)Ystage, ldb,
-                           strideB, n, nrhs, (double2 *)B, d_bidx);
+        hipLaunchKernelGGL(k_rhs_out, vgrid, dim3(256), 0, s, (const double *)in, n, ldb, strideB, r0, nc,
+                           (const int64_t *)nullptr, trans ? perm : (const int *)nullptr, strideQ, d_bidx, d_aidx,
+                           (double2 *)B);
     }
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
@@ -1013,7 +893,7 @@ int precond_solve(wm_ctx *ctx, int n, int nr, const double2 *Fs, int lda, int64_
     const size_t tab_b = (tab.size() * sizeof(int) + 255) & ~(size_t)255;
     const size_t cols_b = (cols.size() * sizeof(int64_t) + 255) & ~(size_t)255;
     const size_t vec_b = (size_t)members * n * kPsW * sizeof(double2);
-    WM_TRY(ctx->ws_group.ensure(tab_b + cols_b + 3 * vec_b));
+    WM_TRY(ctx->ws_group.ensure(tab_b + cols_b + 2 * vec_b));
     char *base = (char *)ctx->ws_group.ptr;
     std::vector<char> host(tab_b + cols_b, 0);
     std::memcpy(host.data(), tab.data(), tab.size() * sizeof(int));
@@ -1021,27 +901,24 @@ int precond_solve(wm_ctx *ctx, int n, int nr, const double2 *Fs, int lda, int64_
     WM_TRY(copy_h2d(base, host.data(), host.size(), s));
     const int *d_tab = (const int *)base;
     const int64_t *d_cols = (const int64_t *)(base + tab_b);
-    double *in = (double *)(base + tab_b + cols_b);
-    uint64_t *pub = (uint64_t *)(base + tab_b + cols_b + vec_b);
-    uint64_t *pub2 = pub + (size_t)members * n * kPsW * 2;
-    const dim3 grid((unsigned)members, (unsigned)(n / TB)), vgrid((unsigned)(n * kPsW / 256), (unsigned)members);
-    const double fl = 4.0 * (double)n * n * items.size() * nr, by = members * 8.0 * (double)n * n;
-    hipLaunchKernelGGL(k_ps_gather, vgrid, dim3(256), 0, s,
-                       (const double2 *)V, n, d_cols, d_tab, perm, strideQ, in, pub, members);
-    PsolveArgs a;
-    a.F = Fs; a.lda = lda; a.strideF = strideF; a.n = n; a.dinv = Dinv;
-    a.fac = d_tab; a.slot = d_tab + members; a.width = d_tab + 2 * members;
+    uint64_t *in = (uint64_t *)(base + tab_b + cols_b), *pub = in + vec_b / sizeof(uint64_t);
+    const dim3 vgrid((unsigned)(n * kPsW / 256), (unsigned)members);
+    hipLaunchKernelGGL(k_rhs_in, vgrid, dim3(256), 0, s, (const double2 *)V, n, n, (int64_t)0, 0, kPsW, d_cols, perm,
+                       strideQ, (const int *)nullptr, d_tab, in, pub);
+    TrsvArgs a = {};
+    a.A = Fs; a.lda = lda; a.strideA = strideF; a.n = n; a.ncols = a.cw = kPsW; a.chunks = 1; a.dinv = Dinv;
+    a.aidx = d_tab; a.slot = d_tab + members; a.width = d_tab + 2 * members;
     a.err = ctx->d_err;
-    a.in = in; a.pub = pub;
-    prof_begin(ctx, K_TRSV, s);
-    hipLaunchKernelGGL(k_psolve<false>, grid, dim3(256 + 64 * kPsPoll), 0, s, a);
-    prof_end(ctx, K_TRSV, s, fl, by);
-    a.in = (const double *)pub; a.pub = pub2;  // the lower triangle's values are the upper one's right-hand sides
-    prof_begin(ctx, K_TRSV, s);
-    hipLaunchKernelGGL(k_psolve<true>, grid, dim3(256 + 64 * kPsPoll), 0, s, a);
-    prof_end(ctx, K_TRSV, s, fl, by);
-    hipLaunchKernelGGL(k_ps_scatter, vgrid, dim3(256), 0, s,
-                       (const double *)pub2, n, d_cols, V);
+    const double fl = 4.0 * (double)n * n * items.size() * nr, by = members * 8.0 * (double)n * n;
+    for (int up = 0; up < 2; ++up) {
+        a.in = up ? pub : in;
+        a.pub = up ? in : pub;
+        prof_begin(ctx, K_TRSV, s);
+        launch_trsv<double, false, true>(a, members, up, s);
+        prof_end(ctx, K_TRSV, s, fl, by);
+    }
+    hipLaunchKernelGGL(k_rhs_out, vgrid, dim3(256), 0, s, (const double *)in, n, n, (int64_t)0, 0, kPsW, d_cols,
+                       (const int *)nullptr, (int64_t)0, (const int *)nullptr, (const int *)nullptr, V);
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
 }
@@ -1139,8 +1016,7 @@ int residual_batched(wm_ctx *ctx, int n, int nrhs, const void *Z, int ldz, int64
 }  // namespace wm
 
 // ---------------------------------------------------------------------------
-// Allocation-free triangular solves: the staging, permutation and packet
-// buffers of wm_getrs_batched live in `scratch`, a file-scope device array of
+// Allocation-free triangular solves: the permutation and the values' buffers of wm_getrs_batched live in `scratch`, a file-scope device array of
 // kNoAllocBytes that every GPU the library runs on holds until the process
 // ends.  Its device address is taken once per device (wm::noalloc_init, from
 // wm_init with that device current); host code uses that address, never the
@@ -1184,11 +1060,14 @@ extern "C" int wm_getrs_batched_noalloc(wm_ctx *ctx, int prec, int n, int nrhs, 
     }
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t perm_b = up((size_t)batch * n * sizeof(int));
-    const size_t stage_b = up((size_t)batch * strideB * sizeof(double2));
-    const size_t pkt_b = up(solve_pkts(n, nrhs, batch) * sizeof(uint64_t));
-    if (perm_b + stage_b + pkt_b > kNoAllocBytes) {
+    // the documented budget; the values of a pass (solve_bytes) always fit in it:
+    // 32 min(nrhs, 32) <= 16 nrhs + 64 nr' bytes per row
+    int nr2 = 1;
+    while (nr2 * 2 <= std::min(nrhs, 8)) nr2 *= 2;
+    const size_t need = perm_b + up((size_t)batch * strideB * sizeof(double2)) + up((size_t)batch * n * nr2 * 64);
+    if (need > kNoAllocBytes) {
         set_error("wm_getrs_batched_noalloc: n=%d, nrhs=%d, batch=%d need %zu bytes of scratch, the maximum is %zu "
-                  "(use wm_getrs_batched)", n, nrhs, batch, perm_b + stage_b + pkt_b, kNoAllocBytes);
+                  "(use wm_getrs_batched)", n, nrhs, batch, need, kNoAllocBytes);
         return WM_ERR_NOMEM;
     }
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
@@ -1200,15 +1079,9 @@ extern "C" int wm_getrs_batched_noalloc(wm_ctx *ctx, int prec, int n, int nrhs, 
     }
     const hipStream_t s = ctx->stream;
     int *perm = (int *)base;
-    SolveBufs sb;
-    sb.stage = (double2 *)(base + perm_b);
-    sb.pkt = (uint64_t *)(base + perm_b + stage_b);
-    // the previous call's packets carry the same epochs: start from zero
-    const int64_t nw = (int64_t)(pkt_b / sizeof(int));
-    hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, s, (int *)sb.pkt, nw);
     WM_TRY(perm_batched(ctx, n, ipiv, strideP, perm, n, batch, s));
     WM_TRY(getrs_any(ctx, prec, n, nrhs, A, lda, strideA, perm, n, B, ldb, strideB, batch, s, nullptr, false, nullptr,
-                     &sb));
+                     base + perm_b));
     return check_device_error(ctx, s);
 }
 

@@ -182,8 +182,10 @@ int getrf_batched(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t stride
                   int64_t strideP, int batch, int *d_info, hipStream_t s, const int *d_bidx = nullptr,
                   const int *d_nmem = nullptr);
 // Row permutation of each factorization: perm[t] = source row of position t.
+// maps: scratch of 32 bytes per row and matrix (null: the context's, which a
+// triangular solve after it uses again).
 int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm, int64_t strideQ, int batch,
-                 hipStream_t s, const int *d_bidx = nullptr);
+                 hipStream_t s, const int *d_bidx = nullptr, void *maps = nullptr);
 // Triangular solves with the LU factors and a precomputed permutation; B complex128.
 // d_aidx (optional): member i solves with the factors and permutation of
 // matrix d_aidx[i] (e.g. another frequency's) on the right-hand sides of

@@ -55,24 +55,50 @@ __device__ inline void cfma(double2 &acc, double2 a, double2 b)
     acc.y = fma(a.y, b.x, acc.y);
 }
 
-// perm[t] = source row of position t after applying ipiv in order: each thread
-// follows its position through the interchanges backwards, last to first, so
-// the matrix's rows are traced side by side instead of the interchanges applied
-// one after another by one thread (N = 8192, two matrices: 0.8 -> 0.36 ms of a
-// solve).
-__global__ __launch_bounds__(256) void k_perm(const int *ipiv, int64_t strideP, int n, int *perm, int64_t strideQ,
-                                              const int *bidx)
+// Source row of position t after applying ipiv in order: each thread follows
+// its position through the interchanges backwards, last to first.  A thread's
+// trace is a serial chain (35 cycles per interchange: the pivots of 64 of them in
+// one load, a lane read each), so a long sequence is cut into kPermParts parts
+// traced side by side (blockIdx.y; map[member][part][position]) and the parts'
+// maps are followed one through the other (k_perm_join).  N = 8192, two
+// matrices: 50 us; one thread swapping in LDS 800, one part 470 (with scalar loads).
+constexpr int kPermParts = 8;
+constexpr int kPermWhole = 512;  // up to here one part: the join costs more than it saves
+
+__global__ __launch_bounds__(256) void k_perm(const int *ipiv, int64_t strideP, int n, int len, int *out,
+                                              int64_t strideOut, const int *bidx, int map)
 {
-    const int b = bidx ? bidx[blockIdx.y] : (int)blockIdx.y;
+    const int bl = blockIdx.z, part = blockIdx.y, lane = threadIdx.x & 63;
+    const int b = bidx ? bidx[bl] : bl;
     const int *ip = ipiv + (size_t)b * strideP;
     const int t = blockIdx.x * 256 + threadIdx.x;
+    const int i_lo = part * len, i_hi = min(n, i_lo + len);  // len is a multiple of 64
+    auto load = [&](int i0) { return i0 + lane < i_hi ? ip[i0 + lane] - 1 : i0 + lane; };
     int row = t;
-#pragma unroll 16
-    for (int i = n - 1; i >= 0; --i) {
-        const int p = ip[i] - 1;  // uniform: scalar loads
-        row = row == i ? p : row == p ? i : row;
+    int i0 = i_lo + (i_hi - i_lo - 1) / 64 * 64;
+    int next = load(i0);
+    for (; i0 >= i_lo; i0 -= 64) {
+        const int cur = next;
+        if (i0 > i_lo) next = load(i0 - 64);
+#pragma unroll
+        for (int k = 63; k >= 0; --k) {
+            const int p = __builtin_amdgcn_readlane(cur, k), i = i0 + k;
+            row = row == i ? p : row == p ? i : row;
+        }
     }
-    if (t < n) perm[(size_t)b * strideQ + t] = row;
+    if (t < n) out[(map ? (size_t)bl * kPermParts + part : (size_t)b) * strideOut + t] = row;
+}
+
+__global__ __launch_bounds__(256) void k_perm_join(const int *map, int n, int *perm, int64_t strideQ, const int *bidx)
+{
+    const int bl = blockIdx.y, t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    int row = t;
+    for (int part = kPermParts - 1; part >= 0; --part) {
+        if ((unsigned)row >= (unsigned)n) break;  // a pivot outside the matrix
+        row = map[((size_t)bl * kPermParts + part) * n + row];
+    }
+    perm[(size_t)(bidx ? bidx[bl] : bl) * strideQ + t] = row;
 }
 
 // Packed entries of one 64 x 64 triangle with its diagonal.
@@ -682,13 +708,27 @@ void launch_trsv(const TrsvArgs &a, int items, bool upper, hipStream_t s)
 }  // namespace
 
 int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm, int64_t strideQ, int batch,
-                 hipStream_t s, const int *d_bidx)
+                 hipStream_t s, const int *d_bidx, void *maps)
 {
     if ((size_t)n * sizeof(int) > ctx->max_lds) {  // the accepted range of n (40960 rows)
         set_error("permutation: n=%d exceeds the LDS capacity", n);
         return WM_ERR_ARG;
     }
-    hipLaunchKernelGGL(k_perm, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, s, ipiv, strideP, n, perm, strideQ, d_bidx);
+    const unsigned nb = (unsigned)((n + 255) / 256);
+    if (n <= kPermWhole) {
+        hipLaunchKernelGGL(k_perm, dim3(nb, 1, (unsigned)batch), dim3(256), 0, s, ipiv, strideP, n, (n + 63) / 64 * 64,
+                           perm, strideQ, d_bidx, 0);
+    } else {
+        if (!maps) {
+            WM_TRY(ctx->ws_solve.ensure((size_t)batch * kPermParts * n * sizeof(int)));
+            maps = ctx->ws_solve.ptr;
+        }
+        const int len = (n + kPermParts * 64 - 1) / (kPermParts * 64) * 64;
+        hipLaunchKernelGGL(k_perm, dim3(nb, kPermParts, (unsigned)batch), dim3(256), 0, s, ipiv, strideP, n, len,
+                           (int *)maps, (int64_t)n, d_bidx, 1);
+        hipLaunchKernelGGL(k_perm_join, dim3(nb, (unsigned)batch), dim3(256), 0, s, (const int *)maps, n, perm,
+                           strideQ, d_bidx);
+    }
     WM_HIP_TRY(hipGetLastError());
     return WM_OK;
 }
@@ -1079,7 +1119,8 @@ extern "C" int wm_getrs_batched_noalloc(wm_ctx *ctx, int prec, int n, int nrhs, 
     }
     const hipStream_t s = ctx->stream;
     int *perm = (int *)base;
-    WM_TRY(perm_batched(ctx, n, ipiv, strideP, perm, n, batch, s));
+    // the parts' maps (32 bytes per row) lie where the values go afterwards (32 per row and column)
+    WM_TRY(perm_batched(ctx, n, ipiv, strideP, perm, n, batch, s, nullptr, base + perm_b));
     WM_TRY(getrs_any(ctx, prec, n, nrhs, A, lda, strideA, perm, n, B, ldb, strideB, batch, s, nullptr, false, nullptr,
                      base + perm_b));
     return check_device_error(ctx, s);

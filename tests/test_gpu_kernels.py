@@ -175,3 +175,31 @@ def test_preconditioner_solve_widths(wm, ctx, n):
         assert not np.isfinite(got[0]).all() and not np.isfinite(got[w - 1]).all()
     dev.free()
     piv.free()
+
+
+@pytest.mark.parametrize("n", [64, 448, 512, 576, 640, 1088, 8192])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_row_permutation(wm, ctx, n, noalloc):
+    """The interchanges of a pivot sequence applied to a right-hand side (factors:
+    the identity, so the solution is the permuted vector, exactly): sequences of
+    a factorization (row i meets a row at or below it) and any others, at sizes
+    of one part, of parts that are empty, ragged or whole."""
+    rng = np.random.RandomState(n)
+    A = wm.DeviceArray(ctx, np.ascontiguousarray(np.broadcast_to(np.eye(n, dtype=np.complex128), (2, n, n))))
+    piv = np.empty((2, n), np.int32)
+    piv[0] = [rng.randint(i, n) + 1 for i in range(n)]
+    piv[1] = rng.randint(0, n, n) + 1
+    P = wm.DeviceArray(ctx, piv)
+    b = np.arange(2 * n, dtype=np.complex128).reshape(2, 1, n)
+    B = wm.DeviceArray(ctx, b)
+    f = wm.lib().wm_getrs_batched_noalloc if noalloc else wm.lib().wm_getrs_batched
+    assert f(ctx.h, wm.PREC_F64, n, 1, A.ptr, n, C.c_int64(n * n), P.ptr, C.c_int64(n),
+             B.ptr, n, C.c_int64(n), 2) == 0
+    ref = b.copy()
+    for m in range(2):
+        for i in range(n):
+            p = piv[m, i] - 1
+            ref[m, 0, [i, p]] = ref[m, 0, [p, i]]
+    assert np.array_equal(B.download(), ref)
+    for d in (A, P, B):
+        d.free()

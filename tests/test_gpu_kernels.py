@@ -203,3 +203,23 @@ def test_row_permutation(wm, ctx, n, noalloc):
     assert np.array_equal(B.download(), ref)
     for d in (A, P, B):
         d.free()
+
+
+@pytest.mark.parametrize("n", [2, 127, 128, 2100])
+def test_host_matrices(wm, geometries, ctx, geo_dir, n):
+    """Matrices to and from the host where the device pads them: a few rows, no padding
+    (128), and 2100 rows (two chunks).  zmatrix equals the batched fill's values
+    bit for bit, and LU_cuBLAS solves with the matrix it is given (residual within
+    n eps of |A| |x|, as partial pivoting gives on random matrices)."""
+    import os
+    p = os.path.join(geo_dir, f"host_{n}.geo")
+    geometries.dipole(p, n + 1, 1.0, 0.2 / (n + 1))
+    Z = wm.zmatrix(wm.configwire(p), wm.wavenumber(150.0))
+    assert Z.shape == (n, n)
+    assert np.array_equal(Z, wm.Geometry.load(ctx, p).fill([150.0])[0])
+    rng = np.random.RandomState(n)
+    A = rng.randn(n, n) + 1j * rng.randn(n, n)
+    b = rng.randn(n, 3) + 1j * rng.randn(n, 3)
+    x = wm.LU_cuBLAS(A, b)
+    r = np.abs(A @ x - b).max() / (np.abs(A).sum(axis=1).max() * np.abs(x).max())
+    assert r <= n * 2.0 ** -52

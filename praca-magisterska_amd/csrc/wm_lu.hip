@@ -1165,16 +1165,23 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32(float2 *Abase, int lda, int
 // load the one after, with one barrier per chunk.  Rows and columns beyond the
 // update load the last one's values (their products reach no stored entry), so
 // the loads need no condition and a column's eight elements come as four 16-byte
-// loads: N = 8192, K = 512: 905 -> 742 us.
+// loads: N = 8192, K = 512: 905 -> 742 us.  A chunk's products are issued before
+// the next one's splitting, which runs beside them: 742 -> 690 (alone on its CU a
+// workgroup's chunk takes 1.35 us instead of 1.75).  Eight lanes per column of U,
+// two k each, whole lines per load but 4-byte LDS stores: 722.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4), aligned(8)));
 constexpr int GB_BM = 128, GB_BN = 128, GB_KC = 16;
 
-__device__ inline void split_bf16(float x, __bf16 &hi, __bf16 &lo)
+// Two values (consecutive k) at once: hi and lo pairs as words.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ inline void split_bf16(float x, float y, unsigned &hi, unsigned &lo)
 {
-    hi = (__bf16)x;
-    lo = (__bf16)(x - (float)hi);
+    hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+    const float hx = __builtin_bit_cast(float, hi << 16), hy = __builtin_bit_cast(float, hi & 0xffff0000u);
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x - hx, y - hy}), bf16x2));
 }
 
 // k offset (bf16) of half h (0: k 0-7, 1: k 8-15) of LDS row r of a chunk
@@ -1222,31 +1229,31 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b3(float2 *Abase, int lda, int6
         for (int e = 0; e < 4; ++e) pb[e] = *(const f32x4 *)(pB + kc + 2 * e);
     };
     auto stash = [&](int buf) {
-        bf16x8 v[4];
+        u32x4 v[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            __bf16 h, l;
-            split_bf16(pa[e].x, h, l);
+        for (int e = 0; e < 4; ++e) {
+            unsigned h, l;
+            split_bf16(pa[2 * e].x, pa[2 * e + 1].x, h, l);
             v[0][e] = h;
             v[1][e] = l;
-            split_bf16(pa[e].y, h, l);
+            split_bf16(pa[2 * e].y, pa[2 * e + 1].y, h, l);
             v[2][e] = h;
             v[3][e] = l;
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) *(bf16x8 *)&sL[buf][q][lr][b3_half(lr, lh)] = v[q];
+        for (int q = 0; q < 4; ++q) *(u32x4 *)&sL[buf][q][lr][b3_half(lr, lh)] = v[q];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            __bf16 h, l;
-            split_bf16(pb[e / 2][e % 2 * 2], h, l);
+        for (int e = 0; e < 4; ++e) {
+            unsigned h, l;
+            split_bf16(pb[e][0], pb[e][2], h, l);
             v[0][e] = h;
             v[1][e] = l;
-            split_bf16(pb[e / 2][e % 2 * 2 + 1], h, l);
+            split_bf16(pb[e][1], pb[e][3], h, l);
             v[2][e] = h;
             v[3][e] = l;
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) *(bf16x8 *)&sU[buf][q][uc][b3_half(uc, uh)] = v[q];
+        for (int q = 0; q < 4; ++q) *(u32x4 *)&sU[buf][q][uc][b3_half(uc, uh)] = v[q];
     };
     v16f accR[2][2], accI[2][2];
 #pragma unroll
@@ -1295,19 +1302,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b3(float2 *Abase, int lda, int6
 
     fetch(0);
     stash(0);
-    if (GB_KC < K) fetch(GB_KC);
+    fetch(GB_KC);  // K is a multiple of 64
     __syncthreads();
     int buf = 0;
-    for (int kc = 0; kc < K; kc += GB_KC, buf ^= 1) {
-        // the next chunk (in registers) to the other buffer, the one after
-        // from memory, then this chunk's products
-        if (kc + GB_KC < K) {
-            stash(buf ^ 1);
-            if (kc + 2 * GB_KC < K) fetch(kc + 2 * GB_KC);
-        }
+    for (int kc = 0; kc + GB_KC < K; kc += GB_KC, buf ^= 1) {
         compute(buf);
+        stash(buf ^ 1);
+        fetch(min(kc + 2 * GB_KC, K - GB_KC));
         __syncthreads();
     }
+    compute(buf);
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll

@@ -51,6 +51,10 @@ constexpr int kSubDefault = 4, kSubLarge = 8, kSubLargeN = 8192;
 // candidate row); complex128 panels measured 208 us with two parts (3 -> 2
 // workgroups per CU) and 165 us with four, complex64 ones 280 us with one and
 // 196 us with two (64 columns, N = 512 .. 4096).
+// Half as many parts, rows of twice as many columns per thread, take a matrix
+// whose clusters do not fit on the device otherwise (n above 64 rows per
+// resident workgroup: 49152 complex128 rows, or fewer where contexts share the
+// device); slower (registers spill), but such a matrix has no other panel.
 constexpr int kTprF64 = 4, kTprF32 = 2;
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
     constexpr int NW = XLayout<V>::NW, NWS = XLayout<V>::NWS, SLS = XLayout<V>::SLS;
     constexpr int G = kPanelGroup;  // columns updated together
     constexpr int NE = NW / TPR / 2;  // values of a chunk's part of a row: one lane each (complex128: re and im apart)
-    static_assert(NE == 32 && RW >= NB && W % 8 == 0 && W % G == 0, "panel layout");
+    static_assert((NE == 32 || NE == 64) && RW >= NB && W % 8 == 0 && W % G == 0, "panel layout");
     const int bl = blockIdx.y, w = blockIdx.x;          // bl: member of this launch
     const int b = a.bidx ? a.bidx[bl] : bl;              // b: matrix index
     const int tid = threadIdx.x, lane = tid & 63;
@@ -371,8 +375,11 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         }
         // the pivot's reciprocal: by a wave whose columns are finished, where
         // there is one
+        V p1 = V{0, 0};  // the lane reads by the whole wave: a register reloaded for
+                         // lane 0 alone would not hold lane wl's value
+        if (TPR == 1 && wl >= 0) p1 = V{readlane_t(nxr, wl), readlane_t(nxi, wl)};
         if (wl >= 0 && owner && c == (cj > 0 ? cj - 1 : 0) && lane == 0) {
-            const V p = TPR > 1 ? s_nx[par][rb * 64 + wl] : V{readlane_t(nxr, wl), readlane_t(nxi, wl)};
+            const V p = TPR > 1 ? s_nx[par][rb * 64 + wl] : p1;
             const double2 rp = p.x != 0 || p.y != 0 ? crecip((double)p.x, (double)p.y) : make_double2(0.0, 0.0);
             if (solo) {
                 s_rinv[par] = rp;
@@ -499,7 +506,9 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
             // matrices, whose pivots stay near the diagonal.
             constexpr int PL = NW / 64;  // pivot-row words per lane, loaded together
             uint64_t wu[PL], wi;
-            auto val = [&](int e) { return e * NE + lane % NE; };  // value whose word this lane takes
+            // the value whose word this lane takes, and which of its two words
+            auto val = [&](int e) { return (64 * e + lane) / (2 * NE) * NE + lane % NE; };
+            auto half = [&](int e) { return (64 * e + lane) / NE % 2; };
             auto load_row = [&](int sl) {
                 const uint64_t *pu = cand + sl * NWS;
 #pragma unroll
@@ -566,7 +575,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
                     load_row(ws);
                 }
 #pragma unroll
-                for (int e = 0; e < PL; ++e) ((uint32_t *)s_u[par])[2 * val(e) + lane / NE] = (uint32_t)wu[e];
+                for (int e = 0; e < PL; ++e) ((uint32_t *)s_u[par])[2 * val(e) + half(e)] = (uint32_t)wu[e];
                 const uint32_t ri = (uint32_t)wi;
                 auto word = [&](int q) { return (unsigned long long)(unsigned)__builtin_amdgcn_readlane(ri, q); };
                 rinv.x = __longlong_as_double((long long)((word(1) << 32) | word(0)));
@@ -1468,21 +1477,29 @@ struct GetrfPlan {
     size_t xbytes = 0;
 };
 
+// Panel workgroups of this context that may be resident at once: the occupancy,
+// shared with the other contexts that factor on the device at the same time
+// (panel_share), so that every cluster of every concurrent panel launch fits on
+// the device together.
+template <typename T, int TPR>
+int panel_resident(wm_ctx *ctx, int *resident)
+{
+    int bpc = 0;
+    WM_TRY((occupancy_panel<T, TPR>(&bpc)));
+    *resident = bpc * ctx->num_cu / std::max(1, ctx->panel_share);
+    if (ctx->panel_resident_cap > 0 && ctx->panel_resident_cap < *resident) *resident = ctx->panel_resident_cap;
+    return WM_OK;
+}
+
 template <typename T, int TPR>
 int getrf_plan(wm_ctx *ctx, int n, int batch, GetrfPlan *pl)
 {
     using V = typename CT<T>::V;
     constexpr int RW = 256 / TPR;
     const int pmax = (n + RW - 1) / RW;
-    int bpc = 0;
-    WM_TRY((occupancy_panel<T, TPR>(&bpc)));
-    // panel workgroups of this context that may be resident at once: the
-    // occupancy, shared with the other contexts that factor on the device at
-    // the same time (panel_share), so that every cluster of every concurrent
-    // panel launch fits on the device together
-    int resident = bpc * ctx->num_cu / std::max(1, ctx->panel_share);
-    if (ctx->panel_resident_cap > 0 && ctx->panel_resident_cap < resident) resident = ctx->panel_resident_cap;
-    if (pmax > resident || bpc <= 0) {
+    int resident = 0;
+    WM_TRY((panel_resident<T, TPR>(ctx, &resident)));
+    if (pmax > resident) {
         set_error("getrf: panel cluster of %d workgroups exceeds %d resident", pmax, resident);
         return WM_ERR_ARG;
     }
@@ -1712,6 +1729,13 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
 {
     const int ks = getrf_block(ctx, prec, n);
     GetrfPlan pl;
+    if constexpr (TPR == (sizeof(T) == 8 ? kTprF64 : kTprF32)) {
+        int resident = 0;
+        WM_TRY((panel_resident<T, TPR>(ctx, &resident)));
+        if ((n + 256 / TPR - 1) / (256 / TPR) > resident)
+            return getrf_run<T, TPR / 2>(ctx, prec, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, gk,
+                                         d_nmem);
+    }
     WM_TRY((getrf_plan<T, TPR>(ctx, n, batch, &pl)));
     const uint64_t ntags = (uint64_t)n;
     WM_TRY(prepare_xbuf(ctx, pl.xbytes, ntags, s));

@@ -710,7 +710,7 @@ void launch_trsv(const TrsvArgs &a, int items, bool upper, hipStream_t s)
 int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm, int64_t strideQ, int batch,
                  hipStream_t s, const int *d_bidx, void *maps)
 {
-    if ((size_t)n * sizeof(int) > ctx->max_lds) {  // the accepted range of n (40960 rows)
+    if ((size_t)n * sizeof(int) > ctx->max_lds) {  // the accepted range of n
         set_error("permutation: n=%d exceeds the LDS capacity", n);
         return WM_ERR_ARG;
     }

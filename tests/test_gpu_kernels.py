@@ -223,3 +223,31 @@ def test_host_matrices(wm, geometries, ctx, geo_dir, n):
     x = wm.LU_cuBLAS(A, b)
     r = np.abs(A @ x - b).max() / (np.abs(A).sum(axis=1).max() * np.abs(x).max())
     assert r <= n * 2.0 ** -52
+
+
+@pytest.mark.parametrize("prec,rows", [("f64", 128), ("f32", 256)])
+@pytest.mark.parametrize("n", [256, 1024, 1088])
+def test_panel_fewer_parts(wm, ctx, prec, rows, n):
+    """A matrix whose clusters do not fit at the usual rows per workgroup is factored
+    with half the parts per row and twice the rows: the same factors and pivots,
+    bit for bit; one workgroup less, and it is refused."""
+    L = wm.lib()
+    L.wmx_set_panel_resident.argtypes = [C.c_void_p, C.c_int]
+    rng = np.random.RandomState(n)
+    A = rng.randn(2, n, n) + 1j * rng.randn(2, n, n)
+    dev, piv, info = wm.getrf_batched(ctx, A, prec)
+    ref, P = dev.download(), piv.download()
+    assert not info.any()
+    cap = -(-n // rows)
+    assert L.wmx_set_panel_resident(ctx.h, cap) == 0
+    try:
+        dev, piv, info = wm.getrf_batched(ctx, A, prec)
+        assert not info.any()
+        assert np.array_equal(piv.download(), P)
+        assert np.array_equal(dev.download(), ref)
+        if cap > 1:
+            assert L.wmx_set_panel_resident(ctx.h, cap - 1) == 0
+            with pytest.raises(wm.WireMoMError):
+                wm.getrf_batched(ctx, A, prec)
+    finally:
+        assert L.wmx_set_panel_resident(ctx.h, 0) == 0

@@ -179,8 +179,8 @@ int wm_getrs_batched(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int 
 
 /* wm_getrs_batched without any device allocation, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  No counterpart in the reference.  Its staging,
- * permutation and packet buffers live in a 32 MiB device array of the library
+ * forbid hipMalloc).  No counterpart in the reference.  Its
+ * permutation and value buffers live in a 32 MiB device array of the library
  * that each GPU holds until the process ends; sizes needing more than that
  * (batch * (4 n + 16 strideB + 64 n nr') bytes with nr' = min(nrhs, 8)
  * rounded down to a power of two, each term rounded up to 256) are rejected

@@ -43,8 +43,11 @@ namespace {
 constexpr int NB = 64;
 // Panels per outer block of the factorization (tunable per context).  Deeper
 // blocks give the trailing update a longer K (better MFMA use) at the cost of
-// more narrow updates inside the block; measured on MI355X at N = 8192, 8
-// panels beat 4 by 1.4-6.5 % for every factor precision.
+// more narrow updates inside the block.  At N = 8192 8 panels beat 4 by 1.4-6.5 %
+// while the narrow updates were slow; now 4 are ahead there (2 x 8192 complex128
+// 69.7 against 72.3 ms, 10 x 8192 split-BF16x3 113.7 against 115.2; 2 x 14336 265.1
+// against 265.9).  The defaults are what wm_get_getrf_block reports and stay;
+// wm_tune_getrf finds the faster depth.
 constexpr int kSubDefault = 4, kSubLarge = 8, kSubLargeN = 8192;
 // Parts per panel row (waves sharing a row).  Narrow parts shorten what each
 // wave does per column (16 or 32 columns of updates, the transposition of a

@@ -1179,13 +1179,13 @@ int run_sweep(wm_ctx *c, const wm_geom *g, const wm_solve_opts &o, std::vector<W
     while (f0 < nfreq) {
         int cnt = std::min(batch, nfreq - f0);
         if (mixed) {
-            // Mixed sweeps go in batches at most one factorization launch wide,
-            // so that each batch is routed with the rates of the frequencies just
-            // above it, and cut where the routed precision changes: a run of
-            // frequencies that all route to FP64 factors (the lower ones once
-            // refinement stops converging) goes as one batch, whose members
-            // share the panel launches.
-            const int w = std::min(cnt, getrf_width(c, WM_PREC_F32, g->ld));
+            // Mixed sweeps go in batches at most mixed_width wide, so that each
+            // batch is routed with the rates of the frequencies just above it,
+            // and cut where the routed precision changes: a run of frequencies
+            // that all route to FP64 factors (the lower ones once refinement
+            // stops converging) goes as one batch, whose members share the
+            // panel launches.
+            const int w = std::min(cnt, mixed_width(c, g->ld));
             if (o.size_policy && prefer_f64(c, o.prec, g->ld, w)) {
                 for (int b = f0; b < f0 + w; ++b) items[b].fprec = WM_PREC_F64;
                 cnt = w;

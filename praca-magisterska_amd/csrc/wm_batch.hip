@@ -476,6 +476,23 @@ void record_rates(const WorkItem *items, int count)
     }
 }
 
+// Launch widths that the cost constants below belong to: three panel workgroups
+// per CU, shared by the contexts that factor at the same time, of 128
+// (complex128) or 256 (complex64) rows each.  The panel kernels now hold half as
+// many rows per workgroup (getrf_width) and take a third of the time per column.
+// Widths and constants go together: with the kernels' widths and these constants
+// the model gave up FP64 factors that the former pair had given (two contexts,
+// FP32, 12 matrices of 4096: ratio 0.99 -> 1.24; 6 of 8192: 1.13 -> 1.33), so work
+// went to fewer bits with no measurement behind it.  The decisions are those of
+// the pair; with today's kernels complex64 factors would be the faster side of
+// some of them (milliseconds, FP64 | complex64: grid 63 x 2048 BF16x3 38 | 34,
+// grid 24 x 4096 FP32 86 | 79, cage 14 x 5376 FP32 112 | 75, 13 x 7040 210 | 133).
+int model_width(int num_cu, int share, int prec, int n)
+{
+    const int rows = prec == WM_PREC_F64 ? 128 : 256;
+    return std::max(1, 3 * num_cu / std::max(1, share) / ((n + rows - 1) / rows));
+}
+
 // Panel launches of a lockstep factorization of `count` matrices of size n
 // when `width` full-height panels fit in one launch: the panel at row s*64
 // (height n - 64 s) goes in ceil(count (n - 64 s) / (width n)) launches.
@@ -503,11 +520,13 @@ double refine_cost(double n, int count)
     return 6.0 * (2.0 * n / 64 * 8e-6 + count * 24.0 * n * n / 5e12);
 }
 
-bool prefer_f64(wm_ctx *c, int prec, int n, int count)
+namespace {
+
+bool f64_cheaper(int num_cu, int share, int prec, int n, int count)
 {
     if (prec == WM_PREC_F64 || count <= 0) return false;
     const double nn = (double)n, flu = 8.0 / 3.0 * nn * nn * nn;
-    const int w64 = getrf_width(c, WM_PREC_F64, n), w32 = getrf_width(c, prec, n);
+    const int w64 = model_width(num_cu, share, WM_PREC_F64, n), w32 = model_width(num_cu, share, prec, n);
     const double t64 = 64 * kPanelColF64 * panel_launches(n, count, w64) + count * flu / kRateF64;
     const double rate = prec == WM_PREC_BF16X3 ? kRateB3 : kRateF32;
     const double tmix = 64 * kPanelColC64 * panel_launches(n, count, w32) + count * flu / rate + refine_cost(nn, count);
@@ -519,19 +538,30 @@ bool prefer_f64(wm_ctx *c, int prec, int n, int count)
     return t64 <= kComplex64Margin * tmix;
 }
 
-bool join_f64(wm_ctx *c, int prec, int n, int r)
+bool f64_joins(int num_cu, int share, int prec, int n, int r)
 {
     if (prec == WM_PREC_F64 || r <= 0) return false;
     // complex128 members of a large lockstep batch cost their products plus a
     // share of its panel launches (n x 7.4 us / (2 x launch width)); a separate
     // complex64 batch pays its own panel launches, products and refinement
     const double nn = (double)n, flu = 8.0 / 3.0 * nn * nn * nn;
-    const int w64 = getrf_width(c, WM_PREC_F64, n), w32 = getrf_width(c, prec, n);
+    const int w64 = model_width(num_cu, share, WM_PREC_F64, n), w32 = model_width(num_cu, share, prec, n);
     const double t_join = r * (flu / kRateF64 + nn * kPanelColF64 / (2.0 * w64));
     const double rate = prec == WM_PREC_BF16X3 ? kRateB3 : kRateF32;
     const double t_sep = 64 * kPanelColC64 * panel_launches(n, r, w32) + r * flu / rate + refine_cost(nn, r);
     return t_join <= t_sep;
 }
+
+}  // namespace
+
+bool prefer_f64(const wm_ctx *c, int prec, int n, int count)
+{
+    return f64_cheaper(c->num_cu, c->panel_share, prec, n, count);
+}
+
+bool join_f64(const wm_ctx *c, int prec, int n, int r) { return f64_joins(c->num_cu, c->panel_share, prec, n, r); }
+
+int mixed_width(const wm_ctx *c, int n) { return model_width(c->num_cu, c->panel_share, WM_PREC_F32, n); }
 
 void route_items(const wm_solve_opts &o, WorkItem *items, int count)
 {
@@ -1093,4 +1123,16 @@ extern "C" int wmx_refine_decide(int nrhs, const double *dm, const double *xm, d
 {
     if (nrhs <= 0 || !dm || !xm || !prev || !first || !rate || !worst) return -100;
     return wm::refine_decide(nrhs, dm, xm, prev, it, tol, max_iter, *first, *rate, *worst);
+}
+
+// Internal test hook (not part of include/wiremom.h): the decisions of the
+// factor precision model for a device of num_cu CUs shared by `share` contexts,
+// without a device.
+extern "C" int wmx_route_model(int num_cu, int share, int prec, int n, int count, int *prefer, int *join, int *width)
+{
+    if (num_cu <= 0 || share <= 0 || prec < 0 || prec > 2 || n <= 0 || !prefer || !join || !width) return WM_ERR_ARG;
+    *prefer = wm::f64_cheaper(num_cu, share, prec, n, count);
+    *join = wm::f64_joins(num_cu, share, prec, n, count);
+    *width = wm::model_width(num_cu, share, WM_PREC_F32, n);
+    return WM_OK;
 }

@@ -311,10 +311,12 @@ void route_items(const wm_solve_opts &o, WorkItem *items, int count);
 // True when a batch of `count` items of size n costs less with FP64 factors
 // than with complex64 factors plus refinement (small n: the factorization is
 // bound by the panels' per-column latency in both precisions).
-bool prefer_f64(wm_ctx *c, int prec, int n, int count);
+bool prefer_f64(const wm_ctx *c, int prec, int n, int count);
 // A run of r complex64-routed frequencies followed by FP64-routed ones: true if
 // factoring the run with the FP64 batch is predicted cheaper than on its own.
-bool join_f64(wm_ctx *c, int prec, int n, int r);
+bool join_f64(const wm_ctx *c, int prec, int n, int r);
+// Most frequencies of a mixed sweep's batch: the model's complex64 launch width.
+int mixed_width(const wm_ctx *c, int n);
 // Matrices per launch of the batched factorization (panel cluster residency).
 int getrf_width(wm_ctx *ctx, int prec, int n);
 // Panels per outer block for a factorization of size n in precision prec.

@@ -251,3 +251,17 @@ def test_panel_fewer_parts(wm, ctx, prec, rows, n):
                 wm.getrf_batched(ctx, A, prec)
     finally:
         assert L.wmx_set_panel_resident(ctx.h, 0) == 0
+
+
+def test_mixed_sweep_routes_by_model(wm, geometries, ctx, geo_dir):
+    """A wide split-BF16x3 sweep of a size where the cost model takes FP64 factors gets them
+    for every frequency, with the FP64 sweep's bits (the model by itself: the host tests)."""
+    import os
+    p = os.path.join(geo_dir, "route_2048.geo")
+    geometries.planar_grid(p, 2048, seed=3, size=5.0)
+    g = wm.Geometry.load(ctx, p)
+    f = np.linspace(20.0, 60.0, 63)
+    zin, cur, st = wm.solve_sweep(g, f, [7], "bf16x3")
+    assert [s["prec"] for s in st] == [wm.PREC_F64] * len(f)
+    z64, c64, _ = wm.solve_sweep(g, f, [7], "f64")
+    assert np.array_equal(zin, z64) and np.array_equal(cur, c64)

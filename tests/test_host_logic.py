@@ -255,3 +255,22 @@ def test_anchor_cover_is_valid_and_minimal(wm):
             if best:
                 break
         assert len(set(anc)) == best, (trial, anc, best, ff, r, diam)
+
+
+@pytest.mark.parametrize("share,prec,n,count,prefer,join,width", [
+    # complex64 precisions (1 FP32, 2 BF16x3); both sides of the model's margin
+    (1, 1, 2432, 64, 1, 1, 76), (1, 1, 2944, 33, 1, 1, 64), (1, 1, 4096, 12, 1, 1, 48), (1, 1, 5376, 14, 1, 1, 36),
+    (1, 1, 7040, 13, 1, 0, 27), (1, 1, 8192, 12, 0, 0, 24), (1, 1, 8832, 8, 1, 0, 21), (1, 2, 2048, 63, 1, 1, 96),
+    (1, 2, 3584, 20, 1, 1, 54), (1, 2, 8192, 12, 0, 0, 24),
+    (2, 1, 4096, 12, 1, 1, 24), (2, 1, 8192, 6, 1, 1, 12), (2, 2, 3584, 12, 1, 1, 27), (2, 2, 8320, 3, 1, 1, 11),
+    (2, 2, 8192, 12, 0, 0, 12), (3, 1, 4992, 8, 1, 1, 12), (4, 1, 3712, 6, 1, 1, 12), (4, 1, 12800, 4, 0, 0, 3),
+    (4, 2, 5120, 4, 1, 1, 9), (4, 2, 8192, 2, 1, 1, 6),
+])
+def test_factor_precision_model(wm, share, prec, n, count, prefer, join, width):
+    """Which batches get FP64 factors although complex64 ones were asked for, whether a run
+    of complex64 frequencies joins the FP64 batch behind it, and the widest batch of a mixed
+    sweep: fixed by the cost model's own launch widths, whatever a panel kernel's workgroups
+    hold (a device of 256 CUs, one to four contexts)."""
+    p, j, w = C.c_int(-1), C.c_int(-1), C.c_int(-1)
+    assert wm.lib().wmx_route_model(256, share, prec, n, count, C.byref(p), C.byref(j), C.byref(w)) == 0
+    assert (p.value, j.value, w.value) == (prefer, join, width)

@@ -38,6 +38,10 @@ HIPFLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "
 # space, VGPR spills nor scratch is accepted for them.  (SGPR spills go to VGPR
 # lanes, not memory, and are allowed.)
 SPILL_FREE = {"wm_fill.hip": ("k_fill", "k_self_terms")}
+# Kernels full of lane reads (readlane, DPP): a spilled register that is reloaded
+# under a partial execution mask does not hold the other lanes' values, so no
+# VGPR spills and no scratch (AGPRs are their matrix accumulators).
+LANE_READS = {"wm_lu.hip": ("k_panel", "k_swap_trsm"), "wm_solve.hip": ("k_perm", "k_trsv")}
 _REMARK = "kernel-resource-usage"
 
 
@@ -60,18 +64,24 @@ def resource_usage(stderr: str) -> dict:
     return out
 
 
-def check_spill_free(src: str, stderr: str) -> None:
-    names = SPILL_FREE.get(src)
-    if not names:
-        return
+def _check(src: str, stderr: str, names, fields) -> None:
     usage = {k: v for k, v in resource_usage(stderr).items() if any(n in k for n in names)}
     if not usage:
         raise RuntimeError(f"{src}: no resource-usage remarks for {names}")
-    bad = [(k, v) for k, v in usage.items()
-           if v.get("AGPRs", 0) or v.get("ScratchSize [bytes/lane]", 0) or v.get("VGPRs Spill", 0)]
+    bad = [(k, v) for k, v in usage.items() if any(v.get(f, 0) for f in fields)]
     if bad:
-        raise RuntimeError(f"{src}: kernels spill (AGPRs, scratch and VGPR spills must be 0):\n"
+        raise RuntimeError(f"{src}: kernels spill ({', '.join(fields)} must be 0):\n"
                            + "\n".join(f"  {k}: {v}" for k, v in bad))
+
+
+def check_spill_free(src: str, stderr: str) -> None:
+    if src in SPILL_FREE:
+        _check(src, stderr, SPILL_FREE[src], ("AGPRs", "ScratchSize [bytes/lane]", "VGPRs Spill"))
+
+
+def check_lane_reads(src: str, stderr: str) -> None:
+    if src in LANE_READS:
+        _check(src, stderr, LANE_READS[src], ("ScratchSize [bytes/lane]", "VGPRs Spill"))
 
 
 def _compile(src: str) -> str:
@@ -79,13 +89,14 @@ def _compile(src: str) -> str:
     cmd = [HIPCC, "-c"]
     if src.endswith(".hip"):
         cmd += ["-x", "hip"] + HIPFLAGS
-    if src in SPILL_FREE:
+    if src in SPILL_FREE or src in LANE_READS:
         cmd += [f"-Rpass-analysis={_REMARK}", "-fno-caret-diagnostics"]
     cmd += [os.path.join(CSRC, src), "-o", obj] + COMMON
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {src}\n{' '.join(cmd)}\n{r.stderr}")
     check_spill_free(src, r.stderr)
+    check_lane_reads(src, r.stderr)
     err = "\n".join(l for l in r.stderr.splitlines()
                     if "packed-fp32-ops" not in l and _REMARK not in l and l.strip())
     if err:

@@ -54,10 +54,10 @@ constexpr int kSubDefault = 4, kSubLarge = 8, kSubLargeN = 8192;
 // candidate row); complex128 panels measured 208 us with two parts (3 -> 2
 // workgroups per CU) and 165 us with four, complex64 ones 280 us with one and
 // 196 us with two (64 columns, N = 512 .. 4096).
-// Half as many parts, rows of twice as many columns per thread, take a matrix
-// whose clusters do not fit on the device otherwise (n above 64 rows per
-// resident workgroup: 49152 complex128 rows, or fewer where contexts share the
-// device); slower (registers spill), but such a matrix has no other panel.
+// Half as many parts, and rows of twice as many columns per thread, take a matrix
+// whose clusters do not fit on the device otherwise (rows above 64, complex64 128,
+// per resident workgroup: 12288 complex128 rows where four contexts share the
+// device), in a kernel of its own (k_panel_tall).
 constexpr int kTprF64 = 4, kTprF32 = 2;
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -88,7 +88,7 @@ struct XLayout {
     static constexpr int NWS = NW + 16;  // stride of the candidate rows (whole 128-byte lines)
     static constexpr int SLS = 4;        // stride of the slots: dense, a poll reads few lines
     size_t par_bytes, perm_off, mat_bytes;
-    int slots;  // candidates per column: one per wave of 64 rows
+    int slots;  // candidates per column: one per wave of 64 rows (k_panel_tall: one per workgroup)
     __host__ __device__ XLayout(int slots_) : slots(slots_)
     {
         par_bytes = (size_t)slots * (SLS + NWS) * sizeof(uint64_t);
@@ -225,6 +225,58 @@ __device__ inline double2 mul_c(double ar, double ai, double br, double bi)
     return make_double2(fma_t(ar, br, -p), fma_t(ai, br, q));
 }
 
+// The end of a panel, by workgroup 0: pivots, the first zero pivot, and the
+// composite permutation of the panel's interchanges for the other columns:
+// after applying them in order, row rows[t] holds the old content of src[t].
+// Slots t < NB are rows k + t; the rows from below the panel that take
+// part get slots NB, NB+1, ... in order of first use.  One wave keeps slot t and
+// slot NB + t in lane t (NB is the wave width), so each interchange is a ballot
+// and two lane reads.
+template <typename T>
+__device__ inline void panel_pivots(const PanelArgs<T> &a, int b, const int *s_piv, int zero, int *pm)
+{
+    const int tid = threadIdx.x, lane = tid & 63, k = a.k;
+    if (tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
+    if (tid == 0 && zero >= 0 && a.info[b] == 0) a.info[b] = zero + 1;
+    if (tid >= 64) return;
+    static_assert(NB == 64, "one slot pair per lane");
+    const int rlo = k + lane;
+    int slo = k + lane, rhi = -1, shi = -1;
+    int cnt = NB;
+    for (int jx = 0; jx < NB; ++jx) {
+        const int pp = s_piv[jx];
+        if (pp == k + jx) continue;
+        int tp;
+        if (pp < k + NB) {
+            tp = pp - k;
+        } else {
+            const unsigned long long hit = __ballot(NB + lane < cnt && rhi == pp);
+            if (hit) {
+                tp = NB + (int)__builtin_ctzll(hit);
+            } else {
+                tp = cnt++;
+                if (lane == tp - NB) { rhi = pp; shi = pp; }
+            }
+        }
+        const int sj = __builtin_amdgcn_readlane(slo, jx);
+        const int st = tp < NB ? __builtin_amdgcn_readlane(slo, tp) : __builtin_amdgcn_readlane(shi, tp - NB);
+        if (lane == jx) slo = st;
+        if (tp < NB) {
+            if (lane == tp) slo = sj;
+        } else if (lane == tp - NB) {
+            shi = sj;
+        }
+    }
+    int *rows = pm + 1, *src = pm + 1 + 2 * NB;
+    rows[lane] = rlo;
+    src[lane] = slo;
+    if (NB + lane < cnt) {
+        rows[NB + lane] = rhi;
+        src[NB + lane] = shi;
+    }
+    if (lane == 0) pm[0] = cnt;
+}
+
 // GEPP of the (n-k) x NB panel at column k for one matrix per blockIdx.y.
 // Workgroup w holds rows k + w*RW .. k + (w+1)*RW - 1 in registers.  A row is
 // split into TPR parts of W = NB/TPR columns held by different waves ("chunk"
@@ -275,7 +327,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
     constexpr int NW = XLayout<V>::NW, NWS = XLayout<V>::NWS, SLS = XLayout<V>::SLS;
     constexpr int G = kPanelGroup;  // columns updated together
     constexpr int NE = NW / TPR / 2;  // values of a chunk's part of a row: one lane each (complex128: re and im apart)
-    static_assert((NE == 32 || NE == 64) && RW >= NB && W % 8 == 0 && W % G == 0, "panel layout");
+    static_assert((NE == 32 || NE == 64) && TPR > 1 && RW >= NB && W % 8 == 0 && W % G == 0, "panel layout");
     const int bl = blockIdx.y, w = blockIdx.x;          // bl: member of this launch
     const int b = a.bidx ? a.bidx[bl] : bl;              // b: matrix index
     const int tid = threadIdx.x, lane = tid & 63;
@@ -310,7 +362,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
     __shared__ int s_wr[NWC], s_wl[NWC];    // each row block's candidate: value, position, lane (-1: none)
     __shared__ T s_cand[NWC][2][NB];        // its row, real and imaginary parts
     __shared__ V s_u[2][NB];                // pivot row
-    __shared__ V s_nx[TPR > 1 ? 2 : 1][TPR > 1 ? RW : 1];  // values in the pivot column, for the other chunks
+    __shared__ V s_nx[2][RW];               // values in the pivot column, for the other chunks
     __shared__ double s_gv[2];
     __shared__ int s_gr[2];
     __shared__ double2 s_rinv[2];           // reciprocal of the pivot
@@ -354,7 +406,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
                     s_wr[rb] = wr;
                 }
             }
-            if (TPR > 1) s_nx[par][rb * 64 + lane] = V{nxr, nxi};
+            s_nx[par][rb * 64 + lane] = V{nxr, nxi};
         }
         __syncthreads();
         const int wl = __builtin_amdgcn_readfirstlane(s_wl[rb]);
@@ -378,11 +430,8 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         }
         // the pivot's reciprocal: by a wave whose columns are finished, where
         // there is one
-        V p1 = V{0, 0};  // the lane reads by the whole wave: a register reloaded for
-                         // lane 0 alone would not hold lane wl's value
-        if (TPR == 1 && wl >= 0) p1 = V{readlane_t(nxr, wl), readlane_t(nxi, wl)};
         if (wl >= 0 && owner && c == (cj > 0 ? cj - 1 : 0) && lane == 0) {
-            const V p = TPR > 1 ? s_nx[par][rb * 64 + wl] : p1;
+            const V p = s_nx[par][rb * 64 + wl];
             const double2 rp = p.x != 0 || p.y != 0 ? crecip((double)p.x, (double)p.y) : make_double2(0.0, 0.0);
             if (solo) {
                 s_rinv[par] = rp;
@@ -595,7 +644,7 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         const int gr = s_gr[par];
         const double2 rinv = s_rinv[par];
         const V un = s_u[par][j + 1 < NB ? j + 1 : j];
-        if (TPR > 1 && c != cj) {
+        if (c != cj) {
             const V x = s_nx[par][rb * 64 + lane];
             nxr = x.x;
             nxi = x.y;
@@ -631,54 +680,232 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
     for (int i = 0; i < W; ++i)
         if (valid) Ab[lr + (size_t)(k + c * W + i) * a.lda] = V{re[i], im[i]};
 
-    // composite permutation of the panel's interchanges, for the other columns:
-    // after applying them in order, row rows[t] holds the old content of src[t].
-    // Slots t < NB are rows k + t; the rows from below the panel that take
-    // part get slots NB, NB+1, ... in order of first use.  One wave of
-    // workgroup 0 keeps slot t and slot NB + t in lane t (NB is the wave
-    // width), so each interchange is a ballot and two lane reads.
     __syncthreads();  // s_piv complete
-    if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
-    if (w == 0 && tid == 0 && zero >= 0 && a.info[b] == 0) a.info[b] = zero + 1;
-    if (w == 0 && wave == 0) {
-        static_assert(NB == 64, "one slot pair per lane");
-        const int rlo = k + lane;
-        int slo = k + lane, rhi = -1, shi = -1;
-        int cnt = NB;
-        for (int jx = 0; jx < NB; ++jx) {
-            const int pp = s_piv[jx];
-            if (pp == k + jx) continue;
-            int tp;
-            if (pp < k + NB) {
-                tp = pp - k;
-            } else {
-                const unsigned long long hit = __ballot(NB + lane < cnt && rhi == pp);
-                if (hit) {
-                    tp = NB + (int)__builtin_ctzll(hit);
-                } else {
-                    tp = cnt++;
-                    if (lane == tp - NB) { rhi = pp; shi = pp; }
+    if (w == 0) panel_pivots(a, b, s_piv, zero, X.perm(xm, a.pslot));
+}
+
+// The panel of a matrix too tall for k_panel's clusters: twice the rows per
+// workgroup (complex128 128 in two parts, complex64 256 in whole rows), the same
+// pivots, arithmetic and order, so the same bits.  A thread's 128 registers of
+// columns leave 40 at three workgroups per CU, and fewer workgroups would refuse
+// matrices that fit now; so nothing is carried from a column to the next but the
+// next pivot column's values: one candidate per workgroup, published after a second
+// barrier, and the update whole before the next argmax.  k_panel's deferred update
+// with this many columns spills 205 (complex128) and 343 registers, which is slow,
+// and lane reads among reloads are not safe (a register reloaded for some lanes
+// only does not hold the others' values): the build refuses it.  Per 64 columns of
+// one matrix of N = 4096 with random pivots 350 us in complex128 (the spilling form
+// 497, k_panel 172) and 438 us in complex64 (697, 207).
+template <typename T, int TPR>
+__global__ __launch_bounds__(256, kPanelOcc) void k_panel_tall(PanelArgs<T> a)
+{
+    using V = typename CT<T>::V;
+    constexpr int W = NB / TPR;     // columns per thread
+    constexpr int NWC = 4 / TPR;    // waves per chunk
+    constexpr int RW = 64 * NWC;    // rows per workgroup
+    constexpr int NW = XLayout<V>::NW, NWS = XLayout<V>::NWS, SLS = XLayout<V>::SLS;
+    static_assert(NW <= 256 && NW % 64 == 0 && RW >= NB, "panel layout");
+    const int bl = blockIdx.y, w = blockIdx.x;          // bl: member of this launch
+    const int b = a.bidx ? a.bidx[bl] : bl;              // b: matrix index
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = wave / NWC, rb = wave % NWC;           // chunk (columns c*W ..), row block
+    const int k = a.k, base = k + w * RW;
+    const int row = base + rb * 64 + lane;
+    const bool valid = row < a.n;
+    V *Ab = a.A + (size_t)b * a.strideA;
+    const XLayout<V> X(a.slots);
+    char *xm = a.xbuf + (size_t)bl * X.mat_bytes;
+    if (a.nmem && k >= a.nmem[b]) {  // as in k_panel
+        if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = k + tid + 1;
+        if (w == 0 && tid == 0) X.perm(xm, a.pslot)[0] = 0;
+        return;
+    }
+
+    T re[W], im[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        V x = V{0, 0};
+        if (valid) x = Ab[row + (size_t)(k + c * W + i) * a.lda];
+        re[i] = x.x;
+        im[i] = x.y;
+    }
+
+    __shared__ double s_wv[NWC];
+    __shared__ int s_wr[NWC];
+    __shared__ V s_cand[NB];  // this workgroup's best row
+    __shared__ V s_u[NB];     // pivot row
+    __shared__ V s_l[TPR > 1 ? RW : 1];  // multipliers for the other chunks
+    __shared__ double s_gv;
+    __shared__ int s_gr;
+    __shared__ double2 s_rinv;  // reciprocal of the pivot
+    __shared__ int s_piv[NB];   // pivot row of each column (workgroup 0)
+    __shared__ int s_zero;      // first column with a zero pivot
+    if (tid == 0) s_zero = -1;
+
+    const uint32_t tag0 = *a.tagp + a.toff;
+    int lr = row;  // current position of this thread's row
+    // this row's value in the column of the next step (column 0 is in chunk 0)
+    T nxr = re[0], nxi = im[0];
+    for (int j = 0; j < NB; ++j) {
+        const int par = j & 1;
+        const int pr = k + j;
+        const int cj = j / W;
+        const uint32_t tag = tag0 + (uint32_t)j + 1u;
+
+        // 1. best row of each wave of the chunk holding column j
+        if (c == cj) {
+            const double v = fabs((double)nxr) + fabs((double)nxi);
+            const int l = wave_best(v, lr, valid && lr >= pr && v == v);
+            const int ll = max(l, 0);
+            const double wv = l < 0 ? -1.0 : readlane_f64(v, ll);
+            const int wr = l < 0 ? kNoRow : __builtin_amdgcn_readlane(lr, ll);
+            if (lane == 0) {
+                s_wv[rb] = wv;
+                s_wr[rb] = wr;
+            }
+        }
+        __syncthreads();
+
+        // 2. this workgroup's candidate: its slot is published at once, so the
+        //    other workgroups' reductions start while the row is staged in LDS
+        double wv = s_wv[0];
+        int wr = s_wr[0];
+#pragma unroll
+        for (int q = 1; q < NWC; ++q)
+            if (better(s_wv[q], s_wr[q], wv, wr)) { wv = s_wv[q]; wr = s_wr[q]; }
+        uint64_t *slot = X.slot(xm, par);
+        uint64_t *cand = X.cand(xm, par);
+        if (tid < 3) {
+            const uint64_t bits = (uint64_t)__double_as_longlong(wv);
+            const uint32_t word = tid == 0 ? (uint32_t)bits : tid == 1 ? (uint32_t)(bits >> 32) : (uint32_t)wr;
+            put_pkt(slot + (size_t)w * SLS + tid, tag, word);
+        }
+        if (wr != kNoRow && lr == wr) {
+#pragma unroll
+            for (int i = 0; i < W; ++i) s_cand[c * W + i] = V{re[i], im[i]};
+        }
+        __syncthreads();
+
+        // 3. publish the candidate row (its words in the order of memory)
+        if (tid < NW) put_pkt(cand + (size_t)w * NWS + tid, tag, ((const uint32_t *)s_cand)[tid]);
+
+        // 4. wave 0 reduces all candidates to the same pivot (first max), then
+        //    fetches the pivot row from the workgroup holding it and takes the
+        //    pivot's reciprocal, so one barrier hands everything to the others
+        if (wave == 0) {
+            double gv = -1.0;
+            int gr = kNoRow, gs = 0;
+            for (int s = lane; s < a.P; s += 64) {
+                const uint64_t *ps = slot + (size_t)s * SLS;
+                uint64_t w0, w1, w2;
+                long it = 0;
+                for (;;) {
+                    w0 = ld_pkt(ps);
+                    w1 = ld_pkt(ps + 1);
+                    w2 = ld_pkt(ps + 2);
+                    if ((uint32_t)(w0 >> 32) == tag && (uint32_t)(w1 >> 32) == tag && (uint32_t)(w2 >> 32) == tag)
+                        break;
+                    if (spin_give_up(it, a.err)) break;
+                }
+                const double v2 = __longlong_as_double((long long)(((w1 & 0xffffffffull) << 32) | (w0 & 0xffffffffull)));
+                const int r2 = (int)(uint32_t)w2;
+                if (better(v2, r2, gv, gr)) { gv = v2; gr = r2; gs = s; }
+            }
+            const int l = wave_best(gv, gr, gr != kNoRow);
+            const int r = l >= 0 ? __builtin_amdgcn_readlane(gr, l) : kNoRow;
+            // no usable candidate (non-finite column): a zero pivot in place
+            const bool ok = r >= pr && r < a.n;
+            double m = 0.0;
+            double2 rinv = make_double2(0.0, 0.0);
+            if (ok) {
+                m = readlane_f64(gv, l);
+                constexpr int PL = NW / 64;  // pivot-row words per lane, loaded together
+                const uint64_t *pu = cand + (size_t)__builtin_amdgcn_readlane(gs, l) * NWS + lane;
+                uint64_t wu[PL];
+                long it = 0;
+                for (;;) {
+                    bool got = true;
+#pragma unroll
+                    for (int e = 0; e < PL; ++e) {
+                        wu[e] = ld_pkt(pu + 64 * e);
+                        got = got && (uint32_t)(wu[e] >> 32) == tag;
+                    }
+                    if (got) break;
+                    if (spin_give_up(it, a.err)) break;
+                }
+#pragma unroll
+                for (int e = 0; e < PL; ++e) ((uint32_t *)s_u)[lane + 64 * e] = (uint32_t)wu[e];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const V p = s_u[j];  // written by this wave above
+                if (m != 0.0) rinv = crecip((double)p.x, (double)p.y);
+            }
+            if (lane == 0) {
+                s_gv = m;
+                s_gr = ok ? r : pr;
+                s_rinv = rinv;
+            }
+        }
+        __syncthreads();
+        const double gv = s_gv;
+        const int gr = s_gr;
+
+        // 5. interchange positions k+j and gr, scale column j, rank-1 update
+        const double2 rinv = s_rinv;
+        if (tid == 0) s_piv[j] = gr;
+        if (tid == 0 && gv == 0.0 && s_zero < 0) s_zero = pr;
+        if (lr == gr) lr = pr;
+        else if (lr == pr) lr = gr;
+        const bool act = gv != 0.0 && valid && lr > pr;
+        T lre = 0, lim = 0;
+        if (c == cj) {
+            if (act) {
+                const double2 l = mul_c((double)nxr, (double)nxi, rinv.x, rinv.y);
+                lre = (T)l.x;
+                lim = (T)l.y;
+            }
+            if (TPR > 1) s_l[rb * 64 + lane] = V{lre, lim};
+        }
+        if (TPR > 1) {
+            __syncthreads();
+            if (c != cj) {
+                const V l = s_l[rb * 64 + lane];
+                lre = l.x;
+                lim = l.y;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            const int col = c * W + i;  // uniform
+            if (col == j) {             // the multiplier replaces column j
+                if (act) {
+                    re[i] = lre;
+                    im[i] = lim;
+                }
+            } else if (col > j) {
+                if (sizeof(T) == 4 || act) {  // as in k_panel
+                    const V u = s_u[col];
+                    re[i] = sub_mul_re(re[i], lre, lim, u.x, u.y);
+                    im[i] = sub_mul_im(im[i], lre, lim, u.x, u.y);
+                }
+                if (col == j + 1) {
+                    nxr = re[i];
+                    nxi = im[i];
                 }
             }
-            const int sj = __builtin_amdgcn_readlane(slo, jx);
-            const int st = tp < NB ? __builtin_amdgcn_readlane(slo, tp) : __builtin_amdgcn_readlane(shi, tp - NB);
-            if (lane == jx) slo = st;
-            if (tp < NB) {
-                if (lane == tp) slo = sj;
-            } else if (lane == tp - NB) {
-                shi = sj;
-            }
+            // keep the scheduler from hoisting every column's pivot-row load at once
+            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        int *pm = X.perm(xm, a.pslot);
-        int *rows = pm + 1, *src = pm + 1 + 2 * NB;
-        rows[lane] = rlo;
-        src[lane] = slo;
-        if (NB + lane < cnt) {
-            rows[NB + lane] = rhi;
-            src[NB + lane] = shi;
-        }
-        if (lane == 0) pm[0] = cnt;
     }
+
+    // each row to its final position
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+        if (valid) Ab[lr + (size_t)(k + c * W + i) * a.lda] = V{re[i], im[i]};
+    __syncthreads();  // s_piv complete
+    if (w == 0) panel_pivots(a, b, s_piv, s_zero, X.perm(xm, a.pslot));
 }
 
 // ---------------------------------------------------------------------------
@@ -1459,10 +1686,20 @@ int prepare_xbuf(wm_ctx *ctx, size_t bytes, uint64_t ntags, hipStream_t s)
     return WM_OK;
 }
 
+// The panel kernel with TPR parts per row.
+template <typename T, int TPR>
+constexpr bool kTall = TPR != (sizeof(T) == 8 ? kTprF64 : kTprF32);
+template <typename T, int TPR>
+auto panel_kernel()
+{
+    if constexpr (kTall<T, TPR>) return k_panel_tall<T, TPR>;
+    else return k_panel<T, TPR>;
+}
+
 template <typename T, int TPR>
 int occupancy_panel(int *blocks_per_cu)
 {
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k_panel<T, TPR>, 256, 0);
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, panel_kernel<T, TPR>(), 256, 0);
     if (e != hipSuccess) {
         set_error("occupancy query failed: %s", hipGetErrorString(e));
         return WM_ERR_HIP;
@@ -1509,7 +1746,7 @@ int getrf_plan(wm_ctx *ctx, int n, int batch, GetrfPlan *pl)
     pl->pmax = pmax;
     pl->resident = resident;
     pl->per_launch = std::min(batch, resident / pmax);
-    pl->slots = pmax * (RW / 64);
+    pl->slots = kTall<T, TPR> ? pmax : pmax * (RW / 64);
     pl->xbytes = (size_t)batch * XLayout<V>(pl->slots).mat_bytes;
     return WM_OK;
 }
@@ -1562,7 +1799,7 @@ int getrf_impl(wm_ctx *ctx, const GetrfPlan &pl, int n, typename CT<T>::V *A, in
             pa.nmem = d_nmem;
             // per column j, (mr-j) scalings and (mr-j)(NB-j-1) complex multiply-adds
             prof_begin(ctx, kPanelClass, G.st);
-            hipLaunchKernelGGL((k_panel<T, TPR>), dim3(P, m), dim3(256), 0, G.st, pa);
+            hipLaunchKernelGGL((panel_kernel<T, TPR>()), dim3(P, m), dim3(256), 0, G.st, pa);
             prof_end(ctx, kPanelClass, G.st, m * 8.0 * (mr * NB * NB / 2.0 - (double)NB * NB * NB / 6.0),
                      m * 2.0 * mr * NB * esz);
         }
@@ -1732,7 +1969,7 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
 {
     const int ks = getrf_block(ctx, prec, n);
     GetrfPlan pl;
-    if constexpr (TPR == (sizeof(T) == 8 ? kTprF64 : kTprF32)) {
+    if constexpr (!kTall<T, TPR>) {
         int resident = 0;
         WM_TRY((panel_resident<T, TPR>(ctx, &resident)));
         if ((n + 256 / TPR - 1) / (256 / TPR) > resident)

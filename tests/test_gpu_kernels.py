@@ -265,3 +265,58 @@ def test_mixed_sweep_routes_by_model(wm, geometries, ctx, geo_dir):
     assert [s["prec"] for s in st] == [wm.PREC_F64] * len(f)
     z64, c64, _ = wm.solve_sweep(g, f, [7], "f64")
     assert np.array_equal(zin, z64) and np.array_equal(cur, c64)
+
+
+@pytest.mark.parametrize("prec,rows", [("f64", 128), ("f32", 256)])
+@pytest.mark.parametrize("n", [192, 576, 8320])
+def test_panel_tall(wm, ctx, prec, rows, n):
+    """The panel of matrices too tall for the usual clusters, at partly filled workgroups and
+    at more workgroups than a wave has lanes: factors, pivots and zero-pivot reports of the
+    usual panel, bit for bit, on random entries, with a zero column and with a NaN row, for
+    every member and through an index table, launched directly and replayed."""
+    L = wm.lib()
+    L.wmx_set_panel_resident.argtypes = [C.c_void_p, C.c_int]
+    L.wmx_getrf_batched_idx.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_int64, C.c_void_p,
+                                        C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
+    rng = np.random.RandomState(n)
+    b, p = 3 if n < 4096 else 1, wm.PREC_NAMES[prec]
+    A = np.empty((b, n, n), np.complex128 if prec == "f64" else np.complex64)
+    A.real = rng.standard_normal((b, n, n))
+    A.imag = rng.standard_normal((b, n, n))
+    if b > 1:
+        A[1, n // 2] = 0.0  # members are stored column by column: a zero column
+        A[2, :, n // 3] = np.nan
+    dev = wm.DeviceArray(ctx, A)
+    piv = wm.DeviceArray(ctx, np.zeros((b, n), np.int32))
+    idx = np.arange(b, dtype=np.int32)[::-1].copy()
+
+    def factor(indexed):
+        dev.upload(A)
+        piv.upload(np.zeros((b, n), np.int32))
+        info = np.zeros(b, np.int32)
+        if indexed:
+            assert L.wmx_getrf_batched_idx(ctx.h, p, n, dev.ptr, n, n * n, piv.ptr, n, b, info.ctypes.data,
+                                           idx.ctypes.data) == 0
+            info = info[idx]
+        else:
+            assert L.wm_getrf_batched(ctx.h, p, n, dev.ptr, n, n * n, piv.ptr, n, b,
+                                      info.ctypes.data_as(C.POINTER(C.c_int))) >= 0  # > 0: a zero pivot
+        ctx.sync()
+        return dev.download(), piv.download(), info
+
+    ref = factor(False)
+    if b > 1:
+        assert ref[2][0] == 0 and ref[2][1] == n // 2 + 1 and ref[2][2] == n
+    try:
+        assert L.wmx_set_panel_resident(ctx.h, -(-n // rows)) == 0
+        for graphs, indexed in ((True, False), (True, False), (False, True)):
+            ctx.set_graphs(graphs)
+            got = factor(indexed)
+            assert np.array_equal(got[2], ref[2])
+            assert np.array_equal(got[1], ref[1])
+            assert np.array_equal(got[0], ref[0], equal_nan=True)
+    finally:
+        ctx.set_graphs(True)
+        assert L.wmx_set_panel_resident(ctx.h, 0) == 0
+    dev.free()
+    piv.free()

@@ -274,3 +274,34 @@ def test_factor_precision_model(wm, share, prec, n, count, prefer, join, width):
     p, j, w = C.c_int(-1), C.c_int(-1), C.c_int(-1)
     assert wm.lib().wmx_route_model(256, share, prec, n, count, C.byref(p), C.byref(j), C.byref(w)) == 0
     assert (p.value, j.value, w.value) == (prefer, join, width)
+
+
+def test_build_rejects_spills_under_lane_reads():
+    """build.py's guard on the kernels full of lane reads (panels, interchanges, row
+    permutation, triangular solves): scratch or VGPR spills in any instantiation fail the
+    build; SGPR spills, matrix accumulators in AGPRs and other kernels do not."""
+    import importlib.util
+    import os
+    here = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "praca-magisterska_amd")
+    spec = importlib.util.spec_from_file_location("wm_build", os.path.join(here, "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+
+    def remarks(name, **f):
+        r = [f"x.hip:1:1: remark: Function Name: {name} [-Rpass-analysis=kernel-resource-usage]"]
+        r += [f"x.hip:1:1: remark:     {k}: {v} [-Rpass-analysis=kernel-resource-usage]" for k, v in f.items()]
+        return "\n".join(r)
+
+    none = {"ScratchSize [bytes/lane]": 0, "VGPRs Spill": 0}
+    ok = remarks("_Z7k_panelIdLi4EE", VGPRs=159, AGPRs=0, **none, **{"SGPRs Spill": 19})
+    other = remarks("_Z9k_gemm_b3", VGPRs=256, AGPRs=0, **{"ScratchSize [bytes/lane]": 8, "VGPRs Spill": 1})
+    b.check_lane_reads("wm_lu.hip", ok + "\n" + other)
+    b.check_lane_reads("wm_solve.hip", remarks("_Z6k_trsvIdLb1E", VGPRs=254, AGPRs=48, **none))
+    b.check_lane_reads("wm_batch.hip", other)       # not a checked source
+    for src, name in (("wm_lu.hip", "_Z12k_panel_tallIdLi2EE"), ("wm_lu.hip", "_Z11k_swap_trsmIfLi8EE"),
+                      ("wm_solve.hip", "_Z6k_permPKi"), ("wm_solve.hip", "_Z6k_trsvIfLb0E")):
+        for bad in ({"ScratchSize [bytes/lane]": 12}, {"VGPRs Spill": 2}):
+            with pytest.raises(RuntimeError):
+                b.check_lane_reads(src, ok + "\n" + remarks(name, VGPRs=168, AGPRs=0, **{**none, **bad}))
+    with pytest.raises(RuntimeError):
+        b.check_lane_reads("wm_lu.hip", other)      # no remarks of a checked kernel

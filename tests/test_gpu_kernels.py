@@ -320,3 +320,48 @@ def test_panel_tall(wm, ctx, prec, rows, n):
         assert L.wmx_set_panel_resident(ctx.h, 0) == 0
     dev.free()
     piv.free()
+
+
+@pytest.mark.parametrize("form", ["f64", "f32", "f64 noalloc", "f32 noalloc", "f64 transposed"])
+@pytest.mark.parametrize("n", [64, 192, 576])
+def test_solve_widths(wm, ctx, n, form):
+    """Triangular solves at every way their right-hand sides are divided: one launch member
+    of up to 16 columns (both forms of the products, one or two columns per wave), two
+    members of even and of uneven widths, and a second pass beyond 32.  Two matrices, a
+    leading dimension above n.  The residual is a backward-stable solve's (n unit roundoffs
+    of the factors' precision), each column has the bits of the same column solved by itself,
+    and the rows between columns keep what they held."""
+    prec, kind = form.split()[0], form.split()[-1]
+    rng = np.random.RandomState(n)
+    A = rng.randn(2, n, n) + 1j * rng.randn(2, n, n)
+    dev, piv, info = wm.getrf_batched(ctx, A, prec)
+    assert not info.any()
+    A = A.astype(np.complex64 if prec == "f32" else np.complex128).astype(np.complex128)
+    op = A.conj().transpose(0, 2, 1) if kind == "transposed" else A
+    L, ld = wm.lib(), n + 5
+    f = {"noalloc": L.wm_getrs_batched_noalloc, "transposed": L.wmx_getrs_trans}.get(kind, L.wm_getrs_batched)
+
+    def solve(B):
+        k = B.shape[1]
+        pad = np.full((2, k, ld), 7.0 - 3.0j)
+        pad[:, :, :n] = B
+        D = wm.DeviceArray(ctx, pad)
+        assert f(ctx.h, wm.PREC_NAMES[prec], n, k, dev.ptr, n, C.c_int64(n * n), piv.ptr,
+                 C.c_int64(n), D.ptr, ld, C.c_int64(k * ld), 2) == 0
+        ctx.sync()
+        X = D.download()
+        D.free()
+        assert np.all(X[:, :, n:] == 7.0 - 3.0j)
+        return X[:, :, :n]
+
+    widths = {"transposed": (1, 9, 17)}.get(kind, (1, 4, 5, 8, 9, 15, 16, 17, 18, 31, 32, 33, 40))
+    B = rng.randn(2, max(widths), n) + 1j * rng.randn(2, max(widths), n)
+    alone = np.concatenate([solve(B[:, r:r + 1]) for r in range(max(widths))], axis=1)
+    u = 2.0 ** (-24 if prec == "f32" else -53)
+    R = np.matmul(alone, op.transpose(0, 2, 1)) - B
+    assert np.abs(R).max() <= n * u * np.abs(op).sum(axis=2).max() * np.abs(alone).max()
+    for k in widths:
+        X = solve(B[:, :k])
+        assert np.array_equal(X.view(np.uint64), alone[:, :k].copy().view(np.uint64)), k
+    dev.free()
+    piv.free()

@@ -193,9 +193,10 @@ int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm
 int getrs_perm_batched(wm_ctx *ctx, int prec, int n, int nrhs, const void *A, int lda, int64_t strideA,
                        const int *perm, int64_t strideQ, void *B, int ldb, int64_t strideB, int batch,
                        hipStream_t s, const int *d_bidx = nullptr, const int *d_aidx = nullptr);
-// Solves with shared factors: column r < nr of item items[q] (at V + items[q] *
-// strideV + r * n) is solved in place with the factors and permutation of
-// index fac[q].  The columns of items that share a factor are the right-hand
+// Solves with shared factors by substitution, a reference for the form below
+// (reached through wmx_getrs_grouped only): column r < nr of item items[q] (at V +
+// items[q] * strideV + r * n) is solved in place with the factors and permutation
+// of index fac[q].  The columns of items that share a factor are the right-hand
 // sides of one launch member (up to max_w <= 8 per member); a column's
 // arithmetic is the same whatever it is grouped with.
 int getrs_grouped(wm_ctx *ctx, int prec, int n, int nr, const void *F, int lda, int64_t strideF, const int *perm,

@@ -2065,10 +2065,8 @@ int getrf_batched(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t stride
 }  // namespace wm
 
 // ---------------------------------------------------------------------------
-// Internal test hooks (not part of include/wiremom.h): run one step of the
-// blocked factorization on a device matrix so tests can check each kernel
-// against numpy.  A is n x n (lda = n), complex128 for prec 0, complex64 else.
-// C -= L U with C = A[K.., K..], L = A[K.., 0..K), U = A[0..K, K..] (no factorization).
+// Internal test hooks (not part of include/wiremom.h).
+
 // Caps the panel workgroups taken as co-resident (0 restores the occupancy
 // query's count), so small factorizations split their panel launches as large
 // ones do; drops captured factorizations, whose launch split it changes.
@@ -2105,17 +2103,9 @@ extern "C" int wmx_getrf_batched_idx(wm_ctx *ctx, int prec, int n, void *A, int 
     return rc;
 }
 
-extern "C" int wmx_gemm_k(wm_ctx *ctx, int prec, int n, void *A, int K, int reps)
-{
-    using namespace wm;
-    if (K <= 0 || K >= n || K % NB || reps <= 0) return WM_ERR_ARG;
-    const GemmArgs g{K, K, n - K, n - K, 0, K, nullptr};
-    for (int r = 0; r < reps; ++r)
-        launch_gemm(prec == WM_PREC_F64 ? 8 : prec == WM_PREC_BF16X3 ? 2 : 4, A, n, 0, g, 1, nullptr, ctx->stream);
-    WM_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    return WM_OK;
-}
-
+// One update of the right-looking factorization on a device matrix (n x n, lda = n,
+// complex128 for prec 0, complex64 else), without the factorization: C -= L U with
+// C = A[k+NB.., k+NB..], L = A[k+NB.., k..k+NB), U = A[k..k+NB, k+NB..).
 extern "C" int wmx_gemm_step(wm_ctx *ctx, int prec, int n, void *A, int k)
 {
     using namespace wm;
@@ -2125,48 +2115,4 @@ extern "C" int wmx_gemm_step(wm_ctx *ctx, int prec, int n, void *A, int k)
     launch_gemm(prec == WM_PREC_F64 ? 8 : prec == WM_PREC_BF16X3 ? 2 : 4, A, n, 0, g, 1, nullptr, ctx->stream);
     WM_HIP_TRY(hipStreamSynchronize(ctx->stream));
     return WM_OK;
-}
-
-// One panel factorization at column k followed by the interchanges and U12.
-extern "C" int wmx_panel_step(wm_ctx *ctx, int prec, int n, void *A, int *ipiv, int k, int do_swap)
-{
-    using namespace wm;
-    if (n % NB || k % NB || k + NB > n) return WM_ERR_ARG;
-    int *info = nullptr;
-    WM_HIP_TRY(hipMalloc(&info, sizeof(int)));
-    WM_HIP_TRY(hipMemset(info, 0, sizeof(int)));
-    auto run = [&](auto tag, auto *Ap, int TPRv) -> int {
-        using T = decltype(tag);
-        using V = typename CT<T>::V;
-        const int RW = 256 / TPRv;
-        const int slots = (n + RW - 1) / RW * (RW / 64);
-        const XLayout<V> X(slots);
-        WM_TRY(prepare_xbuf(ctx, X.mat_bytes, (uint64_t)n, ctx->stream));
-        char *xbuf = (char *)ctx->ws_lu.ptr;
-        hipLaunchKernelGGL(k_tag_bump, dim3(1), dim3(64), 0, ctx->stream, ctx->d_tag, (uint32_t)n);
-        ctx->panel_tag += (uint64_t)n;
-        PanelArgs<T> pa;
-        pa.A = (V *)Ap; pa.lda = n; pa.strideA = 0; pa.n = n; pa.k = k;
-        pa.P = (n - k + RW - 1) / RW; pa.slots = slots; pa.pslot = 0;
-        pa.ipiv = ipiv; pa.strideP = 0; pa.info = info;
-        pa.err = ctx->d_err; pa.xbuf = xbuf; pa.bidx = nullptr; pa.tagp = ctx->d_tag; pa.toff = (uint32_t)k;
-        pa.nmem = nullptr;
-        if (sizeof(T) == 8)
-            hipLaunchKernelGGL((k_panel<double, kTprF64>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<double> *)&pa);
-        else
-            hipLaunchKernelGGL((k_panel<float, kTprF32>), dim3(pa.P, 1), dim3(256), 0, ctx->stream, *(PanelArgs<float> *)&pa);
-        if (do_swap) {
-            SwapArgs sa;
-            sa.n = n; sa.k = k; sa.slots = slots; sa.do_swap = 1; sa.nmem = nullptr;
-            sa.pslot = 0; sa.c_l0 = 0; sa.c_l1 = k;
-            sa.c_tr0 = k + NB; sa.c_tr1 = n; sa.c_sw0 = n;
-            launch_swap<T>(ctx, sa, (V *)Ap, n, 0, xbuf, nullptr, 1, ctx->stream);
-        }
-        return WM_OK;
-    };
-    int rc = (prec == WM_PREC_F64) ? run(double(0), (double2 *)A, kTprF64) : run(float(0), (float2 *)A, kTprF32);
-    WM_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    (void)hipFree(info);
-    if (rc != WM_OK) return rc;
-    return check_device_error(ctx, ctx->stream);
 }

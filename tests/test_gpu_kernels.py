@@ -365,3 +365,39 @@ def test_solve_widths(wm, ctx, n, form):
         assert np.array_equal(X.view(np.uint64), alone[:, :k].copy().view(np.uint64)), k
     dev.free()
     piv.free()
+
+
+def test_preconditioner_solve_grouping(wm, ctx):
+    """The preconditioner's solves with several factors, items in another order than they are
+    stored and members of 16, 4, 12 and 4 columns (20, 12 and 4 columns of three factors):
+    1e-12 of numpy's solutions on diagonally dominant matrices, each item with the bits it
+    has when solved by itself, and items outside the list untouched."""
+    L = wm.lib()
+    L.wmx_getrs_grouped.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_void_p,
+                                    C.c_void_p, C.c_int64, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int]
+    rng = np.random.RandomState(11)
+    n, nf, nr, nv = 192, 3, 4, 10
+    A = rng.randn(nf, n, n) + 1j * rng.randn(nf, n, n) + 4 * n ** 0.5 * np.eye(n)
+    V = rng.randn(nv, nr, n) + 1j * rng.randn(nv, nr, n)
+    items = [8, 1, 2, 3, 4, 5, 6, 7, 0]  # item 9 takes no part
+    fac = [0, 0, 1, 2, 0, 1, 0, 1, 0]
+    dev, piv, info = wm.getrf_batched(ctx, A, "f64")
+    assert not info.any()
+
+    def solve(items, fac):
+        Vd = wm.DeviceArray(ctx, V)
+        it, f = np.array(items, np.int32), np.array(fac, np.int32)
+        assert L.wmx_getrs_grouped(ctx.h, wm.PREC_F64, n, nr, dev.ptr, nf, piv.ptr, Vd.ptr, n * nr, len(it),
+                                   it.ctypes.data, f.ctypes.data, 1, 0) == 0
+        out = Vd.download()
+        Vd.free()
+        return out
+
+    got = solve(items, fac)
+    assert np.array_equal(got[9], V[9])
+    for q, f in zip(items, fac):
+        x = np.linalg.solve(A[f], V[q].T).T
+        assert np.abs(got[q] - x).max() <= 1e-12 * np.abs(x).max()
+        assert np.array_equal(solve([q], [f])[q].view(np.uint64), got[q].view(np.uint64))
+    dev.free()
+    piv.free()

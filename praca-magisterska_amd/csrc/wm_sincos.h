@@ -6,10 +6,11 @@
 // n P2 are exact for n < 2^20) and P3 the remainder, each subtracted with a
 // fused multiply-add; then sin r and cos r on |r| <= pi/4 (a little beyond
 // after rounding n) from minimax polynomials (this project's own fit: weighted
-// least squares in 80-bit arithmetic, reweighted to a level error; truncation
-// errors relative to the result 1.86e-20 and 5.7e-20, where the Taylor sums through r^17
-// and r^16 used before leave 1e-19 and 3e-18 with two more terms), and the
-// quadrant n mod 4.
+// least squares in 80-bit arithmetic, reweighted to a level error; with the
+// coefficients rounded to double the errors relative to the result are 6.0e-18 and
+// 1.5e-18, a twentieth of an ulp at most: the rounding of -1/6 decides the sine's, and the
+// Taylor sums through r^17 and r^16 used before are no better, 6.4e-18 and 1.6e-18,
+// with one more term each), and the quadrant n mod 4.
 // Every rounding is written out, so host and device builds give the same bits.
 #pragma once
 

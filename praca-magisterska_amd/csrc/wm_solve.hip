@@ -710,8 +710,10 @@ void launch_trsv(const TrsvArgs &a, int items, bool upper, hipStream_t s)
 int perm_batched(wm_ctx *ctx, int n, const int *ipiv, int64_t strideP, int *perm, int64_t strideQ, int batch,
                  hipStream_t s, const int *d_bidx, void *maps)
 {
-    if ((size_t)n * sizeof(int) > ctx->max_lds) {  // the accepted range of n
-        set_error("permutation: n=%d exceeds the LDS capacity", n);
+    // the accepted range of n: as many rows as ints in the LDS (40960).  The kernels
+    // below keep no row in LDS; the range is part of the entry points' contract
+    if ((size_t)n * sizeof(int) > ctx->max_lds) {
+        set_error("permutation: n=%d exceeds %zu rows", n, ctx->max_lds / sizeof(int));
         return WM_ERR_ARG;
     }
     const unsigned nb = (unsigned)((n + 255) / 256);

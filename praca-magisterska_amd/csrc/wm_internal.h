@@ -132,6 +132,7 @@ struct wm_geom {
     int npls = 0;     // N, unknowns
     int ld = 0;       // padded size (multiple of 128)
     double diam = 0;  // bounding-box diagonal of the structure (with its image over the PEC ground), m
+    void *d_tables = nullptr;  // the allocation that holds the tables below
     double *d_obs = nullptr;   // 12 arrays of ld doubles: rc1xyz, lm1xyz, rc2xyz, lm2xyz
     // fill: runs of rows ("waves") whose observation points (segment centres)
     // are at most 64 distinct ones, padding rows included

@@ -401,3 +401,24 @@ def test_preconditioner_solve_grouping(wm, ctx):
         assert np.array_equal(solve([q], [f])[q].view(np.uint64), got[q].view(np.uint64))
     dev.free()
     piv.free()
+
+
+@pytest.mark.parametrize("ienv", [1, 2])
+def test_fill_peaks_off_their_segments(wm, geometries, oracle, ctx, geo_dir, ienv):
+    """Bases whose peak is not a node of their segments (arrays a caller may pass): halves of
+    one segment then have several observation points, which the row tables keep apart, within
+    a run of rows and from run to run.  Every entry against the oracle."""
+    import os
+    p = os.path.join(geo_dir, f"peaks_{ienv}.geo")
+    (geometries.monopole if ienv == 2 else geometries.dipole)(p, *((300,) if ienv == 2 else (301, 1.0, 0.0005)))
+    t, o = wm.configwire(p, ienv=ienv), oracle.load(p, ienv=ienv)
+    n = t.npls
+    rng = np.random.RandomState(5)
+    for b in rng.choice(np.arange(5, n - 5), 40, replace=False):
+        # four nodes further along the wire: no half of zero length
+        t.ipc[b] = o.ipc[b] = abs(int(t.ipc[b])) + 4
+    g = wm.Geometry.from_topology(ctx, t, ienv)
+    assert g.npls == n
+    Z = g.fill([90.0])[0]
+    ref = oracle.zmatrix(o, wm.wavenumber(90.0), ienv=ienv)
+    assert np.abs(Z - ref).max() <= 1e-12 * np.abs(ref).max()

@@ -193,8 +193,20 @@ struct TrsvArgs {
 // step) and the product 1; 843 us per triangle instead of 1930 with the poll, the
 // products (values broadcast by lane reads) and a column per wave substitution in
 // the same four waves, eight columns at most per pass.
-template <typename T, bool UPPER, bool TRANS, bool SCALED>
-__global__ __launch_bounds__(256 + 64 * kPsPoll) void k_trsv(TrsvArgs a)
+//
+// SHORT solves matrices of at most two blocks: one product at most and no block
+// loaded ahead, so that two workgroups fit on a CU.  A batch of such matrices has no
+// chain to wait for, only as many blocks as matrices: 1000 x 64 29 -> 20 us per
+// triangle, 300 x 128 27.5 -> 19 (one column; 46 and 42 before the diagonal block's
+// loads were issued together).
+//
+// Otherwise eight waves are two per SIMD, and a third would be another workgroup's:
+// the scheduler is told so, or it shortens the distance of the complex64 form's
+// loads for an occupancy that no launch has (2 x 8192, eight columns: 904 us instead
+// of 852 per triangle).
+template <typename T, bool UPPER, bool TRANS, bool SCALED, bool SHORT>
+__global__ __launch_bounds__(256 + 64 * kPsPoll)
+__attribute__((amdgpu_waves_per_eu(SHORT ? 4 : 2, SHORT ? 4 : 2))) void k_trsv(TrsvArgs a)
 {
     // no contraction: a right-hand side's arithmetic is the same in every form
 #pragma clang fp contract(off)
@@ -231,15 +243,25 @@ __global__ __launch_bounds__(256 + 64 * kPsPoll) void k_trsv(TrsvArgs a)
 
     if (wave >= 4) {
         if (!SCALED) {
-            for (int e = tid - 256; e < TB * TB; e += 64 * kPsPoll) {
-                // consecutive threads walk down a column of the stored factor
-                const int i = TRANS ? e / TB : e % TB, j = TRANS ? e % TB : e / TB;
-                if (!UPPER && i > j) s_d[kPad + dl_idx(i, j)] = elem(r0 + i, r0 + j);
-                if (UPPER && i < j) s_d[kPad + du_idx(i, j)] = elem(r0 + i, r0 + j);
-                if (!UNIT && i == j) {
-                    const double2 u = elem(r0 + i, r0 + j);
-                    s_rd[i] = crecip(u.x, u.y);
-                }
+            // The whole block in loads without conditions, then the triangle of it to
+            // LDS, and the diagonal's reciprocals a lane each.  The blocks that start a
+            // chain wait for this (a load under its condition at a time and a reciprocal
+            // per column: 11.5 us per triangle of one block instead of 8).
+            constexpr int kEl = TB / kPsPoll;
+            V v[kEl];
+            const V *p = A + r0 + lane + (size_t)(r0 + wave - 4) * a.lda;  // down a column of the stored factor
+#pragma unroll
+            for (int q = 0; q < kEl; ++q) v[q] = p[(size_t)(kPsPoll * q) * a.lda];
+            if (!UNIT && wave == 4) {
+                const double2 u = elem(r0 + lane, r0 + lane);
+                s_rd[lane] = crecip(u.x, u.y);
+            }
+#pragma unroll
+            for (int q = 0; q < kEl; ++q) {
+                const int col = wave - 4 + kPsPoll * q, i = TRANS ? col : lane, j = TRANS ? lane : col;
+                const double2 x = make_double2((double)v[q].x, TRANS ? -(double)v[q].y : (double)v[q].y);
+                if (!UPPER && i > j) s_d[kPad + dl_idx(i, j)] = x;
+                if (UPPER && i < j) s_d[kPad + du_idx(i, j)] = x;
             }
         } else {
             __syncthreads();  // the right-hand sides are staged
@@ -382,14 +404,14 @@ __global__ __launch_bounds__(256 + 64 * kPsPoll) void k_trsv(TrsvArgs a)
         int q = noff & 1;
         if (q) {
             load_block(blk(0), lnext);
-            load_block(blk(min(1, noff - 1)), lcur);
+            if (!SHORT) load_block(blk(min(1, noff - 1)), lcur);
             __syncthreads();
             product(lnext, 1);
             subtract();
-        } else if (noff > 0) {
+        } else if (!SHORT && noff > 0) {
             load_block(blk(0), lcur);
         }
-        for (; q < noff; q += 2) {
+        for (; !SHORT && q < noff; q += 2) {
             load_block(blk(q + 1), lnext);
             __syncthreads();
             product(lcur, (q + 1) & 1);
@@ -701,8 +723,13 @@ template <typename T, bool TRANS, bool SCALED>
 void launch_trsv(const TrsvArgs &a, int items, bool upper, hipStream_t s)
 {
     const dim3 grid((unsigned)(items * a.chunks), (unsigned)(a.n / TB)), block(256 + 64 * kPsPoll);
-    if (upper) hipLaunchKernelGGL((k_trsv<T, true, TRANS, SCALED>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_trsv<T, false, TRANS, SCALED>), grid, block, 0, s, a);
+    if (!SCALED && a.n <= 2 * TB) {  // at three blocks a chain's next block is worth loading ahead
+        if (upper) hipLaunchKernelGGL((k_trsv<T, true, TRANS, false, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_trsv<T, false, TRANS, false, true>), grid, block, 0, s, a);
+        return;
+    }
+    if (upper) hipLaunchKernelGGL((k_trsv<T, true, TRANS, SCALED, false>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_trsv<T, false, TRANS, SCALED, false>), grid, block, 0, s, a);
 }
 
 }  // namespace

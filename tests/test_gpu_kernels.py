@@ -323,7 +323,7 @@ def test_panel_tall(wm, ctx, prec, rows, n):
 
 
 @pytest.mark.parametrize("form", ["f64", "f32", "f64 noalloc", "f32 noalloc", "f64 transposed"])
-@pytest.mark.parametrize("n", [64, 192, 576])
+@pytest.mark.parametrize("n", [64, 128, 192, 576])
 def test_solve_widths(wm, ctx, n, form):
     """Triangular solves at every way their right-hand sides are divided: one launch member
     of up to 16 columns (both forms of the products, one or two columns per wave), two

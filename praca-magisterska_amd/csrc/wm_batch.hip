@@ -504,12 +504,13 @@ double panel_launches(int n, int count, int width)
 }
 
 // Cost constants measured on MI355X at N = 8192 (lockstep batches of 48
-// complex128 and 16 complex64 matrices): a panel launch costs 64 columns x
-// 7.4 us (complex128) or x 7.3 us (complex64) whatever the cluster size; the
-// products and interchanges of a factorization run at 76 TF/s (FP64),
-// 122 TF/s (FP32) and 180 TF/s FP32-equivalent (split-BF16x3), all counted at
-// 8 real flops per complex multiply-add; a refinement iteration costs two
-// triangular-solve latency chains per batch (n/64 blocks x 8 us each) plus
+// complex128 and 16 complex64 matrices) with panels of model_width's rows (the
+// panels take 2.2-2.9 us per column now, a block of a solve 4-7.4 us): a panel
+// launch costs 64 columns x 7.4 us (complex128) or x 7.3 us (complex64) whatever
+// the cluster size; the products and interchanges of a factorization run at 76
+// TF/s (FP64), 122 TF/s (FP32) and 180 TF/s FP32-equivalent (split-BF16x3), all
+// counted at 8 real flops per complex multiply-add; a refinement iteration costs
+// two triangular-solve latency chains per batch (n/64 blocks x 8 us each) plus
 // 24 N^2 bytes per member at about 5 TB/s; about 6 iterations.
 constexpr double kPanelColF64 = 7.4e-6, kPanelColC64 = 7.3e-6;
 constexpr double kRateF64 = 76e12, kRateF32 = 122e12, kRateB3 = 180e12;

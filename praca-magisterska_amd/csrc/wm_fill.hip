@@ -26,9 +26,9 @@
 //    through scalar loads) and keeps the last segment's contribution as a first
 //    half: along a wire the second half of basis n is the first half of n + 1.
 // Measured at N = 8192, four frequencies: 968 -> 368 us per frequency (PEC ground
-// 1748 -> 679 us); N = 511: 25 -> 7.5 us.  The launch is bound by the FP64 VALU (69 % of the
-// issue slots at three waves per SIMD; writing the matrix alone would take
-// about 220 us): R, 1/R and the two nodes' weights are shared by the
+// 1748 -> 679 us); N = 511: 25 -> 7.5 us.  The launch is bound by the vector units (active
+// in 84 % of the SIMD cycles at three waves per SIMD, 70 % with the complex64 copy;
+// writing the matrix alone would take about 220 us): R, 1/R and the two nodes' weights are shared by the
 // frequencies, and per frequency and pair a lane issues about 105 instructions.
 // The four-term difference of scalar potentials is taken from values that are
 // the same bits in every entry that uses a pair, scalar and vector parts summed

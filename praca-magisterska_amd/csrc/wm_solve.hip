@@ -188,11 +188,11 @@ struct TrsvArgs {
 // One polling wave instead of four: 470 us for 1 x 3 before the 4x4x4 form, 355
 // with four; real and imaginary words apart (whole lines per store): 470 us
 // instead of 628 for 2 x 16.
-// Not SCALED: 4.4 us a block lower and 8.7 us upper with 8 columns in two matrices of
+// Not SCALED: 5.5 us a block lower and 7.4 us upper with 8 columns in two matrices of
 // N = 8192, of which the substitution is about 2.3 and 4 us (76 and 110 cycles a
-// step) and the product 1; 843 us per triangle instead of 1930 with the poll, the
-// products (values broadcast by lane reads) and a column per wave substitution in
-// the same four waves, eight columns at most per pass.
+// step) and the product 1; 827 us per triangle on average instead of 1977 with the
+// poll, the products (values broadcast by lane reads) and the substitution of two
+// columns per wave in the same four waves, eight columns at most per pass.
 //
 // SHORT solves matrices of at most two blocks: one product at most and no block
 // loaded ahead, so that two workgroups fit on a CU.  A batch of such matrices has no

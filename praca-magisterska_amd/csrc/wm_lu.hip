@@ -225,26 +225,21 @@ __device__ inline double2 mul_c(double ar, double ai, double br, double bi)
     return make_double2(fma_t(ar, br, -p), fma_t(ai, br, q));
 }
 
-// The end of a panel, by workgroup 0: pivots, the first zero pivot, and the
-// composite permutation of the panel's interchanges for the other columns:
-// after applying them in order, row rows[t] holds the old content of src[t].
-// Slots t < NB are rows k + t; the rows from below the panel that take
-// part get slots NB, NB+1, ... in order of first use.  One wave keeps slot t and
-// slot NB + t in lane t (NB is the wave width), so each interchange is a ballot
-// and two lane reads.
-template <typename T>
-__device__ inline void panel_pivots(const PanelArgs<T> &a, int b, const int *s_piv, int zero, int *pm)
+// Composite permutation of a panel's interchanges, for the other columns, by the
+// first wave of workgroup 0: after applying them in order, row rows[t] holds the
+// old content of src[t].  Slots t < NB are rows k + t; the rows from below the
+// panel that take part get slots NB, NB+1, ... in order of first use.  The wave
+// keeps pivot t, slot t and slot NB + t in lane t (NB is the wave width), so each
+// interchange is a ballot and three lane reads.
+__device__ inline void panel_perm(int k, int lane, const int *s_piv, int *pm)
 {
-    const int tid = threadIdx.x, lane = tid & 63, k = a.k;
-    if (tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
-    if (tid == 0 && zero >= 0 && a.info[b] == 0) a.info[b] = zero + 1;
-    if (tid >= 64) return;
     static_assert(NB == 64, "one slot pair per lane");
     const int rlo = k + lane;
     int slo = k + lane, rhi = -1, shi = -1;
+    const int pv = s_piv[lane];  // pivot row of column `lane`
     int cnt = NB;
     for (int jx = 0; jx < NB; ++jx) {
-        const int pp = s_piv[jx];
+        const int pp = __builtin_amdgcn_readlane(pv, jx);
         if (pp == k + jx) continue;
         int tp;
         if (pp < k + NB) {
@@ -681,7 +676,9 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
         if (valid) Ab[lr + (size_t)(k + c * W + i) * a.lda] = V{re[i], im[i]};
 
     __syncthreads();  // s_piv complete
-    if (w == 0) panel_pivots(a, b, s_piv, zero, X.perm(xm, a.pslot));
+    if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
+    if (w == 0 && tid == 0 && zero >= 0 && a.info[b] == 0) a.info[b] = zero + 1;
+    if (w == 0 && wave == 0) panel_perm(k, lane, s_piv, X.perm(xm, a.pslot));
 }
 
 // The panel of a matrix too tall for k_panel's clusters: twice the rows per
@@ -694,8 +691,8 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel(PanelArgs<T> a)
 // with this many columns spills 205 (complex128) and 343 registers, which is slow,
 // and lane reads among reloads are not safe (a register reloaded for some lanes
 // only does not hold the others' values): the build refuses it.  Per 64 columns of
-// one matrix of N = 4096 with random pivots 350 us in complex128 (the spilling form
-// 497, k_panel 172) and 438 us in complex64 (697, 207).
+// one matrix of N = 4096 with random pivots 348 us in complex128 (the spilling form
+// 497, k_panel 171) and 433 us in complex64 (697, 205).
 template <typename T, int TPR>
 __global__ __launch_bounds__(256, kPanelOcc) void k_panel_tall(PanelArgs<T> a)
 {
@@ -905,7 +902,9 @@ __global__ __launch_bounds__(256, kPanelOcc) void k_panel_tall(PanelArgs<T> a)
     for (int i = 0; i < W; ++i)
         if (valid) Ab[lr + (size_t)(k + c * W + i) * a.lda] = V{re[i], im[i]};
     __syncthreads();  // s_piv complete
-    if (w == 0) panel_pivots(a, b, s_piv, s_zero, X.perm(xm, a.pslot));
+    if (w == 0 && tid < NB) a.ipiv[(size_t)b * a.strideP + k + tid] = s_piv[tid] + 1;
+    if (w == 0 && tid == 0 && s_zero >= 0 && a.info[b] == 0) a.info[b] = s_zero + 1;
+    if (w == 0 && wave == 0) panel_perm(k, lane, s_piv, X.perm(xm, a.pslot));
 }
 
 // ---------------------------------------------------------------------------

@@ -344,6 +344,7 @@ int wm_init(int device, wm_ctx **out)
     WM_HIP_TRY(hipMemset(c->d_sync, 0, sizeof(int) * wm_ctx::kSyncCap));
     WM_HIP_TRY(hipMemset(c->d_err, 0, sizeof(int)));
     WM_TRY(noalloc_init(device));
+    WM_TRY(panel_gate_join(c));
     *out = c;
     return WM_OK;
 }
@@ -355,6 +356,7 @@ int wm_shutdown(wm_ctx *c)
     (void)hipStreamSynchronize(c->stream);
     if (c->aux) (void)hipStreamSynchronize(c->aux);
     if (c->lu_side) (void)hipStreamSynchronize(c->lu_side);
+    panel_gate_leave(c);
     drop_graphs(c);
     c->ws_info.release();
     c->ws_fill.release();
@@ -376,6 +378,7 @@ int wm_shutdown(wm_ctx *c)
     for (auto e : c->lu_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->lu_side) (void)hipStreamDestroy(c->lu_side);
+    if (c->lu_done) (void)hipEventDestroy(c->lu_done);
     (void)hipStreamDestroy(c->stream);
     if (c == g_default_ctx) g_default_ctx = nullptr;
     delete c;

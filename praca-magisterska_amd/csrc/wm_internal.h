@@ -123,6 +123,11 @@ struct wm_ctx {
     // stream while the next block's panels are factored; created on first use
     hipStream_t lu_side = nullptr;
     hipEvent_t lu_ev[2] = {nullptr, nullptr};  // launch stream -> lu_side, lu_side -> launch stream
+    // this context's latest factorization, for the other contexts of the device
+    // (panel_gate_*; guarded by the device's gate)
+    enum LuPhase { LU_NONE, LU_ENQUEUING, LU_RECORDED } lu_phase = LU_NONE;
+    int lu_cluster = 0;            // workgroups of its largest panel cluster
+    hipEvent_t lu_done = nullptr;  // LU_RECORDED: recorded behind it
 };
 
 // Geometry as the fill kernel reads it.  Observation data per basis (SoA,
@@ -319,6 +324,10 @@ bool prefer_f64(const wm_ctx *c, int prec, int n, int count);
 bool join_f64(const wm_ctx *c, int prec, int n, int r);
 // Most frequencies of a mixed sweep's batch: the model's complex64 launch width.
 int mixed_width(const wm_ctx *c, int n);
+// A context joins and leaves the contexts of its device whose factorizations
+// keep room for each other's panel clusters (wm_init, wm_shutdown).
+int panel_gate_join(wm_ctx *ctx);
+void panel_gate_leave(wm_ctx *ctx);
 // Matrices per launch of the batched factorization (panel cluster residency).
 int getrf_width(wm_ctx *ctx, int prec, int n);
 // Panels per outer block for a factorization of size n in precision prec.

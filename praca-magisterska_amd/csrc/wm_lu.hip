@@ -32,6 +32,9 @@
 //                     the C read-modify-write is coalesced in column-major
 //                     storage.
 #include <algorithm>
+#include <condition_variable>
+#include <mutex>
+#include <vector>
 
 #include "wm_cplx.h"
 #include "wm_internal.h"
@@ -1721,13 +1724,19 @@ struct GetrfPlan {
 // (panel_share), so that every cluster of every concurrent panel launch fits on
 // the device together.
 template <typename T, int TPR>
-int panel_resident(wm_ctx *ctx, int *resident)
+int panel_total(wm_ctx *ctx, int *total, int share = 1)
 {
     int bpc = 0;
     WM_TRY((occupancy_panel<T, TPR>(&bpc)));
-    *resident = bpc * ctx->num_cu / std::max(1, ctx->panel_share);
-    if (ctx->panel_resident_cap > 0 && ctx->panel_resident_cap < *resident) *resident = ctx->panel_resident_cap;
+    *total = bpc * ctx->num_cu / share;
+    if (ctx->panel_resident_cap > 0 && ctx->panel_resident_cap < *total) *total = ctx->panel_resident_cap;
     return WM_OK;
+}
+
+template <typename T, int TPR>
+int panel_resident(wm_ctx *ctx, int *resident)
+{
+    return panel_total<T, TPR>(ctx, resident, std::max(1, ctx->panel_share));
 }
 
 template <typename T, int TPR>
@@ -1962,6 +1971,93 @@ int getrf_side(wm_ctx *ctx, const GetrfPlan &pl, int n, int batch, int ks, hipSt
     return WM_OK;
 }
 
+// The contexts of one device, whose factorizations may run at the same time.
+// A panel cluster's workgroups wait for each other, so every cluster that may be
+// dispatched in part has to fit on the device beside the others': the lanes of a
+// server share it by panel_share, contexts of several host threads by this gate.
+// A factorization whose largest cluster does not fit beside those still running
+// starts behind them (an event, no wait on the host); clusters of 64 rows per
+// workgroup would otherwise fill the device at half the rows that those of 128
+// did (four threads with one matrix of N = 14336 each: 896 of 768 workgroups).
+// Counted per XCD, to which a launch deals its workgroups round-robin.
+// One context alone pays two uncontended locks.
+struct PanelGate {
+    std::mutex mu;
+    std::condition_variable cv;  // a context has finished enqueuing
+    std::vector<wm_ctx *> live;
+};
+constexpr int kGateDevices = 64;
+PanelGate g_gates[kGateDevices];
+
+class PanelHold {
+    static constexpr int kXcds = 8;
+    wm_ctx *c_;
+    hipStream_t s_;
+
+    static int per_xcd(int workgroups) { return (workgroups + kXcds - 1) / kXcds; }
+
+public:
+    PanelHold(wm_ctx *c, hipStream_t s) : c_(c), s_(s) {}
+    // device_total(int *): panel workgroups that the device holds
+    template <typename F>
+    int enter(int cluster, F device_total)
+    {
+        PanelGate &g = g_gates[c_->device];
+        std::unique_lock<std::mutex> lk(g.mu);
+        hipError_t e = hipSuccess;
+        int total = 0;
+        if (g.live.size() > 1) WM_TRY(device_total(&total));
+        for (bool fits = total == 0; !fits;) {
+            int sum = per_xcd(cluster);
+            bool enqueuing = false;
+            for (wm_ctx *o : g.live) {
+                if (o == c_) continue;
+                if (o->lu_phase == wm_ctx::LU_RECORDED && hipEventQuery(o->lu_done) == hipSuccess)
+                    o->lu_phase = wm_ctx::LU_NONE;
+                if (o->lu_phase == wm_ctx::LU_NONE) continue;
+                sum += per_xcd(o->lu_cluster);
+                enqueuing = enqueuing || o->lu_phase == wm_ctx::LU_ENQUEUING;
+            }
+            (void)hipGetLastError();  // an event that is not ready is no error
+            fits = sum <= total / kXcds;
+            if (!fits && enqueuing) {  // it has no event to wait for yet
+                g.cv.wait(lk);
+                continue;
+            }
+            if (!fits)
+                for (wm_ctx *o : g.live)
+                    if (o != c_ && o->lu_phase == wm_ctx::LU_RECORDED && e == hipSuccess)
+                        e = hipStreamWaitEvent(s_, o->lu_done, 0);
+            fits = true;
+        }
+        // the one before on this stream may still run
+        if (c_->lu_phase == wm_ctx::LU_RECORDED && hipEventQuery(c_->lu_done) != hipSuccess) {
+            (void)hipGetLastError();
+            cluster = std::max(cluster, c_->lu_cluster);
+        }
+        c_->lu_phase = wm_ctx::LU_ENQUEUING;
+        c_->lu_cluster = cluster;
+        lk.unlock();
+        WM_HIP_TRY(e);
+        return WM_OK;
+    }
+    ~PanelHold()
+    {
+        PanelGate &g = g_gates[c_->device];
+        std::lock_guard<std::mutex> lk(g.mu);
+        if (c_->lu_phase != wm_ctx::LU_ENQUEUING) return;
+        c_->lu_phase = wm_ctx::LU_NONE;
+        if (g.live.size() > 1) {
+            if ((c_->lu_done || hipEventCreateWithFlags(&c_->lu_done, hipEventDisableTiming) == hipSuccess) &&
+                hipEventRecord(c_->lu_done, s_) == hipSuccess)
+                c_->lu_phase = wm_ctx::LU_RECORDED;
+            else
+                (void)hipStreamSynchronize(s_);  // no event: finished before anyone else starts
+        }
+        g.cv.notify_all();
+    }
+};
+
 template <typename T, int TPR>
 int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, int *ipiv, int64_t strideP, int batch,
               int *d_info, const int *d_bidx, hipStream_t s, int gk, const int *d_nmem)
@@ -1980,6 +2076,8 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
     WM_TRY(prepare_xbuf(ctx, pl.xbytes, ntags, s));
     hipStream_t side = nullptr;
     WM_TRY(getrf_side(ctx, pl, n, batch, ks, &side));
+    PanelHold hold(ctx, s);
+    WM_TRY(hold.enter(pl.pmax, [&](int *total) { return panel_total<T, TPR>(ctx, total); }));
     if (!ctx->use_graphs || ctx->prof.on) {
         WM_TRY((getrf_enqueue<T, TPR>(ctx, pl, n, A, lda, strideA, ipiv, strideP, batch, d_info, d_bidx, s, gk, ks,
                                       d_nmem, side)));
@@ -2015,6 +2113,32 @@ int getrf_run(wm_ctx *ctx, int prec, int n, void *A, int lda, int64_t strideA, i
 }
 
 }  // namespace
+
+int panel_gate_join(wm_ctx *ctx)
+{
+    if (ctx->device < 0 || ctx->device >= kGateDevices) {
+        set_error("device %d beyond %d", ctx->device, kGateDevices);
+        return WM_ERR_ARG;
+    }
+    PanelGate &g = g_gates[ctx->device];
+    std::unique_lock<std::mutex> lk(g.mu);
+    // a context that was alone has recorded nothing behind its factorizations:
+    // they end before it has company
+    if (g.live.size() == 1) {
+        g.cv.wait(lk, [&] { return g.live.size() != 1 || g.live[0]->lu_phase != wm_ctx::LU_ENQUEUING; });
+        if (g.live.size() == 1) WM_HIP_TRY(hipStreamSynchronize(g.live[0]->stream));
+    }
+    g.live.push_back(ctx);
+    return WM_OK;
+}
+
+void panel_gate_leave(wm_ctx *ctx)
+{
+    PanelGate &g = g_gates[ctx->device];
+    std::lock_guard<std::mutex> lk(g.mu);
+    g.live.erase(std::remove(g.live.begin(), g.live.end(), ctx), g.live.end());
+    g.cv.notify_all();
+}
 
 // Destroys the captured factorizations.  A replay may still be running on the
 // stream it was launched on (nothing waits for it before the exchange buffer

@@ -403,6 +403,49 @@ def test_preconditioner_solve_grouping(wm, ctx):
     piv.free()
 
 
+@pytest.mark.parametrize("prec,n,cap", [("f64", 512, 8), ("f64", 512, 20), ("f32", 640, 5)])
+def test_contexts_factor_side_by_side(wm, ctx, prec, n, cap):
+    """Contexts of four threads on one device that take its panel workgroups to be so few that
+    no two clusters fit (cap 8 or 5), or only two (20): every factorization gives the
+    bits it gives alone, while contexts come and go."""
+    import threading
+    L = wm.lib()
+    L.wmx_set_panel_resident.argtypes = [C.c_void_p, C.c_int]
+    rng = np.random.RandomState(n)
+    A = [rng.randn(3, n, n) + 1j * rng.randn(3, n, n) for _ in range(4)]
+    ref = []
+    for a in A:
+        dev, piv, info = wm.getrf_batched(ctx, a, prec)
+        assert not info.any()
+        ref.append((dev.download(), piv.download()))
+    bad = []
+
+    def work(k):
+        try:
+            c = wm.Context(0)
+            c.set_graphs(False)  # other threads drive the device
+            assert L.wmx_set_panel_resident(c.h, cap) == 0
+            for _ in range(8):
+                dev, piv, info = wm.getrf_batched(c, A[k], prec)
+                if info.any() or not (np.array_equal(dev.download(), ref[k][0]) and
+                                      np.array_equal(piv.download(), ref[k][1])):
+                    bad.append(k)
+                dev.free()
+                piv.free()
+            c.close()
+        except Exception as e:  # reported by the main thread
+            bad.append((k, repr(e)))
+
+    t = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for x in t:
+        x.start()
+    for _ in range(3):
+        wm.Context(0).close()
+    for x in t:
+        x.join()
+    assert not bad
+
+
 @pytest.mark.parametrize("ienv", [1, 2])
 def test_fill_peaks_off_their_segments(wm, geometries, oracle, ctx, geo_dir, ienv):
     """Bases whose peak is not a node of their segments (arrays a caller may pass): halves of
